@@ -78,6 +78,56 @@ void auto_pair_tuning(uint64_t N, uint32_t resident_waves, uint32_t &R, uint32_t
 
 }  // namespace cr
 
+namespace cr {
+namespace {
+
+// 2^k words, inside the carry recursion, and estimated below `seconds`
+bool carry_preferred(uint64_t A, uint64_t num_words, double seconds, CarryPlan *p) {
+    if (num_words == 0 || (num_words & (num_words - 1)) || (unsigned __int128)(num_words - 1) * A >> 64) return false;
+    return carry_plan(A, (uint32_t)__builtin_ctzll(num_words), p) && p->seconds < seconds;
+}
+
+// The carry recursion on the context's buffers (carry.hip).
+cr_status an_pairs_carry(cr_context *ctx, const CarryPlan &p, uint64_t A, uint64_t *raw, uint32_t nbins,
+                         double *kernel_ms) {
+    clear_error();
+    if (!ctx || !raw) return fail(CR_ERR_INVALID_ARGUMENT, "NULL argument");
+    const uint32_t need = pair_max_distance(A, 1ull << p.k) + 1;
+    if (nbins < need) return fail(CR_ERR_INVALID_ARGUMENT, "nbins=%u but distances reach %u", nbins, need - 1);
+    CR_HIP(hipSetDevice(ctx->device));
+    const cr_status st = [&]() -> cr_status {
+        CR_TRY(ctx->table_a.reserve(p.table_bytes));
+        CR_TRY(ctx->table_b.reserve(p.table_bytes));
+        CR_TRY(ctx->hist.reserve(p.hist_entries * sizeof(uint64_t)));
+        CR_TRY(ctx->host.reserve(p.hist_entries * sizeof(uint64_t)));
+        unsigned long long *hist = ctx->hist.as<unsigned long long>();
+        if (kernel_ms) CR_HIP(hipEventRecord(ctx->ev0, ctx->stream));
+        CR_TRY(carry_run(p, ctx->table_a.ptr, ctx->table_b.ptr, hist, ctx->cus, ctx->stream));
+        if (kernel_ms) CR_HIP(hipEventRecord(ctx->ev1, ctx->stream));
+        CR_HIP(hipMemcpyAsync(ctx->host.ptr, hist, p.hist_entries * sizeof(uint64_t), hipMemcpyDeviceToHost,
+                              ctx->stream));
+        CR_HIP(hipStreamSynchronize(ctx->stream));
+        CR_TRY(carry_finish(p, ctx->host.as<uint64_t>(), raw, nbins));
+        if (kernel_ms) {
+            float ms = 0;
+            CR_HIP(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
+            *kernel_ms = ms;
+        }
+        return CR_OK;
+    }();
+    // as the transform buffers of the spectral path: a long-lived context
+    // does not hold tables above 1 GiB
+    if (p.table_bytes > (1ull << 30)) {
+        (void)hipStreamSynchronize(ctx->stream);
+        ctx->table_a.release();
+        ctx->table_b.release();
+    }
+    return st;
+}
+
+}  // namespace
+}  // namespace cr
+
 using namespace cr;
 
 extern "C" {
@@ -246,9 +296,15 @@ cr_status cr_an_pairs_tuned(cr_context *ctx, uint64_t A, uint64_t num_words, uin
 
 cr_status cr_an_pairs(cr_context *ctx, uint64_t A, uint64_t num_words, uint64_t *raw, uint32_t nbins,
                       double *kernel_ms) {
-    // the same histogram from the code's spectrum when that is clearly cheaper
+    // the same histogram by whichever method is estimated to be the fastest:
+    // the pair kernel (measured 40 us a call and about 7e12 pairs/s where it
+    // competes), the code's spectrum, the recursion over carries
     uint32_t k = 0;
-    if (spectral_preferred(A, num_words, &k)) return cr_an_pairs_spectral(ctx, A, k, raw, nbins, kernel_ms);
+    double best = 40e-6 + (double)num_words * (double)num_words / 14e12;
+    const bool spectral = spectral_preferred(A, num_words, &k, &best);
+    CarryPlan carry;
+    if (carry_preferred(A, num_words, best, &carry)) return an_pairs_carry(ctx, carry, A, raw, nbins, kernel_ms);
+    if (spectral) return cr_an_pairs_spectral(ctx, A, k, raw, nbins, kernel_ms);
     return cr_an_pairs_tuned(ctx, A, num_words, raw, nbins, nullptr, kernel_ms);
 }
 

@@ -169,8 +169,8 @@ constexpr uint32_t kHamMaxBatch = 4096;  // requests per cr_hamming_weights_batc
 // True when num_words = 2^k and cr_an_pairs_spectral supports (A, k) and is
 // estimated at under 80 % of the pair kernel's time (measured rates:
 // 2.2e-12 s per transformed element plus about 50 us per call, against
-// 9.6e12 pairs/s).
-bool spectral_preferred(uint64_t A, uint64_t num_words, uint32_t *k);
+// 9.6e12 pairs/s); *seconds (if not NULL) is the estimate.
+bool spectral_preferred(uint64_t A, uint64_t num_words, uint32_t *k, double *seconds = nullptr);
 
 // One exhaustive AN histogram by the code's spectrum, split into batches of
 // transforms (see spectral.hip): shape, device buffer and slot sizes.
@@ -193,6 +193,28 @@ cr_status spectral_run(const SpectralPlan &p, void *X, unsigned long long *slots
                        uint64_t nbatches, hipStream_t stream);
 // raw[] (nbins entries, pair-kernel form) from the host copy of the slots.
 cr_status spectral_finish(const SpectralPlan &p, const uint64_t *slots, uint64_t *raw, uint32_t nbins);
+
+// One exhaustive AN histogram by recursion over the carries of the product
+// (see carry.hip).
+struct CarryPlan {
+    uint32_t A = 0, Ainv = 0;   // odd part of the multiplier, its inverse modulo 2^32
+    uint32_t k = 0, T = 0;      // word bits; low bits that the last kernel takes at once (2^T > A)
+    uint32_t hb = 0;            // bits of the largest carry, A - 1
+    uint32_t levels = 0;        // k - T
+    uint32_t states = 0;        // carry pairs, A^2
+    uint32_t nbins = 0;         // distances 0 .. k + hb
+    uint64_t table_bytes = 0;   // of each of the two tables
+    uint64_t hist_entries = 0;  // dev::kHistCopies copies of nbins
+    double seconds = 0;         // estimated time of a call
+};
+// False when (A, 2^k words) is outside the recursion.
+bool carry_plan(uint64_t A, uint32_t k, CarryPlan *p);
+// Leaves the distribution over ordered pairs in hist (p.hist_entries, cleared here).
+cr_status carry_run(const CarryPlan &p, void *table0, void *table1, unsigned long long *hist, int cus,
+                    hipStream_t stream);
+// raw[] (nbins entries, pair-kernel form) from the host copy of hist; checks
+// the words at distance 0 and the total of 4^k.
+cr_status carry_finish(const CarryPlan &p, const uint64_t *hist, uint64_t *raw, uint32_t nbins);
 
 // Parity masks of the (N,k) extended Hamming codes, truncated to k bits;
 // returns the number of non-overall parity bits.

@@ -69,7 +69,7 @@ bool spectral_shape(uint64_t A, uint32_t k, uint64_t *Ao, uint32_t *n) {
 
 }  // namespace
 
-bool spectral_preferred(uint64_t A, uint64_t num_words, uint32_t *k) {
+bool spectral_preferred(uint64_t A, uint64_t num_words, uint32_t *k, double *seconds) {
     if (num_words == 0 || (num_words & (num_words - 1))) return false;
     const uint32_t kk = (uint32_t)__builtin_ctzll(num_words);
     uint64_t Ao = 0;
@@ -80,6 +80,7 @@ bool spectral_preferred(uint64_t A, uint64_t num_words, uint32_t *k) {
     const double spectral_s = std::ldexp(p.sec_per_element, (int)n) + 50e-6;
     const double pair_s = std::ldexp(1.0, 2 * (int)kk - 1) / 9.6e12;
     *k = kk;
+    if (seconds) *seconds = spectral_s;
     return spectral_s < 0.8 * pair_s;
 }
 

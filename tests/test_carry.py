@@ -1,0 +1,74 @@
+"""The recursion over carries that cr_an_pairs takes for short multipliers:
+the identity restated with Python integers against the oracle's pair counts
+(CPU), and the kernels against the pair kernel and closed forms (GPU)."""
+import math
+
+import pytest
+
+from oracle import oracle as O
+
+
+def carry_distribution(A, k):
+    """Ordered-pair distance distribution of A*i, i < 2^k, A odd, one bit a level."""
+    Q = {(c, d): [int(b == (c ^ d).bit_count()) for b in range(A.bit_length() + 1)] for c in range(A) for d in range(A)}
+    for _ in range(k):
+        nb = len(Q[0, 0]) + 1
+        R = {}
+        for c in range(A):
+            for d in range(A):
+                out = [0] * nb
+                for i in (0, 1):
+                    for j in (0, 1):
+                        v, w = c + A * i, d + A * j
+                        e = (v ^ w) & 1
+                        for b, x in enumerate(Q[v >> 1, w >> 1]):
+                            out[b + e] += x
+                R[c, d] = out
+        Q = R
+    return Q[0, 0]
+
+
+@pytest.mark.parametrize("A,k", [(1, 5), (3, 6), (5, 7), (11, 6), (13, 8)])
+def test_recursion_equals_pair_counts(A, k):
+    got = carry_distribution(A, k)
+    raw = O.an_pairs_raw(A, 1 << k, 65)
+    assert got[0] == 1 << k
+    assert [x // 2 for x in got[1:]] == raw[1:len(got)] and not any(raw[len(got):])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("A", [1, 3, 31, 33, 63, 127, 12 * 16, 255, 257, 511, 769])
+@pytest.mark.parametrize("k", [13, 14, 15, 17, 18])
+def test_carry_matches_pair_kernel(A, k):
+    # multipliers at both ends of a bit length (2^T > A, the largest carry),
+    # even ones, odd and even numbers of levels
+    import coding_reliability_amd as cra
+    with cra.Context(0) as ctx:
+        auto, _ = ctx.an_pairs_auto(A, 1 << k)
+        pair, _ = ctx.an_pairs(A, 1 << k)
+    assert auto == pair
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("A,k", [(61, 22), (641, 22), (1021, 23), (2047, 22), (2049, 24), (4095, 24), (61, 26)])
+def test_carry_matches_spectrum(A, k):
+    # 32-bit counters, then 64-bit ones from level 16 on (A = 61: k - 6 levels)
+    import coding_reliability_amd as cra
+    with cra.Context(0) as ctx:
+        auto, _ = ctx.an_pairs_auto(A, 1 << k)
+        spec, _ = ctx.an_pairs_spectral(A, k)
+    assert auto == spec
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("A,k", [(1, 30), (1 << 9, 32), (3, 32), (511, 32)])
+def test_carry_longest_words(A, k):
+    import coding_reliability_amd as cra
+    with cra.Context(0) as ctx:
+        raw, ms = ctx.an_pairs_auto(A, 1 << k)
+        assert ms < 100
+        with pytest.raises(cra.CRError):
+            ctx.an_pairs_auto(A, 1 << k, nbins=8)
+    assert sum(raw) == (1 << k) * ((1 << k) - 1) // 2
+    if A & (A - 1) == 0:
+        assert raw[1:k + 1] == [(1 << (k - 1)) * math.comb(k, d) for d in range(1, k + 1)]
