@@ -146,6 +146,22 @@ struct RectLaunch {
 };
 cr_status launch_rect(const RectLaunch &L, hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1, int cus);
 
+// The same histogram over rows A*i, i < 2^n, by recursion over the carries
+// (see carry_rows.hip).
+struct CarryRowsPlan {
+    uint32_t A = 0, z = 0;   // odd part of the multiplier, its trailing zero bits
+    uint32_t n = 0;
+    uint32_t rows = 0, threads = 0;  // distances in LDS, threads of a workgroup
+    size_t lds = 0;
+    bool wide = false;       // 64-bit counters
+};
+// False when the recursion does not apply or the rectangle kernel is estimated
+// to be faster; nbins: distances of the words and samples.
+bool carry_rows_plan(uint64_t A, uint32_t n, uint64_t ncols, uint32_t nbins, CarryRowsPlan *p);
+// Adds the histogram of all samples to dev::kHistCopies copies of nbins at out.
+cr_status launch_carry_rows(const CarryRowsPlan &p, const uint64_t *cols, uint32_t ncols, uint32_t nbins,
+                            unsigned long long *out, int cus, hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1);
+
 // Hamming weight jobs (see hamming.hip).
 enum HamSource : uint32_t { kHamRange = 0, kHamStride = 1, kHamList = 2, kHamMc = 3 };
 struct HamJob {

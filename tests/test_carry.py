@@ -72,3 +72,47 @@ def test_carry_longest_words(A, k):
     assert sum(raw) == (1 << k) * ((1 << k) - 1) // 2
     if A & (A - 1) == 0:
         assert raw[1:k + 1] == [(1 << (k - 1)) * math.comb(k, d) for d in range(1, k + 1)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("A", [1, 3, 61, 63, 65, 12, 129, 511, 513, 1000 * 2 + 1])
+@pytest.mark.parametrize("n,m", [(16, 3), (17, 100), (20, 1001)])
+def test_grid_rows_match_oracle(A, n, m):
+    # the grid over all 2^n words through the recursion over carries (from
+    # about A * n * 80 < 2^n) and, for the longer multipliers, the rectangle kernel
+    import coding_reliability_amd as cra
+    with cra.Context(0) as ctx:
+        hist, _ = ctx.an_grid_ref(1, n, m, 0, A)
+    ref, _, _ = O.an_grid_ref(1, n, m, 0, A)
+    assert hist[: len(ref)] == ref[: len(hist)] and not any(hist[len(ref):])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("A,n", [(3, 33), (61, 40), (1, 48), (513, 26), (40, 34)])
+def test_grid_rows_long_words(A, n):
+    # 32- and 64-bit counters beyond what the oracle enumerates: the recursion
+    # restated with Python integers on the oracle's sample list
+    import coding_reliability_amd as cra
+    m = 4
+    with cra.Context(0) as ctx:
+        hist, _ = ctx.an_grid_ref(1, n, m, 0, A)
+    cfg = O.grid_ref_config(A, n, m, 0, 1)
+    samples = [int(v) for v in O.grid1d_ref_samples(cfg["A"], n, cfg["step"], 3, cfg["cc"] <= 32)]
+    want = [0] * 65
+    z = (A & -A).bit_length() - 1
+    a = A >> z
+    for v in samples:
+        below, w = (v & ((1 << z) - 1)).bit_count(), v >> z
+        G = [[int(b == (c ^ (w >> n)).bit_count()) for b in range(65)] for c in range(a)]
+        for r in range(n):
+            bit = w >> (n - 1 - r) & 1
+            H = []
+            for c in range(a):
+                e = (c & 1) ^ bit
+                p, q = (G[c >> 1], G[(c + a) >> 1]) if e == 0 else (G[(c + a) >> 1], G[c >> 1])
+                H.append([p[b] + (q[b - 1] if b else 0) for b in range(65)])
+            G = H
+        for b, x in enumerate(G[0]):
+            if x:
+                want[b + below] += x
+    assert hist == want[: len(hist)]
