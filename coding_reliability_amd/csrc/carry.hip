@@ -233,23 +233,23 @@ cr_status carry_run(const CarryPlan &p, void *table0, void *table1, unsigned lon
     return CR_OK;
 }
 
-cr_status carry_finish(const CarryPlan &p, const uint64_t *hist, uint64_t *raw, uint32_t nbins) {
-    const uint64_t stride = hist_copy_stride(p.nbins);
+cr_status carry_finish(uint32_t k, uint32_t bins, const uint64_t *hist, uint64_t *raw, uint32_t nbins) {
+    const uint64_t stride = hist_copy_stride(bins);
     unsigned __int128 total = 0;
     for (uint32_t b = 0; b < nbins; ++b) raw[b] = 0;
-    for (uint32_t b = 0; b < p.nbins; ++b) {
+    for (uint32_t b = 0; b < bins; ++b) {
         uint64_t s = 0;
         for (uint32_t c = 0; c < kHistCopies; ++c) s += hist[c * stride + b];
         total += s;
         if (b == 0) {
-            if (s != 1ull << p.k) return fail(CR_ERR_DEVICE, "carry recursion: %llu words at distance 0", (unsigned long long)s);
+            if (s != 1ull << k) return fail(CR_ERR_DEVICE, "carry recursion: %llu words at distance 0", (unsigned long long)s);
         } else if (b >= nbins ? s != 0 : (s & 1) != 0) {
             return fail(CR_ERR_DEVICE, "carry recursion: inconsistent count at distance %u", b);
         } else if (b < nbins) {
             raw[b] = s / 2;
         }
     }
-    if (total != (unsigned __int128)1 << (2 * p.k)) return fail(CR_ERR_DEVICE, "carry recursion: inconsistent total");
+    if (total != (unsigned __int128)1 << (2 * k)) return fail(CR_ERR_DEVICE, "carry recursion: inconsistent total");
     return CR_OK;
 }
 

@@ -87,27 +87,28 @@ bool carry_preferred(uint64_t A, uint64_t num_words, double seconds, CarryPlan *
     return carry_plan(A, (uint32_t)__builtin_ctzll(num_words), p) && p->seconds < seconds;
 }
 
-// The carry recursion on the context's buffers (carry.hip).
-cr_status an_pairs_carry(cr_context *ctx, const CarryPlan &p, uint64_t A, uint64_t *raw, uint32_t nbins,
-                         double *kernel_ms) {
+// A carry recursion on the context's buffers: run(hist) enqueues it with the
+// tables reserved.
+template <class Run>
+cr_status an_pairs_carry(cr_context *ctx, uint64_t A, uint32_t k, uint32_t bins, uint64_t entries, uint64_t table_a,
+                         uint64_t table_b, Run run, uint64_t *raw, uint32_t nbins, double *kernel_ms) {
     clear_error();
     if (!ctx || !raw) return fail(CR_ERR_INVALID_ARGUMENT, "NULL argument");
-    const uint32_t need = pair_max_distance(A, 1ull << p.k) + 1;
+    const uint32_t need = pair_max_distance(A, 1ull << k) + 1;
     if (nbins < need) return fail(CR_ERR_INVALID_ARGUMENT, "nbins=%u but distances reach %u", nbins, need - 1);
     CR_HIP(hipSetDevice(ctx->device));
     const cr_status st = [&]() -> cr_status {
-        CR_TRY(ctx->table_a.reserve(p.table_bytes));
-        CR_TRY(ctx->table_b.reserve(p.table_bytes));
-        CR_TRY(ctx->hist.reserve(p.hist_entries * sizeof(uint64_t)));
-        CR_TRY(ctx->host.reserve(p.hist_entries * sizeof(uint64_t)));
+        CR_TRY(ctx->table_a.reserve(table_a));
+        if (table_b) CR_TRY(ctx->table_b.reserve(table_b));
+        CR_TRY(ctx->hist.reserve(entries * sizeof(uint64_t)));
+        CR_TRY(ctx->host.reserve(entries * sizeof(uint64_t)));
         unsigned long long *hist = ctx->hist.as<unsigned long long>();
         if (kernel_ms) CR_HIP(hipEventRecord(ctx->ev0, ctx->stream));
-        CR_TRY(carry_run(p, ctx->table_a.ptr, ctx->table_b.ptr, hist, ctx->cus, ctx->stream));
+        CR_TRY(run(hist));
         if (kernel_ms) CR_HIP(hipEventRecord(ctx->ev1, ctx->stream));
-        CR_HIP(hipMemcpyAsync(ctx->host.ptr, hist, p.hist_entries * sizeof(uint64_t), hipMemcpyDeviceToHost,
-                              ctx->stream));
+        CR_HIP(hipMemcpyAsync(ctx->host.ptr, hist, entries * sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
         CR_HIP(hipStreamSynchronize(ctx->stream));
-        CR_TRY(carry_finish(p, ctx->host.as<uint64_t>(), raw, nbins));
+        CR_TRY(carry_finish(k, bins, ctx->host.as<uint64_t>(), raw, nbins));
         if (kernel_ms) {
             float ms = 0;
             CR_HIP(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
@@ -117,12 +118,17 @@ cr_status an_pairs_carry(cr_context *ctx, const CarryPlan &p, uint64_t A, uint64
     }();
     // as the transform buffers of the spectral path: a long-lived context
     // does not hold tables above 1 GiB
-    if (p.table_bytes > (1ull << 30)) {
+    if (table_a > (1ull << 30)) {
         (void)hipStreamSynchronize(ctx->stream);
         ctx->table_a.release();
-        ctx->table_b.release();
+        if (table_b) ctx->table_b.release();
     }
     return st;
+}
+
+bool tiles_preferred(uint64_t A, uint64_t num_words, double seconds, CarryTilesPlan *p) {
+    if (num_words == 0 || (num_words & (num_words - 1)) || (unsigned __int128)(num_words - 1) * A >> 64) return false;
+    return carry_tiles_plan(A, (uint32_t)__builtin_ctzll(num_words), p) && p->seconds < seconds;
 }
 
 }  // namespace
@@ -303,7 +309,23 @@ cr_status cr_an_pairs(cr_context *ctx, uint64_t A, uint64_t num_words, uint64_t 
     double best = 40e-6 + (double)num_words * (double)num_words / 14e12;
     const bool spectral = spectral_preferred(A, num_words, &k, &best);
     CarryPlan carry;
-    if (carry_preferred(A, num_words, best, &carry)) return an_pairs_carry(ctx, carry, A, raw, nbins, kernel_ms);
+    const bool recursion = carry_preferred(A, num_words, best, &carry);
+    if (recursion) best = carry.seconds;
+    CarryTilesPlan tiles;
+    if (tiles_preferred(A, num_words, best, &tiles))
+        return an_pairs_carry(
+            ctx, A, tiles.k, tiles.nbins, tiles.hist_entries, tiles.table_bytes, 0,
+            [&](unsigned long long *hist) {
+                return carry_tiles_run(tiles, ctx->table_a.ptr, hist, ctx->cus, ctx->stream);
+            },
+            raw, nbins, kernel_ms);
+    if (recursion)
+        return an_pairs_carry(
+            ctx, A, carry.k, carry.nbins, carry.hist_entries, carry.table_bytes, carry.table_bytes,
+            [&](unsigned long long *hist) {
+                return carry_run(carry, ctx->table_a.ptr, ctx->table_b.ptr, hist, ctx->cus, ctx->stream);
+            },
+            raw, nbins, kernel_ms);
     if (spectral) return cr_an_pairs_spectral(ctx, A, k, raw, nbins, kernel_ms);
     return cr_an_pairs_tuned(ctx, A, num_words, raw, nbins, nullptr, kernel_ms);
 }

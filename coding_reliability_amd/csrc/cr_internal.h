@@ -228,9 +228,24 @@ bool carry_plan(uint64_t A, uint32_t k, CarryPlan *p);
 // Leaves the distribution over ordered pairs in hist (p.hist_entries, cleared here).
 cr_status carry_run(const CarryPlan &p, void *table0, void *table1, unsigned long long *hist, int cus,
                     hipStream_t stream);
-// raw[] (nbins entries, pair-kernel form) from the host copy of hist; checks
-// the words at distance 0 and the total of 4^k.
-cr_status carry_finish(const CarryPlan &p, const uint64_t *hist, uint64_t *raw, uint32_t nbins);
+// raw[] (nbins entries, pair-kernel form) from the host copy of an ordered-pair
+// histogram of 2^k words (dev::kHistCopies copies of `bins`); checks the words
+// at distance 0 and the total of 4^k.
+cr_status carry_finish(uint32_t k, uint32_t bins, const uint64_t *hist, uint64_t *raw, uint32_t nbins);
+
+// The same recursion for long multipliers, by tiles of carry pairs with four
+// levels a kernel (see carry_tiles.hip).
+struct CarryTilesPlan {
+    uint32_t A = 0, k = 0;
+    uint32_t F = 0;             // levels of the second kernel, 0 .. 4
+    uint32_t T = 0;             // low bits taken pair by pair, k - 4 - F
+    uint32_t hb = 0, nbins = 0;
+    uint64_t table_bytes = 0, hist_entries = 0;
+    double seconds = 0;         // estimated time of a call
+};
+bool carry_tiles_plan(uint64_t A, uint32_t k, CarryTilesPlan *p);
+cr_status carry_tiles_run(const CarryTilesPlan &p, void *table, unsigned long long *hist, int cus,
+                          hipStream_t stream);
 
 // Parity masks of the (N,k) extended Hamming codes, truncated to k bits;
 // returns the number of non-overall parity bits.

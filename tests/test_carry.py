@@ -61,6 +61,32 @@ def test_carry_matches_spectrum(A, k):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("A,k", [(999, 16), (1023, 17), (2015, 18), (2017, 18), (4033, 18), (4095 * 4, 18)])
+def test_carry_tiles_match_pair_kernel(A, k):
+    # multipliers at the edges of a block of 2016 carries and of its 32-carry
+    # tiles, several blocks, no to four levels after the table
+    import coding_reliability_amd as cra
+    with cra.Context(0) as ctx:
+        pair, _ = ctx.an_pairs(A, 1 << k)
+        for _ in range(3):
+            assert ctx.an_pairs_auto(A, 1 << k)[0] == pair
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("A,k", [(2047, 19), (4097, 21), (8191, 22), (8193, 22), (16385, 22), (32767, 23), (4033, 24),
+                                 (16385, 24), (65535, 20), (58659, 21), (32769, 23), (58659, 24), (4097, 25)])
+def test_carry_tiles_match_spectrum(A, k):
+    # 12- to 16-bit multipliers; k - 8 more bits than the multiplier has: up to
+    # 32 low parts a carry
+    import coding_reliability_amd as cra
+    with cra.Context(0) as ctx:
+        auto, ms = ctx.an_pairs_auto(A, 1 << k)
+        spec, ms_spec = ctx.an_pairs_spectral(A, k)
+    print(f"A={A} k={k}: {ms:.1f} ms, spectral path {ms_spec:.1f} ms", flush=True)
+    assert auto == spec
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("A,k", [(1, 30), (1 << 9, 32), (3, 32), (511, 32)])
 def test_carry_longest_words(A, k):
     import coding_reliability_amd as cra
