@@ -13,14 +13,28 @@ namespace cr {
 namespace {
 
 struct BatchLayout {
-    std::vector<PairJob> jobs;  // longest code first
+    std::vector<PairJob> jobs;      // codes of the pair kernel, longest first
     PairLaunchConfig cfg;
     uint64_t total_items = 0;
+    std::vector<SlicedJob> sliced;  // codes of the sliced kernel, longest first
+    uint64_t sliced_items = 0;
+    size_t job_bytes() const { return sliced.size() * sizeof(SlicedJob) + jobs.size() * sizeof(PairJob); }
+    // device layout: the sliced jobs, then the pair jobs
+    hipError_t upload(void *d, hipStream_t stream) const {
+        const size_t n = sliced.size() * sizeof(SlicedJob);
+        hipError_t e = n ? hipMemcpyAsync(d, sliced.data(), n, hipMemcpyHostToDevice, stream) : hipSuccess;
+        if (e == hipSuccess && !jobs.empty())
+            e = hipMemcpyAsync(static_cast<char *>(d) + n, jobs.data(), jobs.size() * sizeof(PairJob),
+                               hipMemcpyHostToDevice, stream);
+        return e;
+    }
 };
+static_assert(alignof(PairJob) == alignof(SlicedJob) && sizeof(SlicedJob) % alignof(PairJob) == 0, "job array layout");
 
-// Builds the work list: per code a PairJob writing to d_hist + c*stride, the
-// chunk width chosen so that items carry about total_pairs/(items_per_wave *
-// resident waves) pairs, jobs sorted by pair count (longest first).
+// Builds the work lists, jobs sorted by pair count (longest first), each
+// writing to d_hist + c*stride: codes of 2^k words from k = 11 on go to the
+// sliced kernel, the others to the pair kernel with the chunk width chosen so
+// that items carry about total_pairs/(items_per_wave * resident waves) pairs.
 cr_status build_batch(cr_context *ctx, const cr_an_code *codes, uint32_t ncodes, uint32_t stride,
                       const cr_pair_tuning *tuning, unsigned long long *d_hist, BatchLayout &L) {
     if (!codes || ncodes == 0) return fail(CR_ERR_INVALID_ARGUMENT, "empty batch");
@@ -28,6 +42,7 @@ cr_status build_batch(cr_context *ctx, const cr_an_code *codes, uint32_t ncodes,
     const uint32_t ipw = tuning && tuning->items_per_wave ? tuning->items_per_wave : 16;
     uint32_t max_need = 0;
     long double total_pairs = 0;
+    L.jobs.reserve(ncodes);
     for (uint32_t c = 0; c < ncodes; ++c) {
         const uint64_t A = codes[c].A, N = codes[c].num_words;
         if (A == 0 || N == 0) return fail(CR_ERR_INVALID_ARGUMENT, "code %u: A and num_words must be >= 1", c);
@@ -35,10 +50,24 @@ cr_status build_batch(cr_context *ctx, const cr_an_code *codes, uint32_t ncodes,
         const uint32_t need = pair_max_distance(A, N) + 1;
         if (need > stride) return fail(CR_ERR_INVALID_ARGUMENT, "code %u needs %u bins > stride %u", c, need, stride);
         max_need = std::max(max_need, need);
+        SlicedJob sj;
+        if (sliced_job(A, N, &sj)) {
+            sj.out = d_hist + (size_t)c * stride;
+            sj.nbins = need;
+            L.sliced.push_back(sj);
+            continue;
+        }
+        PairJob j{};
+        j.A = A;
+        j.N = N;
+        j.out = d_hist + (size_t)c * stride;
+        j.nbins = need;
+        L.jobs.push_back(j);
+        max_need = std::max(max_need, need);
         total_pairs += (long double)N * (long double)(N - 1) / 2;
     }
     L.cfg.R = R;
-    L.cfg.lds_rows = max_need + 1;
+    L.cfg.lds_rows = std::max(max_need, 1u) + 1;
     L.cfg.waves = tuning ? tuning->waves : 0;
     const uint32_t per_cu = pair_waves_per_cu(R, L.cfg.lds_rows);
     if (per_cu == 0) return fail(CR_ERR_INVALID_ARGUMENT, "rows_per_lane must be 2, 4, 8 or 16 (got %u)", R);
@@ -46,15 +75,8 @@ cr_status build_batch(cr_context *ctx, const cr_an_code *codes, uint32_t ncodes,
     const long double target = std::max<long double>(total_pairs / (ipw * waves), 1.0L);
     const uint64_t RB = 64ull * R;
     const uint64_t qmax = std::max<uint64_t>(((1ull << 30) / R) / RB, 1);
-    L.jobs.resize(ncodes);
-    for (uint32_t c = 0; c < ncodes; ++c) {
-        PairJob &j = L.jobs[c];
-        j = PairJob{};
-        j.A = codes[c].A;
-        j.N = codes[c].num_words;
+    for (PairJob &j : L.jobs) {
         j.mode = pair_mode(j.A, j.N);
-        j.nbins = pair_max_distance(j.A, j.N) + 1;
-        j.out = d_hist + (size_t)c * stride;
         uint64_t Q = (uint64_t)(target / ((long double)RB * RB));
         Q = std::min<uint64_t>(std::max<uint64_t>(Q, 1), qmax);
         pair_job_geometry(j, R, (uint32_t)Q);
@@ -68,6 +90,22 @@ cr_status build_batch(cr_context *ctx, const cr_an_code *codes, uint32_t ncodes,
         total += j.items;
     }
     L.total_items = total;
+    std::stable_sort(L.sliced.begin(), L.sliced.end(),
+                     [](const SlicedJob &a, const SlicedJob &b) { return a.k > b.k; });
+    sliced_ranges(L.sliced, ctx->cus, &L.sliced_items);
+    return CR_OK;
+}
+
+// Both launches; counters: two work-queue heads.
+cr_status launch_batch(cr_context *ctx, const BatchLayout &L, void *d_jobs, unsigned long long *counters) {
+    const SlicedJob *sliced = static_cast<const SlicedJob *>(d_jobs);
+    if (!L.sliced.empty()) {
+        CR_TRY(fill_zero_u64(counters + 1, 1, ctx->stream));
+        CR_TRY(launch_sliced(sliced, (uint32_t)L.sliced.size(), L.sliced_items, counters + 1, ctx->cus, ctx->stream));
+    }
+    if (!L.jobs.empty())
+        CR_TRY(launch_pairs(reinterpret_cast<const PairJob *>(sliced + L.sliced.size()), (uint32_t)L.jobs.size(),
+                            L.total_items, counters, L.cfg, ctx->cus, ctx->stream, nullptr, nullptr));
     return CR_OK;
 }
 
@@ -97,14 +135,13 @@ cr_status cr_an_batch(cr_context *ctx, const cr_an_code *codes, uint32_t ncodes,
     CR_TRY(ctx->hist.reserve(n * sizeof(uint64_t)));
     BatchLayout L;
     CR_TRY(build_batch(ctx, codes, ncodes, stride, tuning, ctx->hist.as<unsigned long long>(), L));
-    CR_TRY(ctx->jobs.reserve(L.jobs.size() * sizeof(PairJob)));
-    CR_TRY(ctx->counters.reserve(sizeof(uint64_t)));
+    CR_TRY(ctx->jobs.reserve(L.job_bytes()));
+    CR_TRY(ctx->counters.reserve(2 * sizeof(uint64_t)));
     CR_TRY(fill_zero_u64(ctx->hist.as<unsigned long long>(), n, ctx->stream));
-    CR_HIP(hipMemcpyAsync(ctx->jobs.ptr, L.jobs.data(), L.jobs.size() * sizeof(PairJob), hipMemcpyHostToDevice,
-                          ctx->stream));
-    CR_TRY(launch_pairs(ctx->jobs.as<PairJob>(), (uint32_t)L.jobs.size(), L.total_items,
-                        ctx->counters.as<unsigned long long>(), L.cfg, ctx->cus, ctx->stream,
-                        kernel_ms ? ctx->ev0 : nullptr, kernel_ms ? ctx->ev1 : nullptr));
+    CR_HIP(L.upload(ctx->jobs.ptr, ctx->stream));
+    if (kernel_ms) CR_HIP(hipEventRecord(ctx->ev0, ctx->stream));
+    CR_TRY(launch_batch(ctx, L, ctx->jobs.ptr, ctx->counters.as<unsigned long long>()));
+    if (kernel_ms) CR_HIP(hipEventRecord(ctx->ev1, ctx->stream));
     CR_TRY(ctx->host.reserve(n * sizeof(uint64_t)));
     CR_HIP(hipMemcpyAsync(ctx->host.ptr, ctx->hist.ptr, n * sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
     CR_HIP(hipStreamSynchronize(ctx->stream));
@@ -147,21 +184,20 @@ cr_status cr_batch_plan_create(cr_context *ctx, const cr_an_code *codes, uint32_
     const size_t n = (size_t)ncodes * stride;
     cr_status s;
     if ((s = p->hist.reserve(n * sizeof(uint64_t))) != CR_OK) return bail(s);
-    if ((s = p->counter.reserve(sizeof(uint64_t))) != CR_OK) return bail(s);
+    if ((s = p->counter.reserve(2 * sizeof(uint64_t))) != CR_OK) return bail(s);
     if ((s = p->host.reserve(n * sizeof(uint64_t))) != CR_OK) return bail(s);
     BatchLayout L;
     if ((s = build_batch(ctx, codes, ncodes, stride, tuning, p->hist.as<unsigned long long>(), L)) != CR_OK)
         return bail(s);
-    if ((s = p->jobs.reserve(L.jobs.size() * sizeof(PairJob))) != CR_OK) return bail(s);
-    hipError_t e = hipMemcpy(p->jobs.ptr, L.jobs.data(), L.jobs.size() * sizeof(PairJob), hipMemcpyHostToDevice);
+    if ((s = p->jobs.reserve(L.job_bytes())) != CR_OK) return bail(s);
+    hipError_t e = L.upload(p->jobs.ptr, ctx->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);  // L goes with this call
     if (e != hipSuccess) return bail(fail(CR_ERR_DEVICE, "job upload failed: %s", hipGetErrorString(e)));
-    // capture: zero histograms, zero queue head + pair kernel, copy back
+    // capture: zero histograms, zero queue heads + kernels, copy back
     e = hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return bail(fail(CR_ERR_DEVICE, "graph capture failed: %s", hipGetErrorString(e)));
     cr_status cs = fill_zero_u64(p->hist.as<unsigned long long>(), n, ctx->stream);
-    if (cs == CR_OK)
-        cs = launch_pairs(p->jobs.as<PairJob>(), (uint32_t)L.jobs.size(), L.total_items,
-                          p->counter.as<unsigned long long>(), L.cfg, ctx->cus, ctx->stream, nullptr, nullptr);
+    if (cs == CR_OK) cs = launch_batch(ctx, L, p->jobs.ptr, p->counter.as<unsigned long long>());
     if (cs == CR_OK) {
         e = hipMemcpyAsync(p->host.ptr, p->hist.ptr, n * sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream);
         if (e != hipSuccess) cs = fail(CR_ERR_DEVICE, "capture of copy-back failed: %s", hipGetErrorString(e));

@@ -126,6 +126,49 @@ cr_status an_pairs_carry(cr_context *ctx, uint64_t A, uint32_t k, uint32_t bins,
     return st;
 }
 
+// One code through the sliced kernel.
+cr_status an_pairs_sliced(cr_context *ctx, const SlicedJob &code, uint64_t A, uint64_t num_words, uint64_t *raw,
+                          uint32_t nbins, double *kernel_ms) {
+    clear_error();
+    if (!ctx || !raw) return fail(CR_ERR_INVALID_ARGUMENT, "NULL argument");
+    const uint32_t need = pair_max_distance(A, num_words) + 1;
+    if (nbins < need) return fail(CR_ERR_INVALID_ARGUMENT, "nbins=%u but distances reach %u", nbins, need - 1);
+    CR_HIP(hipSetDevice(ctx->device));
+    std::vector<SlicedJob> jobs(1, code);
+    uint64_t items = 0;
+    sliced_ranges(jobs, ctx->cus, &items);
+    SlicedJob &job = jobs[0];
+    job.nbins = need;
+    job.out_copies = dev::kHistCopies;
+    // as cr_an_pairs_tuned: the histogram copies and the queue head, cleared
+    // by one fill; pinned: the job descriptor at 0, the copies from 256
+    constexpr size_t kHostResult = 256;
+    static_assert(sizeof(SlicedJob) <= kHostResult, "job staging");
+    const uint64_t cstride = dev::hist_copy_stride(need), entries = cstride * job.out_copies;
+    CR_TRY(ctx->hist.reserve((entries + 1) * sizeof(uint64_t)));
+    CR_TRY(ctx->jobs.reserve(sizeof(SlicedJob)));
+    CR_TRY(ctx->host.reserve(kHostResult + entries * sizeof(uint64_t)));
+    job.out = ctx->hist.as<unsigned long long>();
+    memcpy(ctx->host.ptr, &job, sizeof(job));
+    CR_TRY(fill_zero_u64(job.out, entries + 1, ctx->stream));
+    CR_HIP(hipMemcpyAsync(ctx->jobs.ptr, ctx->host.ptr, sizeof(SlicedJob), hipMemcpyHostToDevice, ctx->stream));
+    if (kernel_ms) CR_HIP(hipEventRecord(ctx->ev0, ctx->stream));
+    CR_TRY(launch_sliced(ctx->jobs.as<SlicedJob>(), 1, items, job.out + entries, ctx->cus, ctx->stream));
+    if (kernel_ms) CR_HIP(hipEventRecord(ctx->ev1, ctx->stream));
+    const uint64_t *res = reinterpret_cast<const uint64_t *>(ctx->host.as<char>() + kHostResult);
+    CR_HIP(hipMemcpyAsync((void *)res, job.out, entries * sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
+    CR_HIP(hipStreamSynchronize(ctx->stream));
+    memset(raw, 0, nbins * sizeof(uint64_t));
+    for (uint32_t b = 0; b < need; ++b)
+        for (uint32_t c = 0; c < job.out_copies; ++c) raw[b] += res[c * cstride + b];
+    if (kernel_ms) {
+        float ms = 0;
+        CR_HIP(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
+        *kernel_ms = ms;
+    }
+    return CR_OK;
+}
+
 bool tiles_preferred(uint64_t A, uint64_t num_words, double seconds, CarryTilesPlan *p) {
     if (num_words == 0 || (num_words & (num_words - 1)) || (unsigned __int128)(num_words - 1) * A >> 64) return false;
     return carry_tiles_plan(A, (uint32_t)__builtin_ctzll(num_words), p) && p->seconds < seconds;
@@ -304,10 +347,22 @@ cr_status cr_an_pairs(cr_context *ctx, uint64_t A, uint64_t num_words, uint64_t 
                       double *kernel_ms) {
     // the same histogram by whichever method is estimated to be the fastest:
     // the pair kernel (measured 40 us a call and about 7e12 pairs/s where it
-    // competes), the code's spectrum, the recursion over carries
+    // competes, up to 2^13 words), the sliced kernel (45 us a call and the
+    // rates of sliced_rate), the code's spectrum, the recursions over carries
     uint32_t k = 0;
-    double best = 40e-6 + (double)num_words * (double)num_words / 14e12;
-    const bool spectral = spectral_preferred(A, num_words, &k, &best);
+    const double pairs = 0.5 * (double)num_words * (double)num_words;
+    double best = 40e-6 + pairs / 7e12;
+    SlicedJob sliced;
+    bool by_planes = false;
+    if (sliced_job(A, num_words, &sliced)) {
+        const double s = 45e-6 + pairs / sliced_rate(sliced);
+        by_planes = s < best;
+        best = std::min(best, s);
+    }
+    const double pairwise = best;
+    double spectral_s = 0;
+    const bool spectral = spectral_preferred(A, num_words, &k, &spectral_s);
+    if (spectral) best = std::min(best, spectral_s);
     CarryPlan carry;
     const bool recursion = carry_preferred(A, num_words, best, &carry);
     if (recursion) best = carry.seconds;
@@ -326,7 +381,8 @@ cr_status cr_an_pairs(cr_context *ctx, uint64_t A, uint64_t num_words, uint64_t 
                 return carry_run(carry, ctx->table_a.ptr, ctx->table_b.ptr, hist, ctx->cus, ctx->stream);
             },
             raw, nbins, kernel_ms);
-    if (spectral) return cr_an_pairs_spectral(ctx, A, k, raw, nbins, kernel_ms);
+    if (spectral && spectral_s < pairwise) return cr_an_pairs_spectral(ctx, A, k, raw, nbins, kernel_ms);
+    if (by_planes) return an_pairs_sliced(ctx, sliced, A, num_words, raw, nbins, kernel_ms);
     return cr_an_pairs_tuned(ctx, A, num_words, raw, nbins, nullptr, kernel_ms);
 }
 

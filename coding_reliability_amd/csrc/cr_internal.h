@@ -132,6 +132,28 @@ cr_status launch_pairs(const PairJob *d_jobs, uint32_t njobs, uint64_t total_ite
 // lane and `lds_rows` histogram rows.
 uint32_t pair_waves_per_cu(uint32_t R, uint32_t lds_rows);
 
+// Pair histograms of whole codes by bit planes (see sliced_pairs.hip).
+struct SlicedJob {
+    uint64_t item_begin, items;  // global range of the job's items in the launch
+    unsigned long long *out;     // device histogram, nbins entries, accumulated with atomics
+    uint32_t A, Ainv, tc;        // odd part, its inverse modulo 2^k, (A * Ainv - 1) >> k
+    uint32_t k;                  // word bits, 11 .. 24
+    uint32_t planes;             // codeword bits above the low k, at most 16
+    uint32_t parts;              // items that share a 64 x 64 block of words: 1, 2 or 4
+    uint32_t nbins, out_copies;  // as PairJob's
+};
+static_assert(sizeof(SlicedJob) == 56, "SlicedJob layout");
+// False when (A, num_words) is outside the kernel.
+bool sliced_job(uint64_t A, uint64_t num_words, SlicedJob *j);
+// Measured pairs per second of a launch that fills the device.
+double sliced_rate(const SlicedJob &j);
+// Fills parts, items and item_begin of the jobs of one launch, in order.
+void sliced_ranges(std::vector<SlicedJob> &jobs, int cus, uint64_t *total_items);
+// counter: the work-queue head, zeroed by the caller, or null for a static
+// assignment of items to workgroups.
+cr_status launch_sliced(const SlicedJob *d_jobs, uint32_t njobs, uint64_t total_items, unsigned long long *counter,
+                        int cus, hipStream_t stream);
+
 // Rectangle histogram rows x column table (see rect_pairs.hip).
 struct RectLaunch {
     uint64_t A = 1, row0 = 0, nrows = 0;
