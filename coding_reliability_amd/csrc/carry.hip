@@ -47,13 +47,12 @@ constexpr uint32_t kStepBins = 4;    // distances per thread of carry_step
 constexpr uint64_t kMaxTable = 1ull << 31;
 constexpr uint32_t kFinalBins = 64;  // distances of a carry_final histogram
 
-// Q_{kInitBits} for 64 carry pairs a wave; workgroup 0 clears the result too.
+// Q_{kInitBits} for 64 carry pairs a wave.
 __global__ __launch_bounds__(64) void carry_init(uint32_t *__restrict__ T, uint32_t A, uint32_t states, uint32_t nb,
-                                                 unsigned long long *__restrict__ hist, uint32_t entries) {
+                                                 const DirectResult out) {
     __shared__ uint32_t lds[kInitRows * kStride];
     const uint32_t lane = threadIdx.x;
-    if (blockIdx.x == 0)
-        for (uint32_t e = lane; e < entries; e += 64) hist[e] = 0;
+    direct_start(out);
     lds_clear(lds, kInitRows);
     const uint32_t s = blockIdx.x * 64 + lane;
     if (s >= states) return;
@@ -121,7 +120,8 @@ __global__ __launch_bounds__(256) void carry_step(const In *__restrict__ Q, Out 
 template <class In>
 __global__ __launch_bounds__(64) void carry_final(const In *__restrict__ Q, uint32_t A, uint32_t Ainv, uint32_t T,
                                                   uint32_t states, uint32_t nb, uint32_t nbins,
-                                                  unsigned long long *__restrict__ out) {
+                                                  const DirectResult out) {
+    __shared__ uint32_t flag;
     __shared__ unsigned long long lds[kFinalBins * kStride];  // 32 KB
     const uint32_t lane = threadIdx.x;
     for (uint32_t b = 0; b < kFinalBins; ++b) lds[b * kStride + lane] = 0;
@@ -139,12 +139,13 @@ __global__ __launch_bounds__(64) void carry_final(const In *__restrict__ Q, uint
             lds[(e + b) * kStride + lane] += (unsigned long long)q[(uint64_t)b * states] << w;
     }
     __syncthreads();
-    unsigned long long *const dst = hist_copy(out, nbins, kHistCopies);
+    unsigned long long *const dst = hist_copy(out.copies, nbins, kHistCopies);
     for (uint32_t b = lane; b < nbins; b += 64) {
         unsigned long long s = 0;
         for (uint32_t l = 0; l < 64; ++l) s += lds[b * kStride + ((l + lane) & 63u)];
         if (s) atomicAdd(dst + b, s);
     }
+    direct_finish(out, nbins, &flag);
 }
 
 template <int F, class In, class Out>
@@ -188,25 +189,24 @@ bool carry_plan(uint64_t A, uint32_t k, CarryPlan *p) {
     if (p->nbins > kFinalBins) return false;
     const uint64_t nb = p->levels + p->hb + 1;
     p->table_bytes = (uint64_t)p->states * nb * (wide(p->levels) ? 8 : 4);
-    p->hist_entries = hist_copy_stride(p->nbins) * kHistCopies;
     // Host and launch time of a call, then measured kernel rates (A = 511 and
     // 1021, k = 14 .. 32): 100 ps a carry pair for the first and the last
     // kernel, 6.5 ps a counter for two levels in 32 bits, 11 ps in 64.
-    double s = 30e-6 + 1.0e-10 * p->states;
+    double s = 28e-6 + 1.0e-10 * p->states;
     for (uint32_t r = kInitBits; r < p->levels;) {
         r += ((p->levels - r) & 1) ? 1 : 2;
-        s += 4.5e-6 + (wide(r) ? 11e-12 : 6.5e-12) * (double)p->states * (r + p->hb + 1);
+        s += 5.5e-6 + (wide(r) ? 11e-12 : 6.5e-12) * (double)p->states * (r + p->hb + 1);
     }
     p->seconds = s;
     return p->table_bytes <= kMaxTable;
 }
 
-cr_status carry_run(const CarryPlan &p, void *table0, void *table1, unsigned long long *hist, int cus,
+cr_status carry_run(const CarryPlan &p, void *table0, void *table1, const DirectResult &out, int cus,
                     hipStream_t stream) {
     uint32_t nb = kInitBits + p.hb + 1;
     if (nb > kInitRows) return fail(CR_ERR_DEVICE, "carry recursion: %u distances", nb);
     hipLaunchKernelGGL(carry_init, dim3((p.states + 63) / 64), dim3(64), 0, stream, (uint32_t *)table0, p.A, p.states,
-                       nb, hist, (uint32_t)p.hist_entries);
+                       nb, out);
     CR_HIP(hipGetLastError());
     void *Q = table0, *T = table1;
     uint32_t r = kInitBits;
@@ -225,21 +225,22 @@ cr_status carry_run(const CarryPlan &p, void *table0, void *table1, unsigned lon
     const uint32_t blocks = (uint32_t)std::min<uint64_t>(tiles, 4ull * cus);
     if (wide(r))
         hipLaunchKernelGGL(carry_final<unsigned long long>, dim3(blocks), dim3(64), 0, stream,
-                           (const unsigned long long *)Q, p.A, p.Ainv, p.T, p.states, nb, p.nbins, hist);
+                           (const unsigned long long *)Q, p.A, p.Ainv, p.T, p.states, nb, p.nbins, out);
     else
         hipLaunchKernelGGL(carry_final<uint32_t>, dim3(blocks), dim3(64), 0, stream, (const uint32_t *)Q, p.A, p.Ainv,
-                           p.T, p.states, nb, p.nbins, hist);
+                           p.T, p.states, nb, p.nbins, out);
     CR_HIP(hipGetLastError());
     return CR_OK;
 }
 
-cr_status carry_finish(uint32_t k, uint32_t bins, const uint64_t *hist, uint64_t *raw, uint32_t nbins) {
+cr_status carry_finish(uint32_t k, uint32_t bins, const uint64_t *hist, uint32_t copies, uint64_t *raw,
+                       uint32_t nbins) {
     const uint64_t stride = hist_copy_stride(bins);
     unsigned __int128 total = 0;
     for (uint32_t b = 0; b < nbins; ++b) raw[b] = 0;
     for (uint32_t b = 0; b < bins; ++b) {
         uint64_t s = 0;
-        for (uint32_t c = 0; c < kHistCopies; ++c) s += hist[c * stride + b];
+        for (uint32_t c = 0; c < copies; ++c) s += hist[c * stride + b];
         total += s;
         if (b == 0) {
             if (s != 1ull << k) return fail(CR_ERR_DEVICE, "carry recursion: %llu words at distance 0", (unsigned long long)s);

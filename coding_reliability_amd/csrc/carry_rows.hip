@@ -37,8 +37,9 @@ constexpr uint32_t kLdsBytes = 150 << 10;  // of the 160 KB of a CU
 template <class T>
 __global__ __launch_bounds__(1024) void carry_rows(uint32_t A, uint32_t z, uint32_t n,
                                                    const uint64_t *__restrict__ cols, uint32_t ncols, uint32_t rows,
-                                                   uint32_t nbins, unsigned long long *__restrict__ out) {
+                                                   uint32_t nbins, const DirectResult out) {
     extern __shared__ unsigned char lds_raw[];
+    direct_start(out);
     T *const G = reinterpret_cast<T *>(lds_raw);
     const uint32_t c = threadIdx.x, P = blockDim.x;
     const bool act = c < A;
@@ -79,7 +80,8 @@ __global__ __launch_bounds__(1024) void carry_rows(uint32_t A, uint32_t z, uint3
         if (c < nbins && c >= below) acc += G[(c - below) * P];
         __syncthreads();
     }
-    if (c < nbins && acc) atomicAdd(hist_copy(out, nbins, kHistCopies) + c, acc);
+    if (c < nbins && acc) atomicAdd(hist_copy(out.copies, nbins, kHistCopies) + c, acc);
+    direct_finish(out, nbins, reinterpret_cast<uint32_t *>(lds_raw));
 }
 
 }  // namespace
@@ -107,18 +109,16 @@ bool carry_rows_plan(uint64_t A, uint32_t n, uint64_t ncols, uint32_t nbins, Car
 }
 
 cr_status launch_carry_rows(const CarryRowsPlan &p, const uint64_t *cols, uint32_t ncols, uint32_t nbins,
-                            unsigned long long *out, int cus, hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1) {
+                            const DirectResult &out, int cus, hipStream_t stream) {
     const void *k = p.wide ? reinterpret_cast<const void *>(&carry_rows<unsigned long long>)
                            : reinterpret_cast<const void *>(&carry_rows<uint32_t>);
     int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, (int)p.threads, p.lds) != hipSuccess || per_cu <= 0)
         return fail(CR_ERR_DEVICE, "occupancy query failed for the carry rows kernel");
     const uint32_t blocks = std::min<uint32_t>(ncols, (uint32_t)per_cu * (uint32_t)cus);
-    if (ev0) CR_HIP(hipEventRecord(ev0, stream));
     uint32_t a_A = p.A, a_z = p.z, a_n = p.n, a_nc = ncols, a_rows = p.rows, a_nb = nbins;
-    void *args[] = {&a_A, &a_z, &a_n, (void *)&cols, &a_nc, &a_rows, &a_nb, &out};
+    void *args[] = {&a_A, &a_z, &a_n, (void *)&cols, &a_nc, &a_rows, &a_nb, (void *)&out};
     CR_HIP(hipLaunchKernel(k, dim3(blocks), dim3(p.threads), args, p.lds, stream));
-    if (ev1) CR_HIP(hipEventRecord(ev1, stream));
     return CR_OK;
 }
 

@@ -79,6 +79,35 @@ void auto_pair_tuning(uint64_t N, uint32_t resident_waves, uint32_t &R, uint32_t
 }  // namespace cr
 
 namespace cr {
+
+cr_status direct_result(cr_context *ctx, dev::DirectResult *r) {
+    if (!ctx->direct.ptr) {
+        CR_TRY(ctx->direct.reserve(dev::kDirectEntries * sizeof(uint64_t)));
+        const cr_status s = fill_zero_u64(ctx->direct.as<unsigned long long>(), dev::kDirectEntries, ctx->stream);
+        if (s != CR_OK) {
+            ctx->direct.release();
+            return s;
+        }
+    }
+    CR_TRY(ctx->host.reserve((dev::kDirectBins + 2) * sizeof(uint64_t)));
+    r->copies = ctx->direct.as<unsigned long long>();
+    r->queue = r->copies + dev::kDirectEntries - 2;
+    r->ticket = reinterpret_cast<unsigned int *>(r->queue + 1);
+    r->host = ctx->host.as<unsigned long long>();
+    return CR_OK;
+}
+
+cr_status direct_wait(cr_context *ctx, uint64_t *raw, uint32_t need, uint32_t nbins, double *kernel_ms) {
+    CR_HIP(hipStreamSynchronize(ctx->stream));
+    memcpy(raw, ctx->host.ptr, need * sizeof(uint64_t));
+    memset(raw + need, 0, (nbins - need) * sizeof(uint64_t));
+    if (kernel_ms) {
+        const uint64_t *clock = ctx->host.as<uint64_t>() + dev::kDirectBins;
+        *kernel_ms = (double)std::max<int64_t>((int64_t)(clock[1] - clock[0]), 1) / ctx->wall_khz;
+    }
+    return CR_OK;
+}
+
 namespace {
 
 // 2^k words, inside the carry recursion, and estimated below `seconds`
@@ -87,43 +116,72 @@ bool carry_preferred(uint64_t A, uint64_t num_words, double seconds, CarryPlan *
     return carry_plan(A, (uint32_t)__builtin_ctzll(num_words), p) && p->seconds < seconds;
 }
 
-// A carry recursion on the context's buffers: run(hist) enqueues it with the
-// tables reserved.
-template <class Run>
-cr_status an_pairs_carry(cr_context *ctx, uint64_t A, uint32_t k, uint32_t bins, uint64_t entries, uint64_t table_a,
-                         uint64_t table_b, Run run, uint64_t *raw, uint32_t nbins, double *kernel_ms) {
+// The carry recursion on the context's buffers (carry.hip).
+cr_status an_pairs_carry(cr_context *ctx, const CarryPlan &p, uint64_t A, uint64_t *raw, uint32_t nbins,
+                         double *kernel_ms) {
     clear_error();
     if (!ctx || !raw) return fail(CR_ERR_INVALID_ARGUMENT, "NULL argument");
-    const uint32_t need = pair_max_distance(A, 1ull << k) + 1;
+    const uint32_t need = pair_max_distance(A, 1ull << p.k) + 1;
     if (nbins < need) return fail(CR_ERR_INVALID_ARGUMENT, "nbins=%u but distances reach %u", nbins, need - 1);
     CR_HIP(hipSetDevice(ctx->device));
     const cr_status st = [&]() -> cr_status {
-        CR_TRY(ctx->table_a.reserve(table_a));
-        if (table_b) CR_TRY(ctx->table_b.reserve(table_b));
-        CR_TRY(ctx->hist.reserve(entries * sizeof(uint64_t)));
-        CR_TRY(ctx->host.reserve(entries * sizeof(uint64_t)));
-        unsigned long long *hist = ctx->hist.as<unsigned long long>();
-        if (kernel_ms) CR_HIP(hipEventRecord(ctx->ev0, ctx->stream));
-        CR_TRY(run(hist));
-        if (kernel_ms) CR_HIP(hipEventRecord(ctx->ev1, ctx->stream));
-        CR_HIP(hipMemcpyAsync(ctx->host.ptr, hist, entries * sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
-        CR_HIP(hipStreamSynchronize(ctx->stream));
-        CR_TRY(carry_finish(k, bins, ctx->host.as<uint64_t>(), raw, nbins));
-        if (kernel_ms) {
-            float ms = 0;
-            CR_HIP(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
-            *kernel_ms = ms;
-        }
-        return CR_OK;
+        CR_TRY(ctx->table_a.reserve(p.table_bytes));
+        CR_TRY(ctx->table_b.reserve(p.table_bytes));
+        dev::DirectResult out;
+        CR_TRY(direct_result(ctx, &out));
+        CR_TRY(carry_run(p, ctx->table_a.ptr, ctx->table_b.ptr, out, ctx->cus, ctx->stream));
+        uint64_t ordered[dev::kDirectBins];
+        CR_TRY(direct_wait(ctx, ordered, p.nbins, p.nbins, kernel_ms));
+        return carry_finish(p.k, p.nbins, ordered, 1, raw, nbins);
     }();
     // as the transform buffers of the spectral path: a long-lived context
     // does not hold tables above 1 GiB
-    if (table_a > (1ull << 30)) {
+    if (p.table_bytes > (1ull << 30)) {
         (void)hipStreamSynchronize(ctx->stream);
         ctx->table_a.release();
-        if (table_b) ctx->table_b.release();
+        ctx->table_b.release();
     }
     return st;
+}
+
+// The same by tiles (carry_tiles.hip).
+cr_status an_pairs_tiles(cr_context *ctx, const CarryTilesPlan &p, uint64_t A, uint64_t *raw, uint32_t nbins,
+                         double *kernel_ms) {
+    clear_error();
+    if (!ctx || !raw) return fail(CR_ERR_INVALID_ARGUMENT, "NULL argument");
+    const uint32_t need = pair_max_distance(A, 1ull << p.k) + 1;
+    if (nbins < need) return fail(CR_ERR_INVALID_ARGUMENT, "nbins=%u but distances reach %u", nbins, need - 1);
+    CR_HIP(hipSetDevice(ctx->device));
+    CR_TRY(ctx->table_a.reserve(p.table_bytes));
+    CR_TRY(ctx->hist.reserve(p.hist_entries * sizeof(uint64_t)));
+    CR_TRY(ctx->host.reserve(p.hist_entries * sizeof(uint64_t)));
+    unsigned long long *hist = ctx->hist.as<unsigned long long>();
+    if (kernel_ms) CR_HIP(hipEventRecord(ctx->ev0, ctx->stream));
+    CR_TRY(carry_tiles_run(p, ctx->table_a.ptr, hist, ctx->cus, ctx->stream));
+    if (kernel_ms) CR_HIP(hipEventRecord(ctx->ev1, ctx->stream));
+    CR_HIP(hipMemcpyAsync(ctx->host.ptr, hist, p.hist_entries * sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
+    CR_HIP(hipStreamSynchronize(ctx->stream));
+    CR_TRY(carry_finish(p.k, p.nbins, ctx->host.as<uint64_t>(), dev::kHistCopies, raw, nbins));
+    if (kernel_ms) {
+        float ms = 0;
+        CR_HIP(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
+        *kernel_ms = ms;
+    }
+    return CR_OK;
+}
+
+// A short code in one launch.
+cr_status an_pairs_short(cr_context *ctx, uint64_t A, uint64_t num_words, uint64_t *raw, uint32_t nbins,
+                         double *kernel_ms) {
+    clear_error();
+    if (!ctx || !raw) return fail(CR_ERR_INVALID_ARGUMENT, "NULL argument");
+    const uint32_t need = pair_max_distance(A, num_words) + 1;
+    if (nbins < need) return fail(CR_ERR_INVALID_ARGUMENT, "nbins=%u but distances reach %u", nbins, need - 1);
+    CR_HIP(hipSetDevice(ctx->device));
+    dev::DirectResult out;
+    CR_TRY(direct_result(ctx, &out));
+    CR_TRY(launch_short_pairs(A, (uint32_t)num_words, need, out, ctx->cus, ctx->stream));
+    return direct_wait(ctx, raw, need, nbins, kernel_ms);
 }
 
 // One code through the sliced kernel.
@@ -138,35 +196,13 @@ cr_status an_pairs_sliced(cr_context *ctx, const SlicedJob &code, uint64_t A, ui
     uint64_t items = 0;
     sliced_ranges(jobs, ctx->cus, &items);
     SlicedJob &job = jobs[0];
+    dev::DirectResult out;
+    CR_TRY(direct_result(ctx, &out));
     job.nbins = need;
     job.out_copies = dev::kHistCopies;
-    // as cr_an_pairs_tuned: the histogram copies and the queue head, cleared
-    // by one fill; pinned: the job descriptor at 0, the copies from 256
-    constexpr size_t kHostResult = 256;
-    static_assert(sizeof(SlicedJob) <= kHostResult, "job staging");
-    const uint64_t cstride = dev::hist_copy_stride(need), entries = cstride * job.out_copies;
-    CR_TRY(ctx->hist.reserve((entries + 1) * sizeof(uint64_t)));
-    CR_TRY(ctx->jobs.reserve(sizeof(SlicedJob)));
-    CR_TRY(ctx->host.reserve(kHostResult + entries * sizeof(uint64_t)));
-    job.out = ctx->hist.as<unsigned long long>();
-    memcpy(ctx->host.ptr, &job, sizeof(job));
-    CR_TRY(fill_zero_u64(job.out, entries + 1, ctx->stream));
-    CR_HIP(hipMemcpyAsync(ctx->jobs.ptr, ctx->host.ptr, sizeof(SlicedJob), hipMemcpyHostToDevice, ctx->stream));
-    if (kernel_ms) CR_HIP(hipEventRecord(ctx->ev0, ctx->stream));
-    CR_TRY(launch_sliced(ctx->jobs.as<SlicedJob>(), 1, items, job.out + entries, ctx->cus, ctx->stream));
-    if (kernel_ms) CR_HIP(hipEventRecord(ctx->ev1, ctx->stream));
-    const uint64_t *res = reinterpret_cast<const uint64_t *>(ctx->host.as<char>() + kHostResult);
-    CR_HIP(hipMemcpyAsync((void *)res, job.out, entries * sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
-    CR_HIP(hipStreamSynchronize(ctx->stream));
-    memset(raw, 0, nbins * sizeof(uint64_t));
-    for (uint32_t b = 0; b < need; ++b)
-        for (uint32_t c = 0; c < job.out_copies; ++c) raw[b] += res[c * cstride + b];
-    if (kernel_ms) {
-        float ms = 0;
-        CR_HIP(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
-        *kernel_ms = ms;
-    }
-    return CR_OK;
+    job.out = out.copies;
+    CR_TRY(launch_sliced_direct(job, items, out, ctx->cus, ctx->stream));
+    return direct_wait(ctx, raw, need, nbins, kernel_ms);
 }
 
 bool tiles_preferred(uint64_t A, uint64_t num_words, double seconds, CarryTilesPlan *p) {
@@ -221,6 +257,8 @@ cr_status cr_context_create(int device, cr_context **out) {
     c->cus = prop.multiProcessorCount;
     c->clock_mhz = prop.clockRate / 1000;
     c->hbm = prop.totalGlobalMem;
+    if (hipDeviceGetAttribute(&c->wall_khz, hipDeviceAttributeWallClockRate, device) != hipSuccess || c->wall_khz <= 0)
+        c->wall_khz = 100000;  // gfx950's constant clock
     snprintf(c->name, sizeof(c->name), "%s", prop.name);
     snprintf(c->arch, sizeof(c->arch), "%s", prop.gcnArchName);
     hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
@@ -241,6 +279,7 @@ cr_status cr_context_destroy(cr_context *ctx) {
     ctx->jobs.release();
     ctx->counters.release();
     ctx->hist.release();
+    ctx->direct.release();
     ctx->table_a.release();
     ctx->table_b.release();
     ctx->host.release();
@@ -346,16 +385,19 @@ cr_status cr_an_pairs_tuned(cr_context *ctx, uint64_t A, uint64_t num_words, uin
 cr_status cr_an_pairs(cr_context *ctx, uint64_t A, uint64_t num_words, uint64_t *raw, uint32_t nbins,
                       double *kernel_ms) {
     // the same histogram by whichever method is estimated to be the fastest:
-    // the pair kernel (measured 40 us a call and about 7e12 pairs/s where it
-    // competes, up to 2^13 words), the sliced kernel (45 us a call and the
-    // rates of sliced_rate), the code's spectrum, the recursions over carries
+    // the short kernel (measured 18 us a call of 2^8 words, 29 us of 2^13), the
+    // pair kernel (40 us a call and about 7e12 pairs/s where it competes), the
+    // sliced kernel (49 us at 2^14 words, then the rates of sliced_rate), the
+    // code's spectrum, the recursions over carries
     uint32_t k = 0;
     const double pairs = 0.5 * (double)num_words * (double)num_words;
-    double best = 40e-6 + pairs / 7e12;
+    const bool is_short = A != 0 && num_words != 0 && num_words <= kShortWords &&
+                          !((unsigned __int128)(num_words - 1) * A >> 64);
+    double best = is_short ? 20e-6 + pairs / 3.5e12 : 40e-6 + pairs / 7e12;
     SlicedJob sliced;
     bool by_planes = false;
     if (sliced_job(A, num_words, &sliced)) {
-        const double s = 45e-6 + pairs / sliced_rate(sliced);
+        const double s = 38e-6 + pairs / sliced_rate(sliced);
         by_planes = s < best;
         best = std::min(best, s);
     }
@@ -367,22 +409,11 @@ cr_status cr_an_pairs(cr_context *ctx, uint64_t A, uint64_t num_words, uint64_t 
     const bool recursion = carry_preferred(A, num_words, best, &carry);
     if (recursion) best = carry.seconds;
     CarryTilesPlan tiles;
-    if (tiles_preferred(A, num_words, best, &tiles))
-        return an_pairs_carry(
-            ctx, A, tiles.k, tiles.nbins, tiles.hist_entries, tiles.table_bytes, 0,
-            [&](unsigned long long *hist) {
-                return carry_tiles_run(tiles, ctx->table_a.ptr, hist, ctx->cus, ctx->stream);
-            },
-            raw, nbins, kernel_ms);
-    if (recursion)
-        return an_pairs_carry(
-            ctx, A, carry.k, carry.nbins, carry.hist_entries, carry.table_bytes, carry.table_bytes,
-            [&](unsigned long long *hist) {
-                return carry_run(carry, ctx->table_a.ptr, ctx->table_b.ptr, hist, ctx->cus, ctx->stream);
-            },
-            raw, nbins, kernel_ms);
+    if (tiles_preferred(A, num_words, best, &tiles)) return an_pairs_tiles(ctx, tiles, A, raw, nbins, kernel_ms);
+    if (recursion) return an_pairs_carry(ctx, carry, A, raw, nbins, kernel_ms);
     if (spectral && spectral_s < pairwise) return cr_an_pairs_spectral(ctx, A, k, raw, nbins, kernel_ms);
     if (by_planes) return an_pairs_sliced(ctx, sliced, A, num_words, raw, nbins, kernel_ms);
+    if (is_short) return an_pairs_short(ctx, A, num_words, raw, nbins, kernel_ms);
     return cr_an_pairs_tuned(ctx, A, num_words, raw, nbins, nullptr, kernel_ms);
 }
 

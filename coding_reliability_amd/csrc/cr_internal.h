@@ -132,6 +132,18 @@ cr_status launch_pairs(const PairJob *d_jobs, uint32_t njobs, uint64_t total_ite
 // lane and `lds_rows` histogram rows.
 uint32_t pair_waves_per_cu(uint32_t R, uint32_t lds_rows);
 
+// Pair histogram of a short code in one launch (see short_pairs.hip).
+constexpr uint32_t kShortWords = 1u << 13;
+namespace dev {
+struct DirectResult;
+}
+cr_status launch_short_pairs(uint64_t A, uint32_t N, uint32_t nbins, const dev::DirectResult &out, int cus,
+                             hipStream_t stream);
+// Buffers of a one-launch call on a context, and its end: waits, raw[0, need)
+// from pinned memory, zeros above, the device time.
+cr_status direct_result(cr_context *ctx, dev::DirectResult *r);
+cr_status direct_wait(cr_context *ctx, uint64_t *raw, uint32_t need, uint32_t nbins, double *kernel_ms);
+
 // Pair histograms of whole codes by bit planes (see sliced_pairs.hip).
 struct SlicedJob {
     uint64_t item_begin, items;  // global range of the job's items in the launch
@@ -153,6 +165,10 @@ void sliced_ranges(std::vector<SlicedJob> &jobs, int cus, uint64_t *total_items)
 // assignment of items to workgroups.
 cr_status launch_sliced(const SlicedJob *d_jobs, uint32_t njobs, uint64_t total_items, unsigned long long *counter,
                         int cus, hipStream_t stream);
+
+// One job (its item range set) whose histogram goes to `out` (out_copies: dev::kHistCopies).
+cr_status launch_sliced_direct(const SlicedJob &job, uint64_t items, const dev::DirectResult &out, int cus,
+                               hipStream_t stream);
 
 // Rectangle histogram rows x column table (see rect_pairs.hip).
 struct RectLaunch {
@@ -180,9 +196,9 @@ struct CarryRowsPlan {
 // False when the recursion does not apply or the rectangle kernel is estimated
 // to be faster; nbins: distances of the words and samples.
 bool carry_rows_plan(uint64_t A, uint32_t n, uint64_t ncols, uint32_t nbins, CarryRowsPlan *p);
-// Adds the histogram of all samples to dev::kHistCopies copies of nbins at out.
+// Leaves the histogram of all samples, nbins counts, in out.host.
 cr_status launch_carry_rows(const CarryRowsPlan &p, const uint64_t *cols, uint32_t ncols, uint32_t nbins,
-                            unsigned long long *out, int cus, hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1);
+                            const dev::DirectResult &out, int cus, hipStream_t stream);
 
 // Hamming weight jobs (see hamming.hip).
 enum HamSource : uint32_t { kHamRange = 0, kHamStride = 1, kHamList = 2, kHamMc = 3 };
@@ -242,18 +258,18 @@ struct CarryPlan {
     uint32_t states = 0;        // carry pairs, A^2
     uint32_t nbins = 0;         // distances 0 .. k + hb
     uint64_t table_bytes = 0;   // of each of the two tables
-    uint64_t hist_entries = 0;  // dev::kHistCopies copies of nbins
     double seconds = 0;         // estimated time of a call
 };
 // False when (A, 2^k words) is outside the recursion.
 bool carry_plan(uint64_t A, uint32_t k, CarryPlan *p);
-// Leaves the distribution over ordered pairs in hist (p.hist_entries, cleared here).
-cr_status carry_run(const CarryPlan &p, void *table0, void *table1, unsigned long long *hist, int cus,
+// Leaves the distribution over ordered pairs, p.nbins counts, in out.host.
+cr_status carry_run(const CarryPlan &p, void *table0, void *table1, const dev::DirectResult &out, int cus,
                     hipStream_t stream);
-// raw[] (nbins entries, pair-kernel form) from the host copy of an ordered-pair
-// histogram of 2^k words (dev::kHistCopies copies of `bins`); checks the words
-// at distance 0 and the total of 4^k.
-cr_status carry_finish(uint32_t k, uint32_t bins, const uint64_t *hist, uint64_t *raw, uint32_t nbins);
+// raw[] (nbins entries, pair-kernel form) from an ordered-pair histogram of 2^k
+// words (`copies` copies of `bins`, dev::hist_copy_stride apart); checks the
+// words at distance 0 and the total of 4^k.
+cr_status carry_finish(uint32_t k, uint32_t bins, const uint64_t *hist, uint32_t copies, uint64_t *raw,
+                       uint32_t nbins);
 
 // The same recursion for long multipliers, by tiles of carry pairs with four
 // levels a kernel (see carry_tiles.hip).
@@ -308,12 +324,14 @@ struct cr_context {
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     int cus = 0;
     int clock_mhz = 0;
+    int wall_khz = 0;          // rate of the device's constant clock
     uint64_t hbm = 0;
     char name[64] = {0};
     char arch[32] = {0};
     cr::DeviceBuffer jobs;     // PairJob array
     cr::DeviceBuffer counters; // work-queue heads
     cr::DeviceBuffer hist;     // histograms
+    cr::DeviceBuffer direct;   // histogram copies, queue head and ticket of one-launch calls, zero between them
     cr::DeviceBuffer table_a;  // row / sample tables
     cr::DeviceBuffer table_b;
     cr::HostBuffer host;       // pinned staging

@@ -137,12 +137,22 @@ extern "C" cr_status cr_an_grid_ref(cr_context *ctx, int gdim, uint32_t n, uint6
     }
     // all 2^n words of a short multiplier: their carries instead of the words
     CarryRowsPlan rp;
-    const bool recursion = gdim == 1 && carry_rows_plan(g.A, n, cols.size(), need, &rp);
-    const uint64_t copies = recursion ? dev::kHistCopies : 1;
-    const uint64_t cstride = dev::hist_copy_stride(need), entries = copies * cstride;
-    CR_TRY(ctx->hist.reserve(entries * sizeof(uint64_t)));
+    if (gdim == 1 && carry_rows_plan(g.A, n, cols.size(), need, &rp)) {
+        dev::DirectResult out;
+        CR_TRY(direct_result(ctx, &out));
+        CR_TRY(launch_carry_rows(rp, ctx->table_a.as<uint64_t>(), (uint32_t)cols.size(), need, out, ctx->cus,
+                                 ctx->stream));
+        CR_TRY(direct_wait(ctx, hist, need, nbins, kernel_ms));
+        // every word meets every sample once
+        unsigned __int128 total = 0;
+        for (uint32_t b = 0; b < need; ++b) total += hist[b];
+        if (total != (unsigned __int128)g.msgs * cols.size())
+            return fail(CR_ERR_DEVICE, "grid recursion: inconsistent total");
+        return CR_OK;
+    }
+    CR_TRY(ctx->hist.reserve(need * sizeof(uint64_t)));
     CR_TRY(ctx->counters.reserve(sizeof(uint64_t)));
-    CR_TRY(fill_zero_u64(ctx->hist.as<unsigned long long>(), entries, ctx->stream));
+    CR_TRY(fill_zero_u64(ctx->hist.as<unsigned long long>(), need, ctx->stream));
 
     RectLaunch L;
     L.A = g.A;
@@ -158,25 +168,12 @@ extern "C" cr_status cr_an_grid_ref(cr_context *ctx, int gdim, uint32_t n, uint6
     L.nbins = need;
     L.first_bin = gdim == 2 ? 1 : 0;  // dancoding_grid_2d flushes bins 1.. (an_coding_grid.cu:138)
     L.lds_rows = need + 1;
-    hipEvent_t ev0 = kernel_ms ? ctx->ev0 : nullptr, ev1 = kernel_ms ? ctx->ev1 : nullptr;
-    if (recursion)
-        CR_TRY(launch_carry_rows(rp, L.cols, (uint32_t)L.ncols, need, L.out, ctx->cus, ctx->stream, ev0, ev1));
-    else
-        CR_TRY(launch_rect(L, ctx->stream, ev0, ev1, ctx->cus));
-    CR_TRY(ctx->host.reserve(entries * sizeof(uint64_t)));
-    CR_HIP(hipMemcpyAsync(ctx->host.ptr, L.out, entries * sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
+    CR_TRY(launch_rect(L, ctx->stream, kernel_ms ? ctx->ev0 : nullptr, kernel_ms ? ctx->ev1 : nullptr, ctx->cus));
+    CR_TRY(ctx->host.reserve(need * sizeof(uint64_t)));
+    CR_HIP(hipMemcpyAsync(ctx->host.ptr, L.out, need * sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
     CR_HIP(hipStreamSynchronize(ctx->stream));
     memset(hist, 0, nbins * sizeof(uint64_t));
-    const uint64_t *h = ctx->host.as<uint64_t>();
-    for (uint64_t c = 0; c < copies; ++c)
-        for (uint32_t b = 0; b < need; ++b) hist[b] += h[c * cstride + b];
-    if (recursion) {
-        // every word meets every sample once
-        unsigned __int128 total = 0;
-        for (uint32_t b = 0; b < need; ++b) total += hist[b];
-        if (total != (unsigned __int128)g.msgs * cols.size())
-            return fail(CR_ERR_DEVICE, "grid recursion: inconsistent total");
-    }
+    memcpy(hist, ctx->host.ptr, need * sizeof(uint64_t));
     if (kernel_ms) {
         float ms = 0;
         CR_HIP(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));

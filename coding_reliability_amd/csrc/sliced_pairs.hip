@@ -16,9 +16,9 @@
 // one.  Bound by VALU issue: 19.9e12 pairs/s for 16-bit multipliers at k = 18
 // (9.4e12 in the pair kernel), 42e12 lane instructions/s of the 42e12 that the
 // device issues; 1024 mixed codes of 8 to 18 bits 199 ms (473 ms).  A single
-// code of 2^16 words takes 0.19 ms (0.34 ms), of 2^14 60 us, as in the pair
-// kernel, which keeps the shorter ones: four workgroups per block of 64 x 64
-// words are too few there.
+// code of 2^16 words takes 0.16 ms (0.34 ms), of 2^14 49 us (64 us); below that
+// four workgroups per block of 64 x 64 words are too few, and the short kernel
+// takes over.
 //
 // The first adders work on triples of planes (p1, p2, p3) stored as p1, p1 ^
 // p2, p1 ^ p3, p1 ^ p2 ^ p3, for either side: the sum is one XOR and the
@@ -329,10 +329,14 @@ __device__ void finish_item(Lds &L, uint32_t base, bool twice) {
     __syncthreads();
 }
 
+// jobs: device array, or null for the one job `single`, whose histogram goes
+// to `direct`.
 __global__ __launch_bounds__(kThreads) void sliced_kernel(const SlicedJob *__restrict__ jobs, uint32_t njobs,
                                                           uint64_t total_items,
-                                                          unsigned long long *__restrict__ counter) {
+                                                          unsigned long long *__restrict__ counter,
+                                                          const SlicedJob single, const DirectResult direct) {
     __shared__ Lds L;
+    if (!jobs) direct_start(direct);
     const uint32_t tid = threadIdx.x;
     for (uint32_t i = tid; i < kClasses * kProducts * kCols; i += kThreads) L.count[i] = 0;
     if (tid < kClasses) L.pairs[tid] = 0;
@@ -341,7 +345,7 @@ __global__ __launch_bounds__(kThreads) void sliced_kernel(const SlicedJob *__res
     uint32_t cur = 0xFFFFFFFFu;
     auto flush = [&]() {
         if (cur == 0xFFFFFFFFu) return;
-        const SlicedJob &job = jobs[cur];
+        const SlicedJob &job = jobs ? jobs[cur] : single;
         if (tid < job.nbins && tid < kHist) {
             const unsigned long long n = L.hist[tid];
             if (n) atomicAdd(hist_copy(job.out, job.nbins, job.out_copies) + tid, n);
@@ -350,8 +354,8 @@ __global__ __launch_bounds__(kThreads) void sliced_kernel(const SlicedJob *__res
         __syncthreads();
     };
     for (uint64_t t = blockIdx.x; t < total_items;) {
-        uint32_t jb = cur;
-        if (cur == 0xFFFFFFFFu || t < jobs[cur].item_begin || t >= jobs[cur].item_begin + jobs[cur].items) {
+        uint32_t jb = jobs ? cur : 0;
+        if (jobs && (cur == 0xFFFFFFFFu || t < jobs[cur].item_begin || t >= jobs[cur].item_begin + jobs[cur].items)) {
             uint32_t lo = 0, hi = njobs - 1;
             while (lo < hi) {
                 const uint32_t mid = (lo + hi + 1) >> 1;
@@ -363,7 +367,7 @@ __global__ __launch_bounds__(kThreads) void sliced_kernel(const SlicedJob *__res
             flush();
             cur = jb;
         }
-        const SlicedJob &job = jobs[jb];
+        const SlicedJob &job = jobs ? jobs[jb] : single;
         const uint32_t local = uniform32((uint32_t)(t - job.item_begin));
         const uint32_t part = local % job.parts, pair = local / job.parts;
         // pair = col (col + 1) / 2 + row, row <= col
@@ -387,6 +391,7 @@ __global__ __launch_bounds__(kThreads) void sliced_kernel(const SlicedJob *__res
         __syncthreads();
     }
     flush();
+    if (!jobs) direct_finish(direct, single.nbins, L.sum);
 }
 
 }  // namespace
@@ -459,7 +464,19 @@ cr_status launch_sliced(const SlicedJob *d_jobs, uint32_t njobs, uint64_t total_
     const uint32_t per_cu = sliced_per_cu();
     if (per_cu == 0) return fail(CR_ERR_DEVICE, "occupancy query failed for the sliced pair kernel");
     const uint32_t blocks = (uint32_t)std::min<uint64_t>(total_items, (uint64_t)per_cu * (uint32_t)cus);
-    hipLaunchKernelGGL(sliced_kernel, dim3(blocks), dim3(kThreads), 0, stream, d_jobs, njobs, total_items, counter);
+    hipLaunchKernelGGL(sliced_kernel, dim3(blocks), dim3(kThreads), 0, stream, d_jobs, njobs, total_items, counter,
+                       SlicedJob{}, DirectResult{});
+    CR_HIP(hipGetLastError());
+    return CR_OK;
+}
+
+cr_status launch_sliced_direct(const SlicedJob &job, uint64_t items, const dev::DirectResult &out, int cus,
+                               hipStream_t stream) {
+    const uint32_t per_cu = sliced_per_cu();
+    if (per_cu == 0) return fail(CR_ERR_DEVICE, "occupancy query failed for the sliced pair kernel");
+    const uint32_t blocks = (uint32_t)std::min<uint64_t>(items, (uint64_t)per_cu * (uint32_t)cus);
+    hipLaunchKernelGGL(sliced_kernel, dim3(blocks), dim3(kThreads), 0, stream, (const SlicedJob *)nullptr, 1u, items,
+                       out.queue, job, out);
     CR_HIP(hipGetLastError());
     return CR_OK;
 }
