@@ -7,6 +7,7 @@ exported by the same library; see include/cr_reference_api.h.
 from __future__ import annotations
 
 import ctypes as C
+import itertools
 
 import numpy as np
 
@@ -61,6 +62,15 @@ def hamming_sdc_table(k: int, method: int = 2, ctx: "Context | None" = None) -> 
 
 def _u64p(a):
     return a.ctypes.data_as(C.POINTER(C.c_uint64))
+
+
+def _rows(out, bins) -> list[list[int]]:
+    """Rows of a 2-D count array as lists of Python integers, row i cut to bins[i]."""
+    rows = out.tolist()
+    for row, n in zip(rows, bins):
+        if n != len(row):
+            del row[n:]
+    return rows
 
 
 def _u128(buf) -> list[int]:
@@ -148,54 +158,56 @@ class Context:
         pair-kernel time in ms."""
         if nbins is None:
             nbins = an_bins(A, num_words)
-        out = np.zeros(nbins, dtype=np.uint64)
+        out = (C.c_uint64 * nbins)()
         ms = C.c_double(0)
         t = cr_pair_tuning(rows_per_lane, chunk_blocks, waves, 0)
-        check(lib().cr_an_pairs_tuned(self._h, A, num_words, _u64p(out), nbins, C.byref(t), C.byref(ms)))
-        return [int(x) for x in out], ms.value
+        check(lib().cr_an_pairs_tuned(self._h, A, num_words, out, nbins, C.byref(t), C.byref(ms)))
+        return list(out), ms.value
 
     def an_pairs_auto(self, A: int, num_words: int, nbins: int | None = None) -> tuple[list[int], float]:
         """The same histogram as an_pairs through cr_an_pairs, which picks the
         spectral path for 2^16 / 2^24 words when it is estimated cheaper."""
         if nbins is None:
             nbins = an_bins(A, num_words)
-        out = np.zeros(nbins, dtype=np.uint64)
+        out = (C.c_uint64 * nbins)()
         ms = C.c_double(0)
-        check(lib().cr_an_pairs(self._h, A, num_words, _u64p(out), nbins, C.byref(ms)))
-        return [int(x) for x in out], ms.value
+        check(lib().cr_an_pairs(self._h, A, num_words, out, nbins, C.byref(ms)))
+        return list(out), ms.value
 
     def an_pairs_spectral(self, A: int, k: int, nbins: int | None = None) -> tuple[list[int], float]:
         """Same raw histogram as an_pairs(A, 2^k), from the Walsh-Hadamard
         spectrum of the code (cr_an_pairs_spectral), and the device time in ms."""
         if nbins is None:
             nbins = an_bins(A, 1 << k)
-        out = np.zeros(nbins, dtype=np.uint64)
+        out = (C.c_uint64 * nbins)()
         ms = C.c_double(0)
-        check(lib().cr_an_pairs_spectral(self._h, A, k, _u64p(out), nbins, C.byref(ms)))
-        return [int(x) for x in out], ms.value
+        check(lib().cr_an_pairs_spectral(self._h, A, k, out, nbins, C.byref(ms)))
+        return list(out), ms.value
 
     # --- batched exhaustive AN -------------------------------------------------
     @staticmethod
     def _codes(codes):
-        arr = (cr_an_code * len(codes))()
-        for i, (A, N) in enumerate(codes):
-            arr[i].A, arr[i].num_words = A, N
-        return arr
+        # (A, num_words) as 64-bit pairs: the layout of cr_an_code
+        try:
+            arr = np.fromiter(itertools.chain.from_iterable(codes), dtype=np.uint64, count=2 * len(codes))
+        except OverflowError:  # taken modulo 2^64, as ctypes takes an argument
+            arr = np.array([x & 0xFFFFFFFFFFFFFFFF for c in codes for x in c], dtype=np.uint64)
+        return arr.ctypes.data_as(C.POINTER(cr_an_code))
 
     @staticmethod
-    def _stride(codes):
-        return max(an_bins(A, N) for A, N in codes)
+    def _bins(codes):
+        return [((N - 1) * A).bit_length() + 1 for A, N in codes]
 
     def an_batch(self, codes, rows_per_lane: int = 0, items_per_wave: int = 0) -> tuple[list[list[int]], float]:
         """Raw histograms of many (A, num_words) codes in one launch."""
-        stride = self._stride(codes)
-        out = np.zeros(len(codes) * stride, dtype=np.uint64)
+        bins = self._bins(codes)
+        stride = max(bins)
+        out = np.empty((len(codes), stride), dtype=np.uint64)
         ms = C.c_double(0)
         t = cr_pair_tuning(rows_per_lane, 0, 0, items_per_wave)
         check(lib().cr_an_batch(self._h, self._codes(codes), len(codes), _u64p(out), stride, C.byref(t),
                                 C.byref(ms)))
-        o = out.reshape(len(codes), stride)
-        return [[int(x) for x in row[: an_bins(A, N)]] for row, (A, N) in zip(o, codes)], ms.value
+        return _rows(out, bins), ms.value
 
     def batch_plan(self, codes, rows_per_lane: int = 0, items_per_wave: int = 0) -> "BatchPlan":
         return BatchPlan(self, codes, rows_per_lane, items_per_wave)
@@ -262,10 +274,10 @@ class Context:
         req = cr_ham_request(k, source, first, count, stride, _u64p(lst) if lst is not None else None, seed,
                              stream, 0)
         nbins = hamming_N(k)
-        out = np.zeros(nbins, dtype=np.uint64)
+        out = (C.c_uint64 * nbins)()
         ms = C.c_double(0)
-        check(lib().cr_hamming_weights(self._h, C.byref(req), _u64p(out), nbins, C.byref(ms)))
-        return [int(x) for x in out], ms.value
+        check(lib().cr_hamming_weights(self._h, C.byref(req), out, nbins, C.byref(ms)))
+        return list(out), ms.value
 
     def hamming_weights_batch(self, requests) -> tuple[list[list[int]], float]:
         """hamming_weights of several requests in one call
@@ -289,14 +301,14 @@ class Context:
         out = np.zeros((len(requests), nbins), dtype=np.uint64)
         ms = C.c_double(0)
         check(lib().cr_hamming_weights_batch(self._h, reqs, len(requests), _u64p(out), nbins, C.byref(ms)))
-        return [[int(x) for x in row[: hamming_N(q["k"])]] for row, q in zip(out, requests)], ms.value
+        return _rows(out, [hamming_N(q["k"]) for q in requests]), ms.value
 
     def an_mc(self, A: int, n: int, m: int, seed: int, nbins: int = 65) -> tuple[list[int], float]:
         """Monte Carlo (word, sample) histogram of run_ancoding_mc with Philox samples."""
-        out = np.zeros(nbins, dtype=np.uint64)
+        out = (C.c_uint64 * nbins)()
         ms = C.c_double(0)
-        check(lib().cr_an_mc(self._h, A, n, m, seed, _u64p(out), nbins, C.byref(ms)))
-        return [int(x) for x in out], ms.value
+        check(lib().cr_an_mc(self._h, A, n, m, seed, out, nbins, C.byref(ms)))
+        return list(out), ms.value
 
     def an_mc_ranges(self, A: int, n: int, bounds, seed: int, nbins: int = 65) -> tuple[list[list[int]], float]:
         """Histograms of the sample ranges [bounds[i], bounds[i+1]) of an_mc
@@ -306,7 +318,7 @@ class Context:
         out = np.zeros((max(count, 0), nbins), dtype=np.uint64)
         ms = C.c_double(0)
         check(lib().cr_an_mc_ranges(self._h, A, n, _u64p(b), count, seed, _u64p(out), nbins, C.byref(ms)))
-        return [[int(x) for x in row] for row in out], ms.value
+        return out.tolist(), ms.value
 
     def an_mc_prefixes(self, A: int, n: int, ms_list, seed: int, nbins: int = 65) -> tuple[list[list[int]], float]:
         """an_mc histograms for each sample count in ms_list (non-decreasing),
@@ -321,10 +333,10 @@ class Context:
     def an_grid_ref(self, gdim: int, n: int, m1: int, m2: int, A: int, nbins: int = 65) -> tuple[list[int], float]:
         """Kernel-level histogram of the reference grid approximation
         (run_ancoding_grid) and the kernel time in ms."""
-        out = np.zeros(nbins, dtype=np.uint64)
+        out = (C.c_uint64 * nbins)()
         ms = C.c_double(0)
-        check(lib().cr_an_grid_ref(self._h, gdim, n, m1, m2, A, _u64p(out), nbins, C.byref(ms)))
-        return [int(x) for x in out], ms.value
+        check(lib().cr_an_grid_ref(self._h, gdim, n, m1, m2, A, out, nbins, C.byref(ms)))
+        return list(out), ms.value
 
 
 class BatchPlan:
@@ -332,20 +344,20 @@ class BatchPlan:
 
     def __init__(self, ctx: Context, codes, rows_per_lane: int = 0, items_per_wave: int = 0):
         self.codes = list(codes)
-        self.stride = Context._stride(self.codes)
+        self.bins = Context._bins(self.codes)
+        self.stride = max(self.bins)
         self._h = C.c_void_p()
         t = cr_pair_tuning(rows_per_lane, 0, 0, items_per_wave)
         check(lib().cr_batch_plan_create(ctx.handle, Context._codes(self.codes), len(self.codes), self.stride,
                                          C.byref(t), C.byref(self._h)))
-        self._out = np.zeros(len(self.codes) * self.stride, dtype=np.uint64)
+        self._out = np.zeros((len(self.codes), self.stride), dtype=np.uint64)
 
     def run(self, fetch: bool = True):
         ms = C.c_double(0)
         check(lib().cr_batch_plan_run(self._h, _u64p(self._out) if fetch else None, C.byref(ms)))
         if not fetch:
             return None, ms.value
-        o = self._out.reshape(len(self.codes), self.stride)
-        return [[int(x) for x in row[: an_bins(A, N)]] for row, (A, N) in zip(o, self.codes)], ms.value
+        return _rows(self._out, self.bins), ms.value
 
     def close(self):
         if self._h:
