@@ -91,8 +91,8 @@ cr_status direct_result(cr_context *ctx, dev::DirectResult *r) {
     }
     CR_TRY(ctx->host.reserve((dev::kDirectBins + 2) * sizeof(uint64_t)));
     r->copies = ctx->direct.as<unsigned long long>();
-    r->queue = r->copies + dev::kDirectEntries - 2;
-    r->ticket = reinterpret_cast<unsigned int *>(r->queue + 1);
+    r->queue = r->copies + (size_t)dev::kHistCopies * dev::kDirectBins;
+    r->tickets = reinterpret_cast<unsigned int *>(r->queue + 16);
     r->host = ctx->host.as<unsigned long long>();
     return CR_OK;
 }

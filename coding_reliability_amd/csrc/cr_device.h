@@ -66,16 +66,19 @@ __device__ __forceinline__ unsigned long long *hist_copy(unsigned long long *out
 
 // A call of one launch: the workgroups add to the histogram copies, the last
 // one to finish sums them into pinned host memory.  The copies, the queue head
-// and the ticket are zero between launches: the last workgroup leaves them so,
+// and the tickets are zero between launches: the last workgroup leaves them so,
 // so a call needs no fill before and no copy after its kernel.
 struct DirectResult {
     unsigned long long *copies = nullptr;  // kHistCopies copies, hist_copy_stride(nbins) apart
     unsigned long long *queue = nullptr;   // work-queue head
-    unsigned int *ticket = nullptr;        // workgroups that are done
+    unsigned int *tickets = nullptr;       // workgroups that are done, by groups of them, then the groups
     unsigned long long *host = nullptr;    // nbins results; from kDirectBins: device clock at the start, at the end
 };
 constexpr uint32_t kDirectBins = 80;  // largest copy stride
-constexpr size_t kDirectEntries = (size_t)kHistCopies * kDirectBins + 2;
+// Device-scope atomics on one address serialize at about 12.5 ns, so the
+// workgroups count themselves in groups, each on a cache line of its own.
+constexpr uint32_t kTicketGroups = 64, kTicketPitch = 32;  // 32-bit tickets between two groups
+constexpr size_t kDirectEntries = (size_t)kHistCopies * kDirectBins + 16 + (kTicketGroups + 1) * kTicketPitch / 2;
 
 // The call's device time by the device's constant-rate clock: events around
 // the launch cost 9 to 18 us of a 15 us call.
@@ -91,8 +94,15 @@ __device__ __forceinline__ void direct_start(const DirectResult &r) {
 __device__ inline void direct_finish(const DirectResult &r, uint32_t nbins, uint32_t *flag) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (threadIdx.x == 0)
-        *flag = __hip_atomic_fetch_add(r.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+    if (threadIdx.x == 0) {
+        const uint32_t g = blockIdx.x % kTicketGroups, groups = gridDim.x < kTicketGroups ? gridDim.x : kTicketGroups;
+        const uint32_t members = (gridDim.x - g + kTicketGroups - 1) / kTicketGroups;
+        bool last = __hip_atomic_fetch_add(r.tickets + (g + 1) * kTicketPitch, 1u, __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT) == members - 1;
+        if (last)
+            last = __hip_atomic_fetch_add(r.tickets, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == groups - 1;
+        *flag = last;
+    }
     __syncthreads();
     if (!*flag) return;
     // thread (b, c): copy c of distance b; eight exchanges in flight a thread
@@ -114,9 +124,10 @@ __device__ inline void direct_finish(const DirectResult &r, uint32_t nbins, uint
             if (c == 0 && b0 + u * step < nbins) r.host[b0 + u * step] = s[u];
         }
     }
+    for (uint32_t g = threadIdx.x; g <= kTicketGroups; g += blockDim.x)
+        __hip_atomic_store(r.tickets + g * kTicketPitch, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (threadIdx.x == 0) {
         __hip_atomic_store(r.queue, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(r.ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         r.host[kDirectBins + 1] = (unsigned long long)wall_clock64();
     }
 }

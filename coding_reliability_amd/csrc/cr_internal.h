@@ -201,9 +201,9 @@ cr_status launch_carry_rows(const CarryRowsPlan &p, const uint64_t *cols, uint32
                             const dev::DirectResult &out, int cus, hipStream_t stream);
 
 // Hamming weight jobs (see hamming.hip).
-enum HamSource : uint32_t { kHamRange = 0, kHamStride = 1, kHamList = 2, kHamMc = 3 };
+enum HamSource : uint32_t { kHamStride = 1, kHamList = 2, kHamMc = 3 };
 struct HamJob {
-    uint64_t first;            // range/stride offset, or first Monte Carlo sample index
+    uint64_t first;            // stride offset, or first Monte Carlo sample index
     uint64_t stride;
     uint64_t count;            // samples
     const uint64_t *list;      // device list (kHamList)
@@ -285,6 +285,24 @@ bool carry_tiles_plan(uint64_t A, uint32_t k, CarryTilesPlan *p);
 cr_status carry_tiles_run(const CarryTilesPlan &p, void *table, unsigned long long *hist, int cus,
                           hipStream_t stream);
 
+// Weight histogram of consecutive data words by aligned blocks (see
+// hamming_range.hip).
+struct HamRange {
+    struct Block {  // the words d0 | x, x < 2^m, counted `weight` times
+        uint64_t weight;
+        uint16_t m, ones, parity, reserved;  // ones: popcount(d0); parity: parity bits of d0
+    };
+    unsigned long long *out;  // device histogram, nbins entries (written, not added to)
+    uint32_t r, nbins, nblocks, reserved;
+    uint32_t cols[64];        // parity bits of 2^m
+    Block blocks[136];        // in order of m: at most two of each size and one for whole turns
+};
+// The blocks of [first, first + count) modulo 2^k.
+void ham_range_job(uint64_t first, uint64_t count, uint32_t k, const uint64_t masks[7], HamRange *job);
+// The jobs of a device array, or (single) one whose histogram goes to out.host.
+cr_status launch_ham_ranges(const HamRange *d_jobs, uint32_t njobs, const HamRange *single,
+                            const dev::DirectResult &out, hipStream_t stream);
+
 // Parity masks of the (N,k) extended Hamming codes, truncated to k bits;
 // returns the number of non-overall parity bits.
 uint32_t hamming_masks(uint32_t k, uint64_t masks[7]);
@@ -298,6 +316,9 @@ uint32_t hamming_waves_per_cu(uint32_t lds_rows);
 cr_status launch_hamming(const HamJob *d_jobs, uint32_t njobs, uint64_t total_items, bool w64,
                          unsigned long long *counter, bool allow_static, uint32_t lds_rows, int cus,
                          hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1);
+// One job whose histogram goes to `out` (out_copies: dev::kHistCopies).
+cr_status launch_hamming_direct(const HamJob &job, bool w64, bool allow_static, uint32_t lds_rows,
+                                const dev::DirectResult &out, int cus, hipStream_t stream);
 // A sample range of an AN Monte Carlo launch and its histogram: the pairs
 // (word i, sample j) for every word i and j0 <= j < j1 (j0 < j1).
 struct McSegment {
@@ -309,9 +330,11 @@ struct McSegment {
 constexpr uint32_t kMcMaxRanges = 64;  // sample ranges per AN Monte Carlo launch
 // segs (host, nsegs entries, kept alive until the stream is synchronized) is
 // completed and copied to d_segs; counter is the work-queue head (zeroed here).
+// direct (one segment): its histogram goes there, nothing is copied or zeroed,
+// and d_segs, counter and the events are not used.
 cr_status launch_an_mc(uint64_t A, uint32_t n, uint64_t seed, McSegment *segs, uint32_t nsegs, McSegment *d_segs,
                        unsigned long long *counter, uint32_t nbins, int cus, hipStream_t stream, hipEvent_t ev0,
-                       hipEvent_t ev1);
+                       hipEvent_t ev1, const dev::DirectResult *direct);
 
 // Zero-fills n 64-bit words on stream (a kernel, so it may be captured in graphs).
 cr_status fill_zero_u64(unsigned long long *p, size_t n, hipStream_t stream);
@@ -331,7 +354,7 @@ struct cr_context {
     cr::DeviceBuffer jobs;     // PairJob array
     cr::DeviceBuffer counters; // work-queue heads
     cr::DeviceBuffer hist;     // histograms
-    cr::DeviceBuffer direct;   // histogram copies, queue head and ticket of one-launch calls, zero between them
+    cr::DeviceBuffer direct;   // histogram copies, queue head and tickets of one-launch calls, zero between them
     cr::DeviceBuffer table_a;  // row / sample tables
     cr::DeviceBuffer table_b;
     cr::HostBuffer host;       // pinned staging

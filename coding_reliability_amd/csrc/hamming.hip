@@ -5,13 +5,15 @@
 // distance_distribution/src/hamming.cu:183-208), so the kernel histograms the
 // weight of the non-extended codeword, popcount(d) + sum_t parity(d & mask_t)
 // (computeHamming<N>, hamming.cu:39-59), over a stream of data words d:
-//   range   d = first + s                       (exhaustive: dhamming, hamming.cu:64-81)
 //   stride  d = (first + s*stride) mod 2^k      (integer grid)
 //   list    d = list[s]                         (the reference grid's sample points)
 //   mc      d = Philox word s of (seed, stream) (replaces dhamming_mc's cuRAND draw)
+// (Ranges of consecutive words, dhamming's exhaustive mode, hamming.cu:64-81, need
+// no enumeration: hamming_range.hip.)
 // AN Monte Carlo: every word A*i against m Philox samples A*u_ij
 // (replaces dancoding_mc_shared, an_coding_mc.cu:94-158).
 #include <algorithm>
+#include <atomic>
 #include <type_traits>
 
 #include "cr_device.h"
@@ -24,24 +26,22 @@ using namespace dev;
 
 // Work item = 64 lanes x job.lane_samples samples.  Items of up to 2^18 words
 // keep the work-queue counter (one device-scope atomic per item) below its
-// throughput limit (about 8e7 items/s, reached with 4096-word items at 3.4e11
-// words/s and with 32768-word items at 2.5e12 words/s on the exhaustive fast
-// path); small jobs use smaller items so that they still fill the device.
+// throughput limit (about 8e7 items/s); small jobs use smaller items so that
+// they still fill the device.
 
 // Syndrome tables: the syndrome (bit t = parity(d & m_t)) is linear over
-// GF(2), so it is the XOR of the syndromes of the data word's bit fields.
-// Each 32-bit half of the word is cut into fields of 7, 7, 7, 7 and 4 bits;
-// table f (f = 5h + i for field i of half h) holds the syndromes of the
-// field's 2^7 (or 2^4) values, one byte each, at byte offset 128 f: 5 tables
-// for 32-bit data, 10 for 64-bit.  A 128-byte table spans 32 consecutive
-// dwords, one in each LDS bank, so two lanes of a lookup only meet in a bank
-// on the same dword, whose read they share: the lookups are free of bank
-// conflicts (a 256-entry byte table puts two dwords in every bank).  The masks
-// are truncated to k bits, so bits of d above k do not change the syndrome.
-constexpr uint32_t kFields = 5;  // fields per 32-bit half
+// GF(2), so it is the XOR of the syndromes of the data word's bytes; table f
+// holds the syndromes of byte f's 256 values, one byte each: 4 tables for 32-bit
+// data, 8 for 64-bit.  A 256-byte table has two dwords in every LDS bank, so
+// some lookups take two passes, where five 7-bit fields a half word would
+// not; but the kernel is bound by VALU issue, and four lookups take one
+// extraction less (LDS stays at about 0.65 of its rate).  Measured with the XORs
+// three operands at a time: (39,32) Monte Carlo of 2^34 words 10.6 -> 9.0 ms,
+// (72,64) of 2^30 1.40 -> 1.31 ms, a (39,32) stride grid of 2^30 0.50 -> 0.43 ms.
+constexpr uint32_t kFields = 4;  // bytes per 32-bit half
 
 template <bool W64>
-constexpr uint32_t kTabBytes = (W64 ? 2 : 1) * kFields * 128;
+constexpr uint32_t kTabBytes = (W64 ? 2 : 1) * kFields * 256;
 
 template <bool W64>
 __device__ void build_tables(uint8_t *tab, const uint64_t *masks) {
@@ -49,13 +49,10 @@ __device__ void build_tables(uint8_t *tab, const uint64_t *masks) {
 #pragma unroll
     for (int t = 0; t < 7; ++t) m[t] = masks[t];
     for (uint32_t e = threadIdx.x; e < kTabBytes<W64>; e += 64) {
-        const uint32_t f = e >> 7, v = e & 127, h = f / kFields, i = f % kFields;
+        const uint64_t x = (uint64_t)(e & 255) << (8 * (e >> 8));
         uint32_t syn = 0;
-        if (i < kFields - 1 || v < 16) {
-            const uint64_t x = (uint64_t)v << (32 * h + 7 * i);
 #pragma unroll
-            for (int t = 0; t < 7; ++t) syn |= (uint32_t)(__popcll(x & m[t]) & 1) << t;
-        }
+        for (int t = 0; t < 7; ++t) syn |= (uint32_t)(__popcll(x & m[t]) & 1) << t;
         tab[e] = (uint8_t)syn;
     }
     __syncthreads();
@@ -71,14 +68,9 @@ __device__ __forceinline__ void table_reads(const uint64_t (&d)[U], const uint8_
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
-        for (uint32_t h = 0; h < (W64 ? 2u : 1u); ++h) {
-            const uint32_t x = (uint32_t)(d[u] >> (32 * h));
-            const uint8_t *t = tab + 128 * kFields * h;
-            r[u][kFields * h + 0] = t[x & 127];
-            r[u][kFields * h + 1] = t[128 + ((x >> 7) & 127)];
-            r[u][kFields * h + 2] = t[256 + ((x >> 14) & 127)];
-            r[u][kFields * h + 3] = t[384 + ((x >> 21) & 127)];
-            r[u][kFields * h + 4] = t[512 + (x >> 28)];
+        for (uint32_t f = 0; f < (W64 ? 2 : 1) * kFields; ++f) {
+            const uint32_t x = (uint32_t)(d[u] >> (32 * (f / kFields)));
+            r[u][f] = tab[256 * f + ((x >> (8 * (f % kFields))) & 255)];
         }
 }
 
@@ -88,9 +80,12 @@ __device__ __forceinline__ void table_weights(const uint64_t (&d)[U], uint64_t d
                                               const uint32_t (&r)[U][(W64 ? 2 : 1) * kFields], uint32_t (&w)[U]) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-        uint32_t syn = r[u][0];
-#pragma unroll
-        for (uint32_t f = 1; f < (W64 ? 2 : 1) * kFields; ++f) syn ^= r[u][f];
+        uint32_t syn = r[u][kFields - 1];
+        if (W64) {
+            syn = __builtin_amdgcn_bitop3_b32(syn, r[u][2 * kFields - 1], r[u][2 * kFields - 2], 0x96);
+            syn = __builtin_amdgcn_bitop3_b32(syn, r[u][kFields], r[u][kFields + 1], 0x96);
+        }
+        syn = __builtin_amdgcn_bitop3_b32(syn, r[u][0], r[u][1], 0x96) ^ r[u][2];
         const uint64_t dm = FULL ? d[u] : d[u] & dmask;
         w[u] = __popc(syn) + (W64 ? (uint32_t)__popcll(dm) : (uint32_t)__popc((uint32_t)dm));
     }
@@ -103,28 +98,6 @@ __device__ __forceinline__ void weights_tab(const uint64_t (&d)[U], uint64_t dma
     table_reads<W64, U>(d, tab, r);
     table_weights<W64, U>(d, dmask, r, w);
 }
-
-// Syndrome of a data word: bit t = parity(x & m_t) (the seventh mask is zero
-// for k <= 32).
-__device__ __forceinline__ uint32_t syndrome32(uint32_t x, const uint64_t (&m)[7]) {
-    uint32_t syn = 0;
-#pragma unroll
-    for (int t = 0; t < 6; ++t) syn |= (__popc(x & (uint32_t)m[t]) & 1u) << t;
-    return syn;
-}
-__device__ __forceinline__ uint32_t syndrome64(uint64_t x, const uint64_t (&m)[7]) {
-    uint32_t syn = 0;
-#pragma unroll
-    for (int t = 0; t < 7; ++t) syn |= (uint32_t)(__popcll(x & m[t]) & 1) << t;
-    return syn;
-}
-
-// Exhaustive fast path: an aligned item holds the words d = dh | 64*q | lane
-// (disjoint bit fields), and both popcount and syndrome split over disjoint
-// fields (the syndrome is linear over GF(2)): weight(d) = popc(dh) + popc(x) +
-// popc(S(dh) ^ S(x)), x = 64*ql | lane, with q = 16*qh + ql.  S(x) and
-// popc(x) are per-lane constants for ql < 16; S(dh), popc(dh) are wave-uniform.
-constexpr uint32_t kFastUnroll = 16;
 
 // One Monte Carlo item: lane l takes the Philox blocks B0 + 64q + l, q <
 // spl/PER, B0 = (first + base)/PER (PER = 4 words per block for k <= 32, 2
@@ -198,14 +171,14 @@ __device__ __forceinline__ void mc_item(uint32_t *lane_col, const uint8_t *tab, 
     }
 }
 
-// Range, stride and list items off the exhaustive fast path.  Lane l takes
-// the words d_q = first + (base + 64q + l) * stride for q < spl (stride 1 for
-// a range), so d advances by 64*stride per step (modulo 2^64, or 2^32 for
-// k <= 32: only the low k bits reach the weight), or list[base + 64q + l].
+// Stride and list items.  Lane l takes the words d_q = first + (base + 64q +
+// l) * stride for q < spl, so d advances by 64*stride per step (modulo 2^64, or
+// 2^32 for k <= 32: only the low k bits reach the weight), or list[base + 64q +
+// l].
 // kSeqUnroll steps per iteration, all table reads (and list loads) of the
 // batch issued before its increments, so the reads overlap instead of each
-// waiting behind the previous increment (8 steps of 5 lookups for 32-bit
-// words, 4 of 10 for 64-bit).  spl is a multiple of kSeqUnroll.
+// waiting behind the previous increment (8 steps of 4 lookups for 32-bit
+// words, 4 of 8 for 64-bit).  spl is a multiple of kSeqUnroll.
 // CHECK: steps past the job's count go to the dummy row.
 template <bool W64>
 constexpr uint32_t kSeqUnroll = W64 ? 4 : 8;
@@ -217,7 +190,7 @@ __device__ __forceinline__ void seq_item(uint32_t *lane_col, const uint8_t *tab,
     const uint32_t lane = threadIdx.x;
     const uint64_t rem = count - base;
     const uint32_t left = rem < 64ull * spl ? (uint32_t)rem : 64u * spl;  // valid samples in the item
-    const uint64_t stride = job.source == kHamRange ? 1 : job.stride;
+    const uint64_t stride = job.stride;
     word_t d = (word_t)(job.first + (base + lane) * stride);
     const word_t step = (word_t)(64 * stride);
     const uint64_t *list = LIST ? job.list + base + lane : nullptr;
@@ -257,34 +230,40 @@ __device__ __forceinline__ uint32_t find_job(const HamJob *jobs, uint32_t njobs,
     return uniform32(lo);
 }
 
-template <bool W64>
+// ONE: the one job `single`, whose histogram goes to `direct`, in place of the
+// device array.
+template <bool W64, bool ONE>
 __global__ __launch_bounds__(64) void ham_kernel(const HamJob *__restrict__ jobs, uint32_t njobs, uint64_t total_items,
-                                                 unsigned long long *__restrict__ counter, uint32_t lds_rows) {
+                                                 unsigned long long *__restrict__ counter, uint32_t lds_rows,
+                                                 const HamJob single, const DirectResult direct) {
     // the tables at a fixed LDS address (their offsets fold into the reads),
     // the histogram rows in the dynamic LDS after them
     __shared__ uint8_t tab[kTabBytes<W64>];
     extern __shared__ uint32_t lds[];
     const uint32_t lane = threadIdx.x;
+    if (ONE) direct_start(direct);
     lds_clear(lds, lds_rows);
     uint32_t *const lane_col = lds + lane;
     const uint32_t dummy = lds_rows - 1;
     uint32_t cur = 0xFFFFFFFFu;
     uint64_t pending = 0;
+    auto flush = [&] {
+        if (cur == 0xFFFFFFFFu) return;
+        const HamJob &job = ONE ? single : jobs[cur];
+        flush_rows(lds, 0, job.nbins, copy_out(job));
+    };
 
     for (uint64_t t = first_item(); t < total_items; t = following_item(counter, t)) {
-        const uint32_t jb = find_job(jobs, njobs, t, cur);
-        const HamJob &job = jobs[jb];
+        const uint32_t jb = ONE ? 0 : find_job(jobs, njobs, t, cur);
+        const HamJob &job = ONE ? single : jobs[jb];
         const uint32_t spl = job.lane_samples;
         if (jb != cur || pending + spl >= 0xFFFFFFFFull) {
-            if (cur != 0xFFFFFFFFu) flush_rows(lds, 0, jobs[cur].nbins, copy_out(jobs[cur]));
+            flush();
             if (jb != cur) build_tables<W64>(tab, job.masks);
             cur = jb;
             pending = 0;
         }
         pending += spl;
-        uint64_t m[7];
-#pragma unroll
-        for (int i = 0; i < 7; ++i) m[i] = job.masks[i];
         const uint64_t dmask = job.k >= 64 ? ~0ull : ((1ull << job.k) - 1);
         const uint64_t base = (t - job.item_begin + job.item_offset) * (64ull * spl);  // first sample of the item
         const uint64_t count = job.count;
@@ -294,40 +273,6 @@ __global__ __launch_bounds__(64) void ham_kernel(const HamJob *__restrict__ jobs
                 mc_item<W64, false>(lane_col, tab, job, base, spl, count, dmask, dummy);
             else
                 mc_item<W64, true>(lane_col, tab, job, base, spl, count, dmask, dummy);
-        } else if (job.source == kHamRange && base + 64ull * spl <= count && spl >= kFastUnroll &&
-                   (spl & (spl - 1)) == 0 && ((job.first + base) & (64ull * spl - 1)) == 0 &&
-                   64ull * spl - 1 <= dmask) {
-            // full item of consecutive words (exhaustive) whose first word is a
-            // multiple of the item size 64*spl, a power of two: the item's
-            // words are d0 | x for x < 64*spl (disjoint bits)
-            // per-lane constants of the item, S(x) from the tables (x < 2^10
-            // spans fields 0 and 1); kept to this path so that they hold no
-            // registers in the others
-            uint32_t fsyn[kFastUnroll], fbase[kFastUnroll];
-#pragma unroll
-            for (uint32_t ql = 0; ql < kFastUnroll; ++ql) {
-                const uint32_t x = (ql << 6) | lane;
-                fsyn[ql] = tab[x & 127] ^ tab[128 + (x >> 7)];
-                fbase[ql] = lane * 4 + ((uint32_t)__popc(x) << 8);  // byte offset in the LDS rows
-            }
-            const uint64_t d0 = (job.first + base) & dmask;
-            for (uint32_t qh = 0; qh < spl / kFastUnroll; ++qh) {
-                uint32_t sh, ph;
-                if (W64) {
-                    const uint64_t dh = uniform64(d0 | ((uint64_t)qh << 10));
-                    sh = uniform32(syndrome64(dh, m));
-                    ph = uniform32((uint32_t)__popcll(dh));
-                } else {
-                    const uint32_t dh = uniform32((uint32_t)d0 | (qh << 10));
-                    sh = uniform32(syndrome32(dh, m));
-                    ph = uniform32(__popc(dh));
-                }
-#pragma unroll
-                for (uint32_t ql = 0; ql < kFastUnroll; ++ql) {
-                    const uint32_t w = __popc(fsyn[ql] ^ sh) + ph;
-                    lds_inc(reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(lds) + ((w << 8) + fbase[ql])));
-                }
-            }
         } else {
             const bool full = base + 64ull * spl <= count;
             if (job.source == kHamList) {
@@ -342,7 +287,8 @@ __global__ __launch_bounds__(64) void ham_kernel(const HamJob *__restrict__ jobs
             }
         }
     }
-    if (cur != 0xFFFFFFFFu) flush_rows(lds, 0, jobs[cur].nbins, copy_out(jobs[cur]));
+    flush();
+    if (ONE) direct_finish(direct, single.nbins, lds);
 }
 
 // AN Monte Carlo: item = (row block of 64*RM words, sample chunk [j0,
@@ -403,12 +349,16 @@ __device__ __forceinline__ void an_mc_item(uint32_t *lane_col, uint64_t A, uint6
 // item holds about 2^18 pairs (one work-queue step per item).  Segments are
 // laid out one after the other, so a wave's items stay in one segment for
 // long runs; its LDS rows go to the segment's histogram when the segment
-// changes.
+// changes.  ONE: the one segment `single`, whose histogram goes to `direct`, in
+// place of the device array.
+template <bool ONE>
 __global__ __launch_bounds__(64) void an_mc_kernel(uint64_t A, uint32_t n, uint64_t seed, uint32_t G,
                                                    const McSegment *__restrict__ segs, uint32_t nsegs,
                                                    uint64_t total_items, unsigned long long *__restrict__ counter,
-                                                   uint32_t nbins, uint32_t lds_rows) {
+                                                   uint32_t nbins, uint32_t lds_rows, const McSegment single,
+                                                   const DirectResult direct) {
     extern __shared__ uint32_t lds[];
+    if (ONE) direct_start(direct);
     const uint32_t lane = threadIdx.x;
     lds_clear(lds, lds_rows);
     uint32_t *const lane_col = lds + lane;
@@ -422,12 +372,18 @@ __global__ __launch_bounds__(64) void an_mc_kernel(uint64_t A, uint32_t n, uint6
     const bool s64 = n > 32;
     uint64_t pending = 0;  // increments per lane counter since the last flush (bound)
     uint32_t cur = 0xFFFFFFFFu;  // segment whose counts the LDS rows hold
+    auto flush = [&] {
+        if (cur != 0xFFFFFFFFu)
+            flush_rows(lds, 0, nbins, ONE ? hist_copy(direct.copies, nbins, kHistCopies) : segs[cur].out);
+    };
     for (uint64_t t = first_item(); t < total_items; t = following_item(counter, t)) {
         uint32_t sg = cur == 0xFFFFFFFFu ? 0 : cur;
-        while (sg + 1 < nsegs && t >= segs[sg + 1].item_begin) ++sg;
-        while (t < segs[sg].item_begin) --sg;
-        sg = uniform32(sg);
-        const McSegment &seg = segs[sg];
+        if (!ONE) {
+            while (sg + 1 < nsegs && t >= segs[sg + 1].item_begin) ++sg;
+            while (t < segs[sg].item_begin) --sg;
+            sg = uniform32(sg);
+        }
+        const McSegment &seg = ONE ? single : segs[sg];
         const uint64_t local = t - seg.item_begin;
         const uint64_t rg = uniform64(local / seg.chunks), c = uniform64(local - rg * seg.chunks);
         const uint64_t j0 = (seg.j0 / CJ + c) * CJ;
@@ -435,7 +391,7 @@ __global__ __launch_bounds__(64) void an_mc_kernel(uint64_t A, uint32_t n, uint6
         const uint64_t j1 = j0 + CJ < seg.j1 ? j0 + CJ : seg.j1;
         const uint64_t add = (uint64_t)G * RM * (j1 - j0);
         if (sg != cur || pending + add >= 0xFFFFFFFFull) {
-            if (cur != 0xFFFFFFFFu) flush_rows(lds, 0, nbins, segs[cur].out);
+            flush();
             cur = sg;
             pending = 0;
         }
@@ -459,47 +415,94 @@ __global__ __launch_bounds__(64) void an_mc_kernel(uint64_t A, uint32_t n, uint6
             }
         }
     }
-    if (cur != 0xFFFFFFFFu) flush_rows(lds, 0, nbins, segs[cur].out);
+    flush();
+    if (ONE) direct_finish(direct, nbins, lds);
 }
 
 // Dynamic LDS of a Hamming wave: the histogram rows (the syndrome tables are
 // the kernel's static LDS).
-size_t ham_lds_bytes(bool, uint32_t lds_rows) { return (size_t)lds_rows * kStride * sizeof(uint32_t); }
+size_t ham_lds_bytes(uint32_t lds_rows) { return (size_t)lds_rows * kStride * sizeof(uint32_t); }
+
+const void *ham_kernel_ptr(bool w64, bool one) {
+    if (one)
+        return w64 ? reinterpret_cast<const void *>(&ham_kernel<true, true>)
+                   : reinterpret_cast<const void *>(&ham_kernel<false, true>);
+    return w64 ? reinterpret_cast<const void *>(&ham_kernel<true, false>)
+               : reinterpret_cast<const void *>(&ham_kernel<false, false>);
+}
+
+// Resident waves per CU (one query per kernel and rows: a property of the
+// kernel and of gfx950's CU), 0 if the query fails.
+uint32_t ham_per_cu(bool w64, uint32_t lds_rows) {
+    static std::atomic<int> cache[2][132];
+    if (lds_rows > 131) return 0;
+    int n = cache[w64][lds_rows].load(std::memory_order_relaxed);
+    if (n > 0) return (uint32_t)n;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, ham_kernel_ptr(w64, false), 64, ham_lds_bytes(lds_rows)) !=
+            hipSuccess ||
+        n <= 0)
+        return 0;
+    cache[w64][lds_rows].store(n, std::memory_order_relaxed);
+    return (uint32_t)n;
+}
 
 }  // namespace
 
-cr_status launch_hamming(const HamJob *d_jobs, uint32_t njobs, uint64_t total_items, bool w64,
-                         unsigned long long *counter, bool allow_static, uint32_t lds_rows, int cus,
-                         hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1) {
-    const void *k = w64 ? reinterpret_cast<const void *>(&ham_kernel<true>)
-                        : reinterpret_cast<const void *>(&ham_kernel<false>);
+namespace {
+
+// Waves of a launch, and whether a static assignment replaces the queue.
+cr_status ham_waves(bool w64, uint64_t total_items, bool allow_static, uint32_t lds_rows, int cus, uint64_t *out) {
     if (lds_rows < 2 || lds_rows > 131) return fail(CR_ERR_INVALID_ARGUMENT, "bad histogram rows %u", lds_rows);
-    const size_t lds = ham_lds_bytes(w64, lds_rows);
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, 64, lds) != hipSuccess || per_cu <= 0)
-        return fail(CR_ERR_DEVICE, "occupancy query failed for the Hamming kernel");
+    const uint32_t per_cu = ham_per_cu(w64, lds_rows);
+    if (per_cu == 0) return fail(CR_ERR_DEVICE, "occupancy query failed for the Hamming kernel");
     uint64_t waves = (uint64_t)per_cu * cus;
     if (waves > total_items) waves = total_items;
     if (waves == 0) waves = 1;
     if (allow_static && total_items > 0) {
         // static assignment over at most one wave per CU less than the
         // resident capacity, each wave taking the same number of items
-        counter = nullptr;
         const uint64_t cap = (uint64_t)(per_cu > 1 ? per_cu - 1 : 1) * cus;
         if (waves > cap) waves = cap;
         const uint64_t per = (total_items + waves - 1) / waves;
         waves = (total_items + per - 1) / per;
     }
-    if (counter) CR_TRY(fill_zero_u64(counter, 1, stream));
-    if (ev0) CR_HIP(hipEventRecord(ev0, stream));
-    const HamJob *a_jobs = d_jobs;
+    *out = waves;
+    return CR_OK;
+}
+
+cr_status ham_launch(const HamJob *jobs, uint32_t njobs, uint64_t total_items, bool w64, unsigned long long *counter,
+                     uint32_t lds_rows, uint64_t waves, const HamJob &single, const DirectResult &out,
+                     hipStream_t stream) {
+    const HamJob *a_jobs = jobs;
     uint32_t a_nj = njobs, a_rows = lds_rows;
     uint64_t a_items = total_items;
     unsigned long long *a_counter = counter;
-    void *args[] = {(void *)&a_jobs, &a_nj, &a_items, &a_counter, &a_rows};
-    CR_HIP(hipLaunchKernel(k, dim3((uint32_t)waves), dim3(64), args, lds, stream));
+    void *args[] = {(void *)&a_jobs, &a_nj, &a_items, &a_counter, &a_rows, (void *)&single, (void *)&out};
+    CR_HIP(hipLaunchKernel(ham_kernel_ptr(w64, !jobs), dim3((uint32_t)waves), dim3(64), args, ham_lds_bytes(lds_rows), stream));
+    return CR_OK;
+}
+
+}  // namespace
+
+cr_status launch_hamming(const HamJob *d_jobs, uint32_t njobs, uint64_t total_items, bool w64,
+                         unsigned long long *counter, bool allow_static, uint32_t lds_rows, int cus,
+                         hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1) {
+    uint64_t waves = 0;
+    CR_TRY(ham_waves(w64, total_items, allow_static, lds_rows, cus, &waves));
+    if (allow_static && total_items > 0) counter = nullptr;
+    if (counter) CR_TRY(fill_zero_u64(counter, 1, stream));
+    if (ev0) CR_HIP(hipEventRecord(ev0, stream));
+    CR_TRY(ham_launch(d_jobs, njobs, total_items, w64, counter, lds_rows, waves, HamJob{}, DirectResult{}, stream));
     if (ev1) CR_HIP(hipEventRecord(ev1, stream));
     return CR_OK;
+}
+
+cr_status launch_hamming_direct(const HamJob &job, bool w64, bool allow_static, uint32_t lds_rows,
+                                const DirectResult &out, int cus, hipStream_t stream) {
+    uint64_t waves = 0;
+    CR_TRY(ham_waves(w64, job.items, allow_static, lds_rows, cus, &waves));
+    return ham_launch(nullptr, 1, job.items, w64, allow_static ? nullptr : out.queue, lds_rows, waves, job, out,
+                      stream);
 }
 
 uint64_t hamming_items(uint64_t count, uint32_t lane_samples) {
@@ -508,27 +511,26 @@ uint64_t hamming_items(uint64_t count, uint32_t lane_samples) {
 }
 
 uint32_t hamming_waves_per_cu(uint32_t lds_rows) {
-    int a = 0, b = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, reinterpret_cast<const void *>(&ham_kernel<false>), 64,
-                                                     ham_lds_bytes(false, lds_rows)) != hipSuccess)
-        a = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, reinterpret_cast<const void *>(&ham_kernel<true>), 64,
-                                                     ham_lds_bytes(true, lds_rows)) != hipSuccess)
-        b = 0;
-    return (uint32_t)std::max(std::max(a, b), 1);
+    return std::max(std::max(ham_per_cu(false, lds_rows), ham_per_cu(true, lds_rows)), 1u);
 }
 
 cr_status launch_an_mc(uint64_t A, uint32_t n, uint64_t seed, McSegment *segs, uint32_t nsegs, McSegment *d_segs,
                        unsigned long long *counter, uint32_t nbins, int cus, hipStream_t stream, hipEvent_t ev0,
-                       hipEvent_t ev1) {
+                       hipEvent_t ev1, const DirectResult *direct) {
     const uint32_t lds_rows = nbins + 1;
     if (lds_rows > 66) return fail(CR_ERR_INVALID_ARGUMENT, "bad histogram rows %u", lds_rows);
     if (nsegs == 0) return fail(CR_ERR_INVALID_ARGUMENT, "no sample range");
-    const void *k = reinterpret_cast<const void *>(&an_mc_kernel);
+    if (direct && nsegs != 1) return fail(CR_ERR_INVALID_ARGUMENT, "one launch, %u sample ranges", nsegs);
+    const void *k = direct ? reinterpret_cast<const void *>(&an_mc_kernel<true>)
+                           : reinterpret_cast<const void *>(&an_mc_kernel<false>);
     const size_t lds = (size_t)lds_rows * kStride * sizeof(uint32_t);
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, 64, lds) != hipSuccess || per_cu <= 0)
-        return fail(CR_ERR_DEVICE, "occupancy query failed for the AN Monte Carlo kernel");
+    static std::atomic<int> cache[2][67];
+    int per_cu = cache[direct != nullptr][lds_rows].load(std::memory_order_relaxed);
+    if (per_cu <= 0) {
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, 64, lds) != hipSuccess || per_cu <= 0)
+            return fail(CR_ERR_DEVICE, "occupancy query failed for the AN Monte Carlo kernel");
+        cache[direct != nullptr][lds_rows].store(per_cu, std::memory_order_relaxed);
+    }
     const uint64_t RBlocks = ((1ull << n) + 64ull * RM - 1) / (64ull * RM);
     uint64_t total_chunks = 0, longest = 0;
     for (uint32_t s = 0; s < nsegs; ++s) {
@@ -553,14 +555,19 @@ cr_status launch_an_mc(uint64_t A, uint32_t n, uint64_t seed, McSegment *segs, u
     }
     uint64_t waves = resident;
     if (waves > items) waves = items;
-    CR_HIP(hipMemcpyAsync(d_segs, segs, nsegs * sizeof(McSegment), hipMemcpyHostToDevice, stream));
-    CR_TRY(fill_zero_u64(counter, 1, stream));
+    if (!direct) {
+        CR_HIP(hipMemcpyAsync(d_segs, segs, nsegs * sizeof(McSegment), hipMemcpyHostToDevice, stream));
+        CR_TRY(fill_zero_u64(counter, 1, stream));
+    }
     if (ev0) CR_HIP(hipEventRecord(ev0, stream));
     uint64_t a_A = A, a_seed = seed, a_items = items;
     uint32_t a_n = n, a_G = G, a_nsegs = nsegs, a_nbins = nbins, a_rows = lds_rows;
-    const McSegment *a_segs = d_segs;
-    unsigned long long *a_counter = counter;
-    void *args[] = {&a_A, &a_n, &a_seed, &a_G, &a_segs, &a_nsegs, &a_items, &a_counter, &a_nbins, &a_rows};
+    const McSegment *a_segs = direct ? nullptr : d_segs;
+    unsigned long long *a_counter = direct ? direct->queue : counter;
+    McSegment a_single = segs[0];
+    DirectResult a_direct = direct ? *direct : DirectResult{};
+    void *args[] = {&a_A, &a_n, &a_seed, &a_G, &a_segs, &a_nsegs, &a_items, &a_counter, &a_nbins, &a_rows, &a_single,
+                    &a_direct};
     CR_HIP(hipLaunchKernel(k, dim3((uint32_t)waves), dim3(64), args, lds, stream));
     if (ev1) CR_HIP(hipEventRecord(ev1, stream));
     return CR_OK;

@@ -36,156 +36,223 @@ extern "C" uint32_t cr_hamming_parity_bits(uint32_t k) {
 
 namespace {
 
-// Requests [0, n) as one Hamming job each: the jobs of 32-bit words in one
-// launch, those of 64-bit words (k > 32) in a second on the same stream, each
-// launch's jobs in request order; requests without samples launch nothing.
-// hists[i * nbins + b] is request i's count of weight b.
+// The weight bins of a request, after its checks.
+cr_status ham_check(const cr_ham_request *req, uint32_t nbins, uint32_t *need, uint32_t *parity, uint64_t masks[7]) {
+    if (req->k < 1 || req->k > 64) return fail(CR_ERR_INVALID_ARGUMENT, "k=%u outside [1, 64]", req->k);
+    if (req->source > CR_HAM_MC) return fail(CR_ERR_INVALID_ARGUMENT, "unknown source %u", req->source);
+    if (req->source == CR_HAM_LIST && req->count && !req->list)
+        return fail(CR_ERR_INVALID_ARGUMENT, "list source without a list");
+    const uint32_t per = req->k <= 32 ? 4 : 2;
+    if (req->source == CR_HAM_MC && req->first % per)
+        return fail(CR_ERR_INVALID_ARGUMENT, "Monte Carlo first sample must be a multiple of %u", per);
+    *parity = hamming_masks(req->k, masks);
+    *need = req->k + *parity + 1;  // weights 0..k+r
+    if (nbins < *need) return fail(CR_ERR_INVALID_ARGUMENT, "nbins=%u but weights reach %u", nbins, *need - 1);
+    return CR_OK;
+}
+
+HamRange ham_range(const cr_ham_request *req, uint32_t need, uint32_t parity, const uint64_t masks[7]) {
+    HamRange job{};
+    job.r = parity;
+    job.nbins = need;
+    ham_range_job(req->first, req->count, req->k, masks, &job);
+    return job;
+}
+
+// Measured rates (words/s): 32-bit stride 1.9e12, 64-bit 0.55e12, Monte Carlo
+// 1.55e12 / 0.75e12, lists about half the stride rates.
+double ham_rate(const cr_ham_request *req) {
+    if (req->source == CR_HAM_MC) return req->k > 32 ? 0.75e12 : 1.55e12;
+    return (req->k > 32 ? 0.55e12 : 1.9e12) * (req->source == CR_HAM_LIST ? 0.5 : 1.0);
+}
+
+// A job and its work assignment in a launch of `waves` resident waves.  The
+// queue balances waves that advance at different rates (a static assignment
+// measured about 25 % slower on launches of 0.5 ms and more), but each queue
+// step is a device-scope atomic on one counter, serialized at about 12.5 ns, one
+// per item plus one per wave: 40-150 us per launch.  Launches estimated below
+// 100 us of work (short_launch) therefore run with a static assignment.
+HamJob ham_job(const cr_ham_request *req, uint32_t need, const uint64_t masks[7], bool short_launch, uint64_t waves) {
+    HamJob job{};
+    memcpy(job.masks, masks, sizeof(job.masks));
+    job.first = req->first;
+    job.stride = req->stride;
+    job.count = req->count;
+    job.seed = req->seed;
+    job.source = req->source;
+    job.k = req->k;
+    job.stream = req->stream;
+    job.nbins = need;
+    // items of 64 x spl words, spl the smallest power of two in [16,
+    // kHamMaxLaneSamples] that gives at most 8 items per resident wave for a
+    // static assignment or 32 for the queue (the last items set the launch's
+    // tail: with at most 4 per wave a 2^30-word (72,64) Monte Carlo launch ran
+    // 20 % below the rate of 2^34 words), and for the queue at least rate/8e7
+    // words per item (the counter's 8e7 items/s)
+    const uint64_t per_wave = short_launch ? 8 : 32;
+    const uint64_t want = (job.count + 64 * per_wave * waves - 1) / (64 * per_wave * waves);
+    const double min_words = short_launch ? 0.0 : ham_rate(req) / 8e7;
+    uint64_t spl = 16;
+    while ((spl < want || 64.0 * (double)spl < min_words) && spl < kHamMaxLaneSamples) spl *= 2;
+    job.lane_samples = (uint32_t)spl;
+    job.items = hamming_items(job.count, job.lane_samples);
+    // dev::kHistCopies line-aligned copies of each histogram, summed at the end
+    job.out_copies = dev::kHistCopies;
+    return job;
+}
+
+// One request in one launch.
+cr_status hamming_single(cr_context *ctx, const cr_ham_request *req, uint64_t *hist, uint32_t nbins,
+                         double *kernel_ms) {
+    if (!ctx || !req || !hist) return fail(CR_ERR_INVALID_ARGUMENT, "NULL argument");
+    uint32_t need = 0, parity = 0;
+    uint64_t masks[7];
+    CR_TRY(ham_check(req, nbins, &need, &parity, masks));
+    CR_HIP(hipSetDevice(ctx->device));
+    if (req->count == 0) {
+        memset(hist, 0, nbins * sizeof(uint64_t));
+        if (kernel_ms) *kernel_ms = 0;
+        return CR_OK;
+    }
+    dev::DirectResult out;
+    if (req->source == CR_HAM_RANGE) {
+        CR_TRY(direct_result(ctx, &out));
+        const HamRange job = ham_range(req, need, parity, masks);
+        CR_TRY(launch_ham_ranges(nullptr, 1, &job, out, ctx->stream));
+        return direct_wait(ctx, hist, need, nbins, kernel_ms);
+    }
+    const bool short_launch = (double)req->count / ham_rate(req) < 100e-6;
+    const uint32_t rows = need + 1;
+    HamJob job = ham_job(req, need, masks, short_launch, (uint64_t)hamming_waves_per_cu(rows) * ctx->cus);
+    if (req->source == CR_HAM_LIST) {
+        CR_TRY(ctx->table_a.reserve(req->count * sizeof(uint64_t)));
+        CR_HIP(hipMemcpyAsync(ctx->table_a.ptr, req->list, req->count * sizeof(uint64_t), hipMemcpyHostToDevice,
+                              ctx->stream));
+        job.list = ctx->table_a.as<uint64_t>();
+    }
+    CR_TRY(direct_result(ctx, &out));
+    job.out = out.copies;
+    CR_TRY(launch_hamming_direct(job, req->k > 32, short_launch, rows, out, ctx->cus, ctx->stream));
+    return direct_wait(ctx, hist, need, nbins, kernel_ms);
+}
+
+// Requests [0, n): ranges as the workgroups of one launch, the others as one
+// Hamming job each, those of 32-bit words in one launch, those of 64-bit words
+// (k > 32) in another on the same stream, each launch's jobs in request order;
+// requests without samples launch nothing.  hists[i * nbins + b] is request
+// i's count of weight b.
 cr_status hamming_run(cr_context *ctx, const cr_ham_request *reqs, uint32_t n, uint64_t *hists, uint32_t nbins,
                       double *kernel_ms) {
     if (!ctx || !reqs || !hists) return fail(CR_ERR_INVALID_ARGUMENT, "NULL argument");
     if (n == 0 || n > kHamMaxBatch)
         return fail(CR_ERR_INVALID_ARGUMENT, "%u requests outside [1, %u]", n, kHamMaxBatch);
+    if (n == 1) return hamming_single(ctx, reqs, hists, nbins, kernel_ms);
+    struct Pending {
+        uint32_t index, need;
+        uint64_t masks[7];
+    };
     struct Launch {
+        std::vector<Pending> requests;
         std::vector<HamJob> jobs;
-        std::vector<uint32_t> index, needs;  // request of each job, and its weight bins
-        std::vector<double> rates;
         double est_s = 0;
         uint32_t rows = 2;
         uint64_t items = 0;
         bool short_launch = false;
     } launches[2];
-    uint64_t list_words = 0;
+    std::vector<HamRange> ranges;
+    struct Result {
+        uint32_t index, need, copies;
+        uint64_t at;
+    };
+    std::vector<Result> results, range_results;
+    uint64_t list_words = 0, entries = 0;
     for (uint32_t q = 0; q < n; ++q) {
         const cr_ham_request *req = reqs + q;
-        if (req->k < 1 || req->k > 64) return fail(CR_ERR_INVALID_ARGUMENT, "k=%u outside [1, 64]", req->k);
-        if (req->source > CR_HAM_MC) return fail(CR_ERR_INVALID_ARGUMENT, "unknown source %u", req->source);
-        if (req->source == CR_HAM_LIST && req->count && !req->list)
-            return fail(CR_ERR_INVALID_ARGUMENT, "list source without a list");
-        const uint32_t per = req->k <= 32 ? 4 : 2;
-        if (req->source == CR_HAM_MC && req->first % per)
-            return fail(CR_ERR_INVALID_ARGUMENT, "Monte Carlo first sample must be a multiple of %u", per);
-        HamJob job{};
-        const uint32_t r = hamming_masks(req->k, job.masks);
-        const uint32_t need = req->k + r + 1;  // weights 0..k+r
-        if (nbins < need) return fail(CR_ERR_INVALID_ARGUMENT, "nbins=%u but weights reach %u", nbins, need - 1);
+        Pending p{q, 0, {}};
+        uint32_t parity = 0;
+        CR_TRY(ham_check(req, nbins, &p.need, &parity, p.masks));
         if (req->count == 0) continue;
-        job.first = req->first;
-        job.stride = req->stride;
-        job.count = req->count;
-        job.seed = req->seed;
-        job.source = req->source;
-        job.k = req->k;
-        job.stream = req->stream;
-        job.nbins = need;
-        // Measured rates (words/s): exhaustive 7.5e12, 32-bit range/stride
-        // 1.9e12, 64-bit 0.55e12, Monte Carlo 1.55e12 / 0.75e12, lists about
-        // half the stride rates.
-        double rate = req->k > 32 ? 0.55e12 : 1.9e12;
-        if (req->source == CR_HAM_RANGE && req->first == 0) rate = 7.5e12;
-        if (req->source == CR_HAM_MC) rate = req->k > 32 ? 0.75e12 : 1.55e12;
-        if (req->source == CR_HAM_LIST) {
-            rate *= 0.5;
-            list_words += req->count;
+        if (req->source == CR_HAM_RANGE) {
+            ranges.push_back(ham_range(req, p.need, parity, p.masks));
+            range_results.push_back({q, p.need, 1, 0});
+            continue;
         }
+        if (req->source == CR_HAM_LIST) list_words += req->count;
         Launch &L = launches[req->k > 32];
-        L.est_s += (double)req->count / rate;
-        L.rows = std::max(L.rows, need + 1);
-        L.jobs.push_back(job);
-        L.index.push_back(q);
-        L.needs.push_back(need);
-        L.rates.push_back(rate);
+        L.est_s += (double)req->count / ham_rate(req);
+        L.rows = std::max(L.rows, p.need + 1);
+        L.requests.push_back(p);
     }
     CR_HIP(hipSetDevice(ctx->device));
     memset(hists, 0, (size_t)n * nbins * sizeof(uint64_t));
     if (kernel_ms) *kernel_ms = 0;
-    if (launches[0].jobs.empty() && launches[1].jobs.empty()) return CR_OK;
+    if (launches[0].requests.empty() && launches[1].requests.empty() && ranges.empty()) return CR_OK;
     if (list_words) CR_TRY(ctx->table_a.reserve(list_words * sizeof(uint64_t)));
-    uint64_t list_at = 0, entries = 0;
-    std::vector<uint64_t> out_at[2];
+    uint64_t list_at = 0;
     for (Launch &L : launches) {
-        // Work assignment.  The queue balances waves that advance at different
-        // rates (a static assignment measured about 25 % slower on launches
-        // of 0.5 ms and more), but each queue step is a device-scope atomic
-        // on one counter, serialized at about 12.5 ns, one per item plus one
-        // per wave: 40-150 us per launch.  Launches estimated below 100 us of
-        // work therefore run with a static assignment.
         L.short_launch = L.est_s < 100e-6;
         const uint64_t waves = (uint64_t)hamming_waves_per_cu(L.rows) * ctx->cus;
-        std::vector<uint64_t> &at = out_at[&L - launches];
-        at.resize(L.jobs.size());
-        for (size_t j = 0; j < L.jobs.size(); ++j) {
-            HamJob &job = L.jobs[j];
-            // items of 64 x spl words, spl the smallest power of two in [16,
-            // kHamMaxLaneSamples] that gives at most 8 items per resident
-            // wave for a static assignment or 32 for the queue (the last
-            // items set the launch's tail: with at most 4 per wave a
-            // 2^30-word (72,64) Monte Carlo launch ran 20 % below the rate of
-            // 2^34 words), and for the queue at least rate/8e7 words per item
-            // (the counter's 8e7 items/s)
-            const uint64_t per_wave = L.short_launch ? 8 : 32;
-            const uint64_t want = (job.count + 64 * per_wave * waves - 1) / (64 * per_wave * waves);
-            const double min_words = L.short_launch ? 0.0 : L.rates[j] / 8e7;
-            uint64_t spl = 16;
-            while ((spl < want || 64.0 * (double)spl < min_words) && spl < kHamMaxLaneSamples) spl *= 2;
-            job.lane_samples = (uint32_t)spl;
-            job.items = hamming_items(job.count, job.lane_samples);
+        for (const Pending &p : L.requests) {
+            const cr_ham_request *req = reqs + p.index;
+            HamJob job = ham_job(req, p.need, p.masks, L.short_launch, waves);
             job.item_begin = L.items;
             L.items += job.items;
             if (job.source == kHamList) {
-                const cr_ham_request *req = reqs + L.index[j];
-                CR_HIP(hipMemcpyAsync(ctx->table_a.as<uint64_t>() + list_at, req->list,
-                                      req->count * sizeof(uint64_t), hipMemcpyHostToDevice, ctx->stream));
+                CR_HIP(hipMemcpyAsync(ctx->table_a.as<uint64_t>() + list_at, req->list, req->count * sizeof(uint64_t),
+                                      hipMemcpyHostToDevice, ctx->stream));
                 job.list = ctx->table_a.as<uint64_t>() + list_at;
                 list_at += req->count;
             }
-            // dev::kHistCopies line-aligned copies of each histogram, summed
-            // on the host
-            job.out_copies = dev::kHistCopies;
-            at[j] = entries;
-            entries += dev::hist_copy_stride(L.needs[j]) * job.out_copies;
+            results.push_back({p.index, p.need, job.out_copies, entries});
+            entries += dev::hist_copy_stride(p.need) * job.out_copies;
+            L.jobs.push_back(job);
         }
     }
+    for (Result &r : range_results) {
+        r.at = entries;
+        entries += dev::hist_copy_stride(r.need);
+    }
     const size_t njobs = launches[0].jobs.size() + launches[1].jobs.size();
+    const size_t job_bytes = njobs * sizeof(HamJob), range_bytes = ranges.size() * sizeof(HamRange);
     CR_TRY(ctx->hist.reserve(entries * sizeof(uint64_t)));
     CR_TRY(ctx->counters.reserve(2 * sizeof(uint64_t)));
-    CR_TRY(ctx->jobs.reserve(njobs * sizeof(HamJob)));
+    CR_TRY(ctx->jobs.reserve(job_bytes + range_bytes));
+    unsigned long long *hist = ctx->hist.as<unsigned long long>();
     std::vector<HamJob> all;
     all.reserve(njobs);
     for (Launch &L : launches)
-        for (size_t j = 0; j < L.jobs.size(); ++j) {
-            L.jobs[j].out = ctx->hist.as<unsigned long long>() + out_at[&L - launches][j];
-            all.push_back(L.jobs[j]);
+        for (HamJob &job : L.jobs) {
+            job.out = hist + results[all.size()].at;
+            all.push_back(job);
         }
-    CR_TRY(fill_zero_u64(ctx->hist.as<unsigned long long>(), entries, ctx->stream));
-    CR_HIP(hipMemcpyAsync(ctx->jobs.ptr, all.data(), njobs * sizeof(HamJob), hipMemcpyHostToDevice, ctx->stream));
+    for (size_t j = 0; j < ranges.size(); ++j) ranges[j].out = hist + range_results[j].at;
+    CR_TRY(fill_zero_u64(hist, entries, ctx->stream));
+    if (njobs) CR_HIP(hipMemcpyAsync(ctx->jobs.ptr, all.data(), job_bytes, hipMemcpyHostToDevice, ctx->stream));
+    HamRange *d_ranges = reinterpret_cast<HamRange *>(ctx->jobs.as<char>() + job_bytes);
+    if (!ranges.empty())
+        CR_HIP(hipMemcpyAsync(d_ranges, ranges.data(), range_bytes, hipMemcpyHostToDevice, ctx->stream));
     // HIP events before the first launch and after the last
-    const bool both = !launches[0].jobs.empty() && !launches[1].jobs.empty();
-    for (int w = 0, first = 1; w < 2; ++w) {
+    if (kernel_ms) CR_HIP(hipEventRecord(ctx->ev0, ctx->stream));
+    if (!ranges.empty())
+        CR_TRY(launch_ham_ranges(d_ranges, (uint32_t)ranges.size(), nullptr, dev::DirectResult{}, ctx->stream));
+    for (int w = 0; w < 2; ++w) {
         const Launch &L = launches[w];
         if (L.jobs.empty()) continue;
-        const bool last = w == 1 || !both;
         CR_TRY(launch_hamming(ctx->jobs.as<HamJob>() + (w ? launches[0].jobs.size() : 0), (uint32_t)L.jobs.size(),
                               L.items, w == 1, ctx->counters.as<unsigned long long>() + w, L.short_launch, L.rows,
-                              ctx->cus, ctx->stream, kernel_ms && first ? ctx->ev0 : nullptr,
-                              kernel_ms && last ? ctx->ev1 : nullptr));
-        first = 0;
+                              ctx->cus, ctx->stream, nullptr, nullptr));
     }
+    if (kernel_ms) CR_HIP(hipEventRecord(ctx->ev1, ctx->stream));
     CR_TRY(ctx->host.reserve(entries * sizeof(uint64_t)));
-    CR_HIP(hipMemcpyAsync(ctx->host.ptr, ctx->hist.ptr, entries * sizeof(uint64_t), hipMemcpyDeviceToHost,
-                          ctx->stream));
+    CR_HIP(hipMemcpyAsync(ctx->host.ptr, hist, entries * sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
     CR_HIP(hipStreamSynchronize(ctx->stream));
     const uint64_t *copies = static_cast<const uint64_t *>(ctx->host.ptr);
-    for (const Launch &L : launches)
-        for (size_t j = 0; j < L.jobs.size(); ++j) {
-            const uint64_t cstride = dev::hist_copy_stride(L.needs[j]);
-            const uint64_t base = out_at[&L - launches][j];
-            uint64_t *hist = hists + (uint64_t)L.index[j] * nbins;
-            for (uint32_t b = 0; b < L.needs[j]; ++b) {
-                uint64_t sum = 0;
-                for (uint32_t c = 0; c < L.jobs[j].out_copies; ++c) sum += copies[base + c * cstride + b];
-                hist[b] = sum;
-            }
-        }
+    results.insert(results.end(), range_results.begin(), range_results.end());
+    for (const Result &r : results) {
+        uint64_t *h = hists + (uint64_t)r.index * nbins;
+        for (uint32_t c = 0; c < r.copies; ++c)
+            for (uint32_t b = 0; b < r.need; ++b) h[b] += copies[r.at + c * dev::hist_copy_stride(r.need) + b];
+    }
     if (kernel_ms) {
         float ms = 0;
         CR_HIP(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
@@ -260,6 +327,14 @@ cr_status an_mc_ranges(cr_context *ctx, uint64_t A, uint32_t n, const uint64_t *
     const uint32_t need = bits + 1;
     if (nbins < need) return fail(CR_ERR_INVALID_ARGUMENT, "nbins=%u but distances reach %u", nbins, need - 1);
     CR_HIP(hipSetDevice(ctx->device));
+    if (count == 1 && bounds[1] > bounds[0]) {
+        dev::DirectResult direct;
+        CR_TRY(direct_result(ctx, &direct));
+        McSegment one{bounds[0], bounds[1], 0, 0, nullptr};
+        CR_TRY(launch_an_mc(A, n, seed, &one, 1, nullptr, nullptr, need, ctx->cus, ctx->stream, nullptr, nullptr,
+                            &direct));
+        return direct_wait(ctx, hists, need, nbins, kernel_ms);
+    }
     memset(hists, 0, (size_t)count * nbins * sizeof(uint64_t));
     if (kernel_ms) *kernel_ms = 0;
     const uint64_t entries = (uint64_t)count * need;
@@ -274,7 +349,7 @@ cr_status an_mc_ranges(cr_context *ctx, uint64_t A, uint32_t n, const uint64_t *
     CR_TRY(fill_zero_u64(out, entries, ctx->stream));
     CR_TRY(launch_an_mc(A, n, seed, segs.data(), (uint32_t)segs.size(), ctx->jobs.as<McSegment>(),
                         ctx->counters.as<unsigned long long>(), need, ctx->cus, ctx->stream,
-                        kernel_ms ? ctx->ev0 : nullptr, kernel_ms ? ctx->ev1 : nullptr));
+                        kernel_ms ? ctx->ev0 : nullptr, kernel_ms ? ctx->ev1 : nullptr, nullptr));
     CR_TRY(ctx->host.reserve(entries * sizeof(uint64_t)));
     CR_HIP(hipMemcpyAsync(ctx->host.ptr, out, entries * sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
     CR_HIP(hipStreamSynchronize(ctx->stream));

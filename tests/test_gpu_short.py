@@ -64,3 +64,21 @@ def test_calls_leave_the_buffers_clean(ctx):
             want[kind, A, N] = ref()
         w = want[kind, A, N]
         assert got[: len(w)] == w[: len(got)], (kind, A, N)
+
+
+def test_single_requests_between_short_codes(ctx):
+    # one-launch Hamming and sample calls of 1 to 66 bins between one-launch
+    # codes: each against the oracle, so a copy or counter left over would show
+    for k, count in [(1, 1), (4, 4), (8, 1000), (32, 4096), (33, 12346), (57, 77778), (64, 2)]:
+        got, ms = ctx.hamming_weights(k, cra.HAM_MC, count=count, seed=7, stream=k)
+        assert got == O.hamming_mc(k, 7, k, 0, count)[:len(got)] and ms > 0
+        words = [(i * 0x9E3779B97F4A7C15) & ((1 << k) - 1) for i in range(count)]
+        got, _ = ctx.hamming_weights(k, cra.HAM_LIST, words=words)
+        assert got == O.hamming_weights_list(k, words)[:len(got)]
+        got, _ = ctx.hamming_weights(k, cra.HAM_STRIDE, count=count, stride=0x9E3779B97F4A7C15)
+        assert got == O.hamming_weights_list(k, words)[:len(got)]
+        got, _ = ctx.an_pairs_auto(61, 256)
+        assert got == O.an_pairs_raw(61, 256, len(got))
+        n = min(k, 20)
+        got, _ = ctx.an_mc(61, n, 33, seed=k)
+        assert got == O.an_mc(61, n, 33, k)[:len(got)]
