@@ -9,7 +9,8 @@
 //   * the column codeword is wave-uniform and advances in SGPRs (v += A), so a
 //     pair costs one v_xor + one v_bcnt (+ bcnt accumulate of the constant
 //     high-dword distance for 33..64-bit words) + one LDS address mad + one
-//     ds_add_u32 into the lane's private column of the histogram;
+//     ds_add_u32 into the lane's private column of the histogram (multipliers
+//     above 2^22: the matrix cores compute the address, see pairs_wide);
 //   * LDS histogram rows are 64 dwords (one per lane), so the bank of every
 //     per-pair atomic is fixed by the lane whatever the distance is: the hot
 //     loop never bank-conflicts; the flush reads each row in a lane-rotated
@@ -119,20 +120,67 @@ __device__ void pairs_w2seg(uint32_t *lane_col, const Rows<R> &rw, uint64_t A, u
     }
 }
 
-// 64-bit codewords, generic: two xors and two bcnts per pair.
+// 64-bit codewords whose high dwords change from column to column: per pair,
+// two XORs, two bit counts and the address, 5 VALU instructions, bounded
+// pairs_w2gen at 6.4e12 pairs/s.  Here the matrix cores deliver the LDS addresses:
+// with a row's bits as +-2 and a column's as -+64,
+//   lane_address + 128 * 64 + sum over 64 bits = lane_address + 256 * distance,
+// the byte address of the pair's counter, so a pair costs its LDS increment alone,
+// and a tile of 32 x 32 pairs two MFMAs.  (Which lane holds which pair of a
+// tile does not matter, nor the order of the bits, alike for both operands.)
+// Measured, A = 58659 * 4097, 1048321 words: 84.4 -> 59.5 ms, 9.25e12 pairs/s
+// of the LDS's 9.5e12; 2^16 words of A = 2^23 + 1 0.40 -> 0.31 ms.
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v16i __attribute__((ext_vector_type(16)));
+
+// 16 bits of a word's low and high dword (the upper ones for lanes 32 .. 63) as
+// bytes: `zero` for a 0, zero ^ flip for a 1.
+__device__ __forceinline__ void bit_bytes(uint64_t w, uint32_t zero, uint32_t flip, v4i (&out)[2]) {
+    const uint32_t shift = (threadIdx.x >> 5) * 16;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+        const uint32_t x = (uint32_t)(w >> (32 * s)) >> shift;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint32_t t = (((x >> (4 * q)) & 15u) * 0x204081u) & 0x01010101u;
+            out[s][q] = (int)((((t << 8) - t) & flip) ^ zero);
+        }
+    }
+}
+
+// Columns [j0, j0 + 32 n) against 64 R full rows from row0.
+template <int R>
+__device__ void pairs_wide(uint32_t *lds, uint64_t A, uint64_t row0, uint64_t j0, uint32_t n) {
+    constexpr int T = R < 4 ? 2 * R : 8;  // row tiles held at a time
+    const uint32_t l = threadIdx.x & 31;
+    v16i c;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) c[e] = (int)(threadIdx.x * 4 + 128 * 64);
+    for (uint32_t p = 0; p < 2 * R; p += T) {
+        v4i rows[T][2];
+#pragma unroll
+        for (int t = 0; t < T; ++t) bit_bytes(A * (row0 + 32 * (p + t) + l), 0x02020202u, 0xFCFCFCFCu, rows[t]);
+        uint64_t v = A * (j0 + l);
+        for (uint32_t q = 0; q < n; ++q, v += 32 * A) {
+            v4i col[2];
+            bit_bytes(v, 0xC0C0C0C0u, 0x80808080u, col);
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                v16i d = __builtin_amdgcn_mfma_i32_32x32x32_i8(rows[t][0], col[0], c, 0, 0, 0);
+                d = __builtin_amdgcn_mfma_i32_32x32x32_i8(rows[t][1], col[1], d, 0, 0, 0);
+#pragma unroll
+                for (int e = 0; e < 16; ++e)
+                    lds_inc(reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(lds) + (uint32_t)d[e]));
+            }
+        }
+    }
+}
+
+// The same pair by pair: the columns that fill no tile.
 template <int R>
 __device__ void pairs_w2gen(uint32_t *lane_col, const Rows<R> &rw, uint64_t A, uint64_t j0, uint64_t j1) {
     uint64_t v = uniform64(A * j0);
-    uint32_t n = uniform32((uint32_t)(j1 - j0));
-    for (; n >= kUnroll; n -= kUnroll) {
-#pragma unroll
-        for (uint32_t u = 0; u < kUnroll; ++u) {
-#pragma unroll
-            for (int r = 0; r < R; ++r) lds_inc(lane_col + __popcll(rw.w[r] ^ v) * kStride);
-            v += A;
-        }
-    }
-    for (; n; --n) {
+    for (uint32_t n = uniform32((uint32_t)(j1 - j0)); n; --n) {
 #pragma unroll
         for (int r = 0; r < R; ++r) lds_inc(lane_col + __popcll(rw.w[r] ^ v) * kStride);
         v += A;
@@ -144,8 +192,11 @@ __global__ void fill_zero_kernel(unsigned long long *p, size_t n) {
         p[i] = 0;
 }
 
-template <int R>
-__global__ __launch_bounds__(64) void pair_kernel(const PairJob *__restrict__ jobs, uint32_t njobs,
+// WIDE: also the code for kModeWide, whose tiles take 130 to 170 registers (3
+// waves a SIMD, which is what keeps the LDS busiest: 9.25e12 pairs/s, 9.0 to
+// 9.1 with 4); with it in one kernel the narrow codes lost 2 to 6 %.
+template <int R, bool WIDE>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WIDE ? 3 : 1))) void pair_kernel(const PairJob *__restrict__ jobs, uint32_t njobs,
                                                   uint64_t total_items, unsigned long long *__restrict__ counter,
                                                   uint32_t lds_rows) {
     extern __shared__ uint32_t lds[];
@@ -213,8 +264,11 @@ __global__ __launch_bounds__(64) void pair_kernel(const PairJob *__restrict__ jo
                 pairs_w1<R>(lane_col, rw, A, jr0, j1);
             else if (job.mode == kModeW2Seg)
                 pairs_w2seg<R>(lane_col, rw, A, jr0, j1);
-            else
-                pairs_w2gen<R>(lane_col, rw, A, jr0, j1);
+            else {
+                const uint32_t tiles = WIDE ? uniform32((uint32_t)(j1 - jr0) / 32) : 0;
+                if (WIDE) pairs_wide<R>(lds, A, row0, jr0, tiles);
+                pairs_w2gen<R>(lane_col, rw, A, jr0 + 32ull * tiles, j1);
+            }
         }
     }
     if (cur != 0xFFFFFFFFu)
@@ -222,16 +276,17 @@ __global__ __launch_bounds__(64) void pair_kernel(const PairJob *__restrict__ jo
 }
 
 template <int R>
-const void *pair_kernel_ptr() {
-    return reinterpret_cast<const void *>(&pair_kernel<R>);
+const void *pair_kernel_ptr(bool wide) {
+    return wide ? reinterpret_cast<const void *>(&pair_kernel<R, true>)
+                : reinterpret_cast<const void *>(&pair_kernel<R, false>);
 }
 
-const void *pair_kernel_for(uint32_t R) {
+const void *pair_kernel_for(uint32_t R, bool wide) {
     switch (R) {
-    case 2: return pair_kernel_ptr<2>();
-    case 4: return pair_kernel_ptr<4>();
-    case 8: return pair_kernel_ptr<8>();
-    case 16: return pair_kernel_ptr<16>();
+    case 2: return pair_kernel_ptr<2>(wide);
+    case 4: return pair_kernel_ptr<4>(wide);
+    case 8: return pair_kernel_ptr<8>(wide);
+    case 16: return pair_kernel_ptr<16>(wide);
     default: return nullptr;
     }
 }
@@ -249,8 +304,9 @@ uint32_t pair_mode(uint64_t A, uint64_t N) {
     const uint32_t bits = pair_max_distance(A, N);
     if (bits <= 32) return kModeW1;
     // high dword of A*j stays constant for about 2^32/A consecutive columns
+    // (at A = 2^22 both modes run at 9.25e12 pairs/s)
     if (A <= (1ull << 22)) return kModeW2Seg;
-    return kModeW2Gen;
+    return kModeWide;
 }
 
 void pair_job_geometry(PairJob &job, uint32_t R, uint32_t Q) {
@@ -263,12 +319,13 @@ void pair_job_geometry(PairJob &job, uint32_t R, uint32_t Q) {
     job.items = pair_prefix(job.T, job.NC, job.Q);
 }
 
-uint32_t pair_waves_per_cu(uint32_t R, uint32_t lds_rows) {
-    // one occupancy query per (R, rows): the answer is a property of the
+uint32_t pair_waves_per_cu(uint32_t R, uint32_t lds_rows, bool wide) {
+    // one occupancy query per (R, rows, kernel): the answer is a property of the
     // kernel and of gfx950's CU, the only target
-    static std::atomic<uint32_t> cache[17][67];
-    const void *k = pair_kernel_for(R);
+    static std::atomic<uint32_t> caches[2][17][67];
+    const void *k = pair_kernel_for(R, wide);
     if (!k || lds_rows > 66) return 0;
+    auto &cache = caches[wide];
     const uint32_t hit = cache[R][lds_rows].load(std::memory_order_relaxed);
     if (hit) return hit;
     int blocks = 0;
@@ -290,14 +347,14 @@ cr_status fill_zero_u64(unsigned long long *p, size_t n, hipStream_t stream) {
 
 cr_status launch_pairs(const PairJob *d_jobs, uint32_t njobs, uint64_t total_items, unsigned long long *counter,
                        const PairLaunchConfig &cfg, int cus, hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1) {
-    const void *k = pair_kernel_for(cfg.R);
+    const void *k = pair_kernel_for(cfg.R, cfg.wide);
     if (!k) return fail(CR_ERR_INVALID_ARGUMENT, "rows_per_lane must be 2, 4, 8 or 16 (got %u)", cfg.R);
     if (cfg.lds_rows < 2 || cfg.lds_rows > 66)
         return fail(CR_ERR_INVALID_ARGUMENT, "histogram rows %u outside [2, 66]", cfg.lds_rows);
     if (njobs == 0) return fail(CR_ERR_INVALID_ARGUMENT, "no jobs");
     uint32_t waves = cfg.waves;
     if (waves == 0) {
-        const uint32_t per_cu = pair_waves_per_cu(cfg.R, cfg.lds_rows);
+        const uint32_t per_cu = pair_waves_per_cu(cfg.R, cfg.lds_rows, cfg.wide);
         if (per_cu == 0) return fail(CR_ERR_DEVICE, "occupancy query failed for the pair kernel");
         waves = per_cu * (uint32_t)cus;
     }
@@ -307,7 +364,7 @@ cr_status launch_pairs(const PairJob *d_jobs, uint32_t njobs, uint64_t total_ite
         // at most one wave per CU less than the resident capacity, each
         // taking the same number of items
         counter = nullptr;
-        const uint32_t per_cu = pair_waves_per_cu(cfg.R, cfg.lds_rows);
+        const uint32_t per_cu = pair_waves_per_cu(cfg.R, cfg.lds_rows, cfg.wide);
         const uint64_t cap = (uint64_t)(per_cu > 1 ? per_cu - 1 : 1) * cus;
         if (waves > cap) waves = (uint32_t)cap;
         const uint64_t per = (total_items + waves - 1) / waves;

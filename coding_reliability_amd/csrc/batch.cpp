@@ -69,14 +69,17 @@ cr_status build_batch(cr_context *ctx, const cr_an_code *codes, uint32_t ncodes,
     L.cfg.R = R;
     L.cfg.lds_rows = std::max(max_need, 1u) + 1;
     L.cfg.waves = tuning ? tuning->waves : 0;
-    const uint32_t per_cu = pair_waves_per_cu(R, L.cfg.lds_rows);
+    for (PairJob &j : L.jobs) {
+        j.mode = pair_mode(j.A, j.N);
+        L.cfg.wide = L.cfg.wide || j.mode == kModeWide;
+    }
+    const uint32_t per_cu = pair_waves_per_cu(R, L.cfg.lds_rows, L.cfg.wide);
     if (per_cu == 0) return fail(CR_ERR_INVALID_ARGUMENT, "rows_per_lane must be 2, 4, 8 or 16 (got %u)", R);
     const long double waves = (long double)per_cu * ctx->cus;
     const long double target = std::max<long double>(total_pairs / (ipw * waves), 1.0L);
     const uint64_t RB = 64ull * R;
     const uint64_t qmax = std::max<uint64_t>(((1ull << 30) / R) / RB, 1);
     for (PairJob &j : L.jobs) {
-        j.mode = pair_mode(j.A, j.N);
         uint64_t Q = (uint64_t)(target / ((long double)RB * RB));
         Q = std::min<uint64_t>(std::max<uint64_t>(Q, 1), qmax);
         pair_job_geometry(j, R, (uint32_t)Q);

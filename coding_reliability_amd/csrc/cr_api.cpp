@@ -327,8 +327,10 @@ cr_status cr_an_pairs_tuned(cr_context *ctx, uint64_t A, uint64_t num_words, uin
     uint32_t R = tuning ? tuning->rows_per_lane : 0, Q = tuning ? tuning->chunk_blocks : 0;
     PairLaunchConfig cfg;
     cfg.lds_rows = need + 1;
+    const uint32_t mode = pair_mode(A, num_words);
+    cfg.wide = mode == kModeWide;
     uint32_t Rr = R ? R : 8;
-    const uint32_t per_cu = pair_waves_per_cu(Rr, cfg.lds_rows);
+    const uint32_t per_cu = pair_waves_per_cu(Rr, cfg.lds_rows, cfg.wide);
     auto_pair_tuning(num_words, per_cu * (uint32_t)ctx->cus, R, Q);
     cfg.R = R;
     cfg.waves = tuning ? tuning->waves : 0;
@@ -341,7 +343,7 @@ cr_status cr_an_pairs_tuned(cr_context *ctx, uint64_t A, uint64_t num_words, uin
     PairJob job{};
     job.A = A;
     job.N = num_words;
-    job.mode = pair_mode(A, num_words);
+    job.mode = mode;
     job.nbins = need;
     pair_job_geometry(job, R, Q);
 

@@ -61,7 +61,7 @@ struct HostBuffer {
 enum PairMode : uint32_t {
     kModeW1 = 0,     // all codewords < 2^32: xor + bcnt per pair
     kModeW2Seg = 1,  // 64-bit codewords, column high dword constant over long segments
-    kModeW2Gen = 2,  // 64-bit codewords, generic two-dword xor + bcnt
+    kModeWide = 2,   // 64-bit codewords, high dword of every column: matrix instructions
 };
 
 struct PairJob {
@@ -116,6 +116,7 @@ struct PairLaunchConfig {
     uint32_t R = 8;
     uint32_t waves = 0;         // 0 = resident capacity of the device
     uint32_t lds_rows = 0;      // histogram rows in LDS (max nbins + 1 dummy row)
+    bool wide = false;          // some job has kModeWide
     bool zero_counter = true;   // false: the caller cleared the queue head already
     bool allow_static = false;  // a short launch: static assignment of items to waves, no queue
 };
@@ -130,7 +131,7 @@ cr_status launch_pairs(const PairJob *d_jobs, uint32_t njobs, uint64_t total_ite
 
 // Resident single-wave workgroups per CU for the pair kernel with R rows per
 // lane and `lds_rows` histogram rows.
-uint32_t pair_waves_per_cu(uint32_t R, uint32_t lds_rows);
+uint32_t pair_waves_per_cu(uint32_t R, uint32_t lds_rows, bool wide);
 
 // Pair histogram of a short code in one launch (see short_pairs.hip).
 constexpr uint32_t kShortWords = 1u << 13;

@@ -102,7 +102,9 @@ extern "C" cr_status cr_an_pairs_noalloc(int device, uint64_t A, uint64_t num_wo
     // histogram always as kHistCopies copies (summed by noalloc_reduce)
     PairLaunchConfig cfg;
     cfg.lds_rows = need + 1;
-    const uint32_t per_cu = pair_waves_per_cu(8, cfg.lds_rows);
+    const uint32_t mode = pair_mode(A, num_words);
+    cfg.wide = mode == kModeWide;
+    const uint32_t per_cu = pair_waves_per_cu(8, cfg.lds_rows, cfg.wide);
     uint32_t R = 0, Q = 0;
     auto_pair_tuning(num_words, per_cu * (uint32_t)g_cus[device], R, Q);
     cfg.R = R;
@@ -113,7 +115,7 @@ extern "C" cr_status cr_an_pairs_noalloc(int device, uint64_t A, uint64_t num_wo
     PairJob job{};
     job.A = A;
     job.N = num_words;
-    job.mode = pair_mode(A, num_words);
+    job.mode = mode;
     job.nbins = need;
     pair_job_geometry(job, R, Q);
     job.item_begin = 0;

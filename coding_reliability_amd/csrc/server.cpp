@@ -180,6 +180,7 @@ cr_status cr_server::iterate(std::vector<Request *> &run) {
     std::vector<std::pair<Request *, uint64_t>> took;
     uint64_t ptotal = 0, htotal = 0;
     uint32_t lds_pair = 2, lds_ham = 2;
+    bool wide = false;
     uint64_t n_an = 0, n_mc = 0;
     for (Request *r : run) {
         if (r->kind == CR_JOB_HAMMING_MC) {
@@ -187,12 +188,13 @@ cr_status cr_server::iterate(std::vector<Request *> &run) {
             ++n_mc;
         } else if (!r->spectral) {
             lds_pair = std::max(lds_pair, r->pj.nbins + 1);
+            wide = wide || r->pj.mode == kModeWide;
             ++n_an;
         }
     }
     std::vector<std::pair<Request *, uint64_t>> spec;
     // waves each launch runs with: a slice floor of two items per wave
-    const uint64_t wp = n_an ? (uint64_t)pair_waves_per_cu(cfg.rows_per_lane, lds_pair) * ctx->cus : 0;
+    const uint64_t wp = n_an ? (uint64_t)pair_waves_per_cu(cfg.rows_per_lane, lds_pair, wide) * ctx->cus : 0;
     const uint64_t wh = n_mc ? (uint64_t)hamming_waves_per_cu(lds_ham) * ctx->cus : 0;
     long double pair_units = 0, ham_units = 0;
     for (Request *r : run) {
@@ -281,6 +283,7 @@ cr_status cr_server::iterate(std::vector<Request *> &run) {
         PairLaunchConfig pc;
         pc.R = cfg.rows_per_lane;
         pc.lds_rows = lds_pair;
+        pc.wide = wide;
         CR_TRY(launch_pairs(pair_jobs.as<PairJob>(), (uint32_t)pjobs.size(), ptotal, ctr, pc, ctx->cus, stream,
                             nullptr, nullptr));
     }
@@ -448,7 +451,7 @@ cr_status cr_server_create(cr_context *ctx, const cr_server_config *cfg, cr_serv
     if (s->cfg.max_active == 0) s->cfg.max_active = 64;
     if (s->cfg.rows_per_lane == 0) s->cfg.rows_per_lane = 8;
     if (s->cfg.iteration_ms <= 0) s->cfg.iteration_ms = 50;
-    if (pair_waves_per_cu(s->cfg.rows_per_lane, 66) == 0)
+    if (pair_waves_per_cu(s->cfg.rows_per_lane, 66, true) == 0)
         return fail(CR_ERR_INVALID_ARGUMENT, "rows_per_lane must be 2, 4, 8 or 16");
     // from here on a failure releases what was created (no worker yet)
     cr_server *raw = s.release();
