@@ -115,12 +115,12 @@ __device__ __forceinline__ void mc_words(const uint32_t (&c)[4], uint64_t (&x)[P
         x[u] = PER == 4 ? (uint64_t)c[u] : ((uint64_t)c[2 * u] | ((uint64_t)c[2 * u + 1] << 32));
 }
 
-__device__ __forceinline__ void mc_block(uint32_t (&c)[4], uint64_t b, uint32_t stream, uint32_t k0, uint32_t k1) {
+__device__ __forceinline__ void mc_block(uint32_t (&c)[4], uint64_t b, uint32_t stream, const PhiloxKeys &keys) {
     c[0] = (uint32_t)b;
     c[1] = (uint32_t)(b >> 32);
     c[2] = stream;
     c[3] = kMcTag;
-    philox4x32_10(c, k0, k1);
+    philox_rounds<0>(c, keys);
 }
 
 template <bool W64, uint32_t PER, bool CHECK, bool FULL>
@@ -128,16 +128,16 @@ __device__ __forceinline__ void mc_blocks(uint32_t *lane_col, const uint8_t *tab
                                           uint32_t spl, uint64_t count, uint64_t dmask, uint32_t dummy) {
     constexpr uint32_t F = (W64 ? 2 : 1) * kFields;
     const uint32_t lane = threadIdx.x;
-    const uint32_t k0 = (uint32_t)job.seed, k1 = (uint32_t)(job.seed >> 32);
+    const PhiloxKeys keys = philox_keys(job.seed);
     const uint32_t nq = spl / PER;
     const uint64_t b0 = (job.first + base) / PER + lane;
     uint32_t c[4];
     uint64_t x[2][PER];
     uint32_t r[2][PER][F];
-    mc_block(c, b0, job.stream, k0, k1);
+    mc_block(c, b0, job.stream, keys);
     mc_words<PER>(c, x[0]);
     table_reads<W64, PER>(x[0], tab, r[0]);
-    mc_block(c, b0 + 64, job.stream, k0, k1);
+    mc_block(c, b0 + 64, job.stream, keys);
     // nq is even (spl is a power of two >= 16): two steps per iteration, the
     // buffers of blocks q and q+1 trading places
     for (uint32_t q = 0; q < nq; q += 2) {
@@ -145,7 +145,7 @@ __device__ __forceinline__ void mc_blocks(uint32_t *lane_col, const uint8_t *tab
         for (uint32_t h = 0; h < 2; ++h) {
             mc_words<PER>(c, x[h ^ 1]);
             table_reads<W64, PER>(x[h ^ 1], tab, r[h ^ 1]);
-            mc_block(c, b0 + 64ull * (q + h + 2), job.stream, k0, k1);
+            mc_block(c, b0 + 64ull * (q + h + 2), job.stream, keys);
             uint32_t w[PER];
             table_weights<W64, PER, FULL>(x[h], dmask, r[h], w);
             const uint64_t s = base + ((uint64_t)(q + h) * 64 + lane) * PER;  // first local sample of this lane
@@ -301,16 +301,20 @@ constexpr int RM = 4;
 constexpr uint32_t CJ = 256;  // samples per item (multiple of 4)
 
 // One AN Monte Carlo item: samples [jlo, j1) of the chunk that starts at j0
-// (a multiple of CJ, so of the words per Philox block).  W1: every codeword
-// fits 32 bits (32-bit multiply, xor and popcount).  S64: 64-bit samples
-// (n > 32).  CHECK: rows past 2^n and samples outside [jlo, j1) (a partial
+// (a multiple of CJ, so of the words per Philox block: the upper half of the
+// block number is the item's).  WIDTH 0: every codeword fits 32 bits (32-bit
+// multiply, xor and popcount), 1: the multiplier does, 2: any.  S64: 64-bit
+// samples (n > 32).  The first two rounds split into what depends on the row,
+// computed once, and what depends on the block number, scalar but for S64.  CHECK: rows past 2^n and samples outside [jlo, j1) (a partial
 // chunk) go to the dummy row; without CHECK, jlo = j0 and j1 - j0 is a
 // multiple of the words per Philox block.
-template <bool W1, bool S64, bool CHECK>
+template <int WIDTH, bool S64, bool CHECK>
 __device__ __forceinline__ void an_mc_item(uint32_t *lane_col, uint64_t A, uint64_t rb, uint64_t nwords, uint64_t j0,
-                                           uint64_t jlo, uint64_t j1, uint64_t smask, uint32_t k0, uint32_t k1,
-                                           uint32_t dummy) {
-    const uint32_t lane = threadIdx.x;
+                                           uint64_t jlo, uint64_t j1, uint64_t smask, uint64_t seed,
+                                           const PhiloxKeys &keys, uint32_t dummy) {
+    constexpr uint32_t M0 = 0xD2511F53u, M1 = 0xCD9E8D57u, W0 = 0x9E3779B9u;
+    const uint32_t k0 = (uint32_t)seed, k1 = (uint32_t)(seed >> 32);
+    const uint32_t lane = threadIdx.x, mask32 = vector_copy((uint32_t)smask), a = vector_copy((uint32_t)A);
     constexpr uint32_t per = S64 ? 2 : 4;
 #pragma unroll
     for (int r = 0; r < RM; ++r) {
@@ -318,10 +322,17 @@ __device__ __forceinline__ void an_mc_item(uint32_t *lane_col, uint64_t A, uint6
         const bool ok = !CHECK || i < nwords;
         const uint64_t w = A * i;
         const uint32_t tag = S64 ? kMcTag ^ (uint32_t)(i >> 32) : kMcTag;
+        const uint64_t row1 = (uint64_t)M1 * (uint32_t)i;  // round 0
+        const uint64_t row2 = (uint64_t)M0 * ((uint32_t)(row1 >> 32) ^ (uint32_t)(j0 / per >> 32) ^ k0);  // round 1
+        const uint32_t e0 = (uint32_t)row1 ^ keys.a[1], e2 = (uint32_t)(row2 >> 32) ^ keys.b[1],
+                       e3 = (uint32_t)row2 ^ keys.b[2];
         for (uint64_t j = CHECK ? jlo / per * per : j0; j < j1; j += per) {
-            const uint64_t blk = j / per;
-            uint32_t c[4] = {(uint32_t)blk, (uint32_t)(blk >> 32), (uint32_t)i, tag};
-            philox4x32_10(c, k0, k1);
+            const uint64_t q0 = (uint64_t)M0 * (uint32_t)(j / per);
+            const uint64_t q1 = (uint64_t)M1 * ((uint32_t)(q0 >> 32) ^ tag ^ k1);
+            const uint64_t p0 = (uint64_t)keys.m0 * (e0 ^ (uint32_t)(q1 >> 32)), p1 = (uint64_t)keys.m1 * (e2 ^ (uint32_t)q0);
+            uint32_t c[4] = {(uint32_t)(p1 >> 32) ^ ((uint32_t)q1 ^ (k0 + 2 * W0)), (uint32_t)p1,
+                             (uint32_t)(p0 >> 32) ^ e3, (uint32_t)p0};
+            philox_rounds<3>(c, keys);
             if (S64) {
 #pragma unroll
                 for (uint32_t u = 0; u < 2; ++u) {
@@ -332,9 +343,10 @@ __device__ __forceinline__ void an_mc_item(uint32_t *lane_col, uint64_t A, uint6
             } else {
 #pragma unroll
                 for (uint32_t u = 0; u < 4; ++u) {
-                    const uint32_t x = c[u] & (uint32_t)smask;
-                    const uint32_t d = W1 ? (uint32_t)__popc((uint32_t)w ^ ((uint32_t)A * x))
-                                          : (uint32_t)__popcll(w ^ (A * (uint64_t)x));
+                    const uint32_t x = c[u] & mask32;
+                    const uint32_t d = WIDTH == 0   ? (uint32_t)__popc((uint32_t)w ^ (a * x))
+                                       : WIDTH == 1 ? (uint32_t)__popcll(w ^ ((uint64_t)a * x))
+                                                    : (uint32_t)__popcll(w ^ (A * (uint64_t)x));
                     lds_inc(lane_col + ((!CHECK || (ok && j + u >= jlo && j + u < j1)) ? d : dummy) * kStride);
                 }
             }
@@ -366,7 +378,7 @@ __global__ __launch_bounds__(64) void an_mc_kernel(uint64_t A, uint32_t n, uint6
     const uint64_t nwords = 1ull << n;
     const uint64_t RBlocks = (nwords + 64ull * RM - 1) / (64ull * RM);
     const uint64_t smask = nwords - 1;
-    const uint32_t k0 = (uint32_t)seed, k1 = (uint32_t)(seed >> 32);
+    const PhiloxKeys keys = philox_keys(seed);
     // all codewords (A * (2^n - 1)) below 2^32
     const bool w1 = ((unsigned __int128)A * (nwords - 1)) >> 32 == 0;
     const bool s64 = n > 32;
@@ -403,15 +415,17 @@ __global__ __launch_bounds__(64) void an_mc_kernel(uint64_t A, uint32_t n, uint6
             const bool full = (rb + 1) * (64ull * RM) <= nwords && jlo == j0 && (j1 - j0) % (s64 ? 2 : 4) == 0;
             if (s64) {
                 if (full)
-                    an_mc_item<false, true, false>(lane_col, A, rb, nwords, j0, jlo, j1, smask, k0, k1, dummy);
+                    an_mc_item<2, true, false>(lane_col, A, rb, nwords, j0, jlo, j1, smask, seed, keys, dummy);
                 else
-                    an_mc_item<false, true, true>(lane_col, A, rb, nwords, j0, jlo, j1, smask, k0, k1, dummy);
-            } else if (w1 && full) {
-                an_mc_item<true, false, false>(lane_col, A, rb, nwords, j0, jlo, j1, smask, k0, k1, dummy);
-            } else if (full) {
-                an_mc_item<false, false, false>(lane_col, A, rb, nwords, j0, jlo, j1, smask, k0, k1, dummy);
+                    an_mc_item<2, true, true>(lane_col, A, rb, nwords, j0, jlo, j1, smask, seed, keys, dummy);
+            } else if (!full) {
+                an_mc_item<2, false, true>(lane_col, A, rb, nwords, j0, jlo, j1, smask, seed, keys, dummy);
+            } else if (w1) {
+                an_mc_item<0, false, false>(lane_col, A, rb, nwords, j0, jlo, j1, smask, seed, keys, dummy);
+            } else if (A >> 32 == 0) {
+                an_mc_item<1, false, false>(lane_col, A, rb, nwords, j0, jlo, j1, smask, seed, keys, dummy);
             } else {
-                an_mc_item<false, false, true>(lane_col, A, rb, nwords, j0, jlo, j1, smask, k0, k1, dummy);
+                an_mc_item<2, false, false>(lane_col, A, rb, nwords, j0, jlo, j1, smask, seed, keys, dummy);
             }
         }
     }
