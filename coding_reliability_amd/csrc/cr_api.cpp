@@ -92,7 +92,7 @@ cr_status direct_result(cr_context *ctx, dev::DirectResult *r) {
     CR_TRY(ctx->host.reserve((dev::kDirectBins + 2) * sizeof(uint64_t)));
     r->copies = ctx->direct.as<unsigned long long>();
     r->queue = r->copies + (size_t)dev::kHistCopies * dev::kDirectBins;
-    r->tickets = reinterpret_cast<unsigned int *>(r->queue + 16);
+    r->tickets = reinterpret_cast<unsigned int *>(r->queue + dev::kQueues * dev::kQueuePitch);
     r->host = ctx->host.as<unsigned long long>();
     return CR_OK;
 }

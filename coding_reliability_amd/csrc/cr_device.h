@@ -70,7 +70,7 @@ __device__ __forceinline__ unsigned long long *hist_copy(unsigned long long *out
 // so a call needs no fill before and no copy after its kernel.
 struct DirectResult {
     unsigned long long *copies = nullptr;  // kHistCopies copies, hist_copy_stride(nbins) apart
-    unsigned long long *queue = nullptr;   // work-queue head
+    unsigned long long *queue = nullptr;   // work-queue heads, kQueuePitch apart
     unsigned int *tickets = nullptr;       // workgroups that are done, by groups of them, then the groups
     unsigned long long *host = nullptr;    // nbins results; from kDirectBins: device clock at the start, at the end
 };
@@ -78,7 +78,11 @@ constexpr uint32_t kDirectBins = 80;  // largest copy stride
 // Device-scope atomics on one address serialize at about 12.5 ns, so the
 // workgroups count themselves in groups, each on a cache line of its own.
 constexpr uint32_t kTicketGroups = 64, kTicketPitch = 32;  // 32-bit tickets between two groups
-constexpr size_t kDirectEntries = (size_t)kHistCopies * kDirectBins + 16 + (kTicketGroups + 1) * kTicketPitch / 2;
+// A launch of many short items divides them over kQueues heads for the same
+// reason (most kernels use the first alone).
+constexpr uint32_t kQueues = 8, kQueuePitch = 16;
+constexpr size_t kDirectEntries =
+    (size_t)kHistCopies * kDirectBins + kQueues * kQueuePitch + (kTicketGroups + 1) * kTicketPitch / 2;
 
 // The call's device time by the device's constant-rate clock: events around
 // the launch cost 9 to 18 us of a 15 us call.
@@ -126,8 +130,9 @@ __device__ inline void direct_finish(const DirectResult &r, uint32_t nbins, uint
     }
     for (uint32_t g = threadIdx.x; g <= kTicketGroups; g += blockDim.x)
         __hip_atomic_store(r.tickets + g * kTicketPitch, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x < kQueues)
+        __hip_atomic_store(r.queue + threadIdx.x * kQueuePitch, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (threadIdx.x == 0) {
-        __hip_atomic_store(r.queue, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         r.host[kDirectBins + 1] = (unsigned long long)wall_clock64();
     }
 }
@@ -148,6 +153,14 @@ __device__ __forceinline__ uint64_t next_item(unsigned long long *counter) {
 __device__ __forceinline__ uint64_t first_item() { return blockIdx.x; }
 __device__ __forceinline__ uint64_t following_item(unsigned long long *counter, uint64_t t) {
     return counter ? (uint64_t)gridDim.x + next_item(counter) : t + gridDim.x;
+}
+
+// The same over n <= kQueues heads: item t belongs to the queue t mod n, wave w
+// to the queue w mod n (with fewer waves than queues each wave has an item and
+// none is left).
+__device__ __forceinline__ uint64_t following_item_of(unsigned long long *heads, uint32_t n) {
+    const uint32_t q = blockIdx.x % n, waves = (gridDim.x - q + n - 1) / n;
+    return q + (uint64_t)n * (waves + next_item(heads + q * kQueuePitch));
 }
 
 // Philox4x32-10 (Salmon, Moraes, Dror, Shaw, SC'11): ten rounds of the 4x32

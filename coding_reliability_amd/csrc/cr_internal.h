@@ -330,7 +330,7 @@ struct McSegment {
 };
 constexpr uint32_t kMcMaxRanges = 64;  // sample ranges per AN Monte Carlo launch
 // segs (host, nsegs entries, kept alive until the stream is synchronized) is
-// completed and copied to d_segs; counter is the work-queue head (zeroed here).
+// completed and copied to d_segs; counter holds the work-queue heads (zeroed here).
 // direct (one segment): its histogram goes there, nothing is copied or zeroed,
 // and d_segs, counter and the events are not used.
 cr_status launch_an_mc(uint64_t A, uint32_t n, uint64_t seed, McSegment *segs, uint32_t nsegs, McSegment *d_segs,

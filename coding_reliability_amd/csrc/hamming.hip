@@ -298,14 +298,16 @@ __global__ __launch_bounds__(64) void ham_kernel(const HamJob *__restrict__ jobs
 //   n >  32: b = j/2, words 2(j%2) (low) and 2(j%2)+1 (high), masked to n bits;
 // the codewords A*i and A*u_ij are compared.
 constexpr int RM = 4;
-constexpr uint32_t CJ = 256;  // samples per item (multiple of 4)
+constexpr uint32_t kMaxChunk = 256;  // most samples per item (CJ: a power of two, 4 or more)
 
 // One AN Monte Carlo item: samples [jlo, j1) of the chunk that starts at j0
 // (a multiple of CJ, so of the words per Philox block: the upper half of the
 // block number is the item's).  WIDTH 0: every codeword fits 32 bits (32-bit
 // multiply, xor and popcount), 1: the multiplier does, 2: any.  S64: 64-bit
 // samples (n > 32).  The first two rounds split into what depends on the row,
-// computed once, and what depends on the block number, scalar but for S64.  CHECK: rows past 2^n and samples outside [jlo, j1) (a partial
+// computed once, and what depends on the block number, scalar but for S64.
+// Bound by VALU issue: 2.95e12 pairs/s at A = 61 (32-bit words; 2.2e12 with whole
+// rounds, scalar keys and a 64-bit sample counter), 2.5e12 at A = 58659, n = 24.  CHECK: rows past 2^n and samples outside [jlo, j1) (a partial
 // chunk) go to the dummy row; without CHECK, jlo = j0 and j1 - j0 is a
 // multiple of the words per Philox block.
 template <int WIDTH, bool S64, bool CHECK>
@@ -324,10 +326,13 @@ __device__ __forceinline__ void an_mc_item(uint32_t *lane_col, uint64_t A, uint6
         const uint32_t tag = S64 ? kMcTag ^ (uint32_t)(i >> 32) : kMcTag;
         const uint64_t row1 = (uint64_t)M1 * (uint32_t)i;  // round 0
         const uint64_t row2 = (uint64_t)M0 * ((uint32_t)(row1 >> 32) ^ (uint32_t)(j0 / per >> 32) ^ k0);  // round 1
-        const uint32_t e0 = (uint32_t)row1 ^ keys.a[1], e2 = (uint32_t)(row2 >> 32) ^ keys.b[1],
-                       e3 = (uint32_t)row2 ^ keys.b[2];
-        for (uint64_t j = CHECK ? jlo / per * per : j0; j < j1; j += per) {
-            const uint64_t q0 = (uint64_t)M0 * (uint32_t)(j / per);
+        uint32_t e0 = (uint32_t)row1 ^ keys.a[1], e2 = (uint32_t)(row2 >> 32) ^ keys.b[1],
+                 e3 = (uint32_t)row2 ^ keys.b[2];
+        asm("" : "+v"(e0), "+v"(e2), "+v"(e3));  // or they are taken apart again in the loop
+        const uint64_t jb = CHECK ? jlo / per * per : j0;
+        uint64_t q0 = (uint64_t)M0 * (uint32_t)(jb / per);
+        for (uint32_t left = uniform32((uint32_t)((j1 - jb + per - 1) / per)), o = 0; left; --left, o += per, q0 += M0) {
+            const uint64_t j = jb + o;
             const uint64_t q1 = (uint64_t)M1 * ((uint32_t)(q0 >> 32) ^ tag ^ k1);
             const uint64_t p0 = (uint64_t)keys.m0 * (e0 ^ (uint32_t)(q1 >> 32)), p1 = (uint64_t)keys.m1 * (e2 ^ (uint32_t)q0);
             uint32_t c[4] = {(uint32_t)(p1 >> 32) ^ ((uint32_t)q1 ^ (k0 + 2 * W0)), (uint32_t)p1,
@@ -365,9 +370,10 @@ __device__ __forceinline__ void an_mc_item(uint32_t *lane_col, uint64_t A, uint6
 // place of the device array.
 template <bool ONE>
 __global__ __launch_bounds__(64) void an_mc_kernel(uint64_t A, uint32_t n, uint64_t seed, uint32_t G,
-                                                   const McSegment *__restrict__ segs, uint32_t nsegs,
-                                                   uint64_t total_items, unsigned long long *__restrict__ counter,
-                                                   uint32_t nbins, uint32_t lds_rows, const McSegment single,
+                                                   uint32_t CJ, uint32_t heads, const McSegment *__restrict__ segs,
+                                                   uint32_t nsegs, uint64_t total_items,
+                                                   unsigned long long *__restrict__ counter, uint32_t nbins,
+                                                   uint32_t lds_rows, const McSegment single,
                                                    const DirectResult direct) {
     extern __shared__ uint32_t lds[];
     if (ONE) direct_start(direct);
@@ -388,7 +394,7 @@ __global__ __launch_bounds__(64) void an_mc_kernel(uint64_t A, uint32_t n, uint6
         if (cur != 0xFFFFFFFFu)
             flush_rows(lds, 0, nbins, ONE ? hist_copy(direct.copies, nbins, kHistCopies) : segs[cur].out);
     };
-    for (uint64_t t = first_item(); t < total_items; t = following_item(counter, t)) {
+    for (uint64_t t = first_item(); t < total_items; t = following_item_of(counter, heads)) {
         uint32_t sg = cur == 0xFFFFFFFFu ? 0 : cur;
         if (!ONE) {
             while (sg + 1 < nsegs && t >= segs[sg + 1].item_begin) ++sg;
@@ -398,7 +404,7 @@ __global__ __launch_bounds__(64) void an_mc_kernel(uint64_t A, uint32_t n, uint6
         const McSegment &seg = ONE ? single : segs[sg];
         const uint64_t local = t - seg.item_begin;
         const uint64_t rg = uniform64(local / seg.chunks), c = uniform64(local - rg * seg.chunks);
-        const uint64_t j0 = (seg.j0 / CJ + c) * CJ;
+        const uint64_t j0 = (seg.j0 & ~(uint64_t)(CJ - 1)) + c * CJ;
         const uint64_t jlo = j0 > seg.j0 ? j0 : seg.j0;
         const uint64_t j1 = j0 + CJ < seg.j1 ? j0 + CJ : seg.j1;
         const uint64_t add = (uint64_t)G * RM * (j1 - j0);
@@ -546,14 +552,25 @@ cr_status launch_an_mc(uint64_t A, uint32_t n, uint64_t seed, McSegment *segs, u
         cache[direct != nullptr][lds_rows].store(per_cu, std::memory_order_relaxed);
     }
     const uint64_t RBlocks = ((1ull << n) + 64ull * RM - 1) / (64ull * RM);
-    uint64_t total_chunks = 0, longest = 0;
+    uint64_t total_chunks = 0, longest = 0, samples = 0;
     for (uint32_t s = 0; s < nsegs; ++s) {
         if (segs[s].j1 <= segs[s].j0) return fail(CR_ERR_INVALID_ARGUMENT, "empty sample range");
-        segs[s].chunks = (segs[s].j1 - segs[s].j0 / CJ * CJ + CJ - 1) / CJ;
-        total_chunks += segs[s].chunks;
         longest = std::max(longest, segs[s].j1 - segs[s].j0);
+        samples += segs[s].j1 - segs[s].j0;
     }
     const uint64_t resident = (uint64_t)per_cu * cus;
+    // Samples per item, and queue heads.  Waves of a CU progress unevenly (the
+    // oldest issues first), so a short launch needs some six items a wave, and
+    // that many steps of one head would serialize (12.5 ns each): 8 heads, one an
+    // XCD.  Longer launches have one, which also evens out the XCDs (with 8
+    // heads 4 % slower).  A = 61, calls of 2^8 words x 10000 samples 65 -> 26 us,
+    // 2^16 x 1000 78 -> 62 us, 2^16 x 10000 332 -> 285 us (some 15 of it this).
+    uint32_t CJ = 16;
+    while (CJ < kMaxChunk && (long double)CJ * 6 * resident < (long double)RBlocks * samples) CJ *= 2;
+    for (uint32_t s = 0; s < nsegs; ++s) {
+        segs[s].chunks = (segs[s].j1 - segs[s].j0 / CJ * CJ + CJ - 1) / CJ;
+        total_chunks += segs[s].chunks;
+    }
     // row blocks per item: about 2^18 pairs per item (a power of two up to
     // 4096), keeping at least 16 items per resident wave
     const uint64_t chunk = longest < CJ ? longest : CJ;
@@ -571,16 +588,16 @@ cr_status launch_an_mc(uint64_t A, uint32_t n, uint64_t seed, McSegment *segs, u
     if (waves > items) waves = items;
     if (!direct) {
         CR_HIP(hipMemcpyAsync(d_segs, segs, nsegs * sizeof(McSegment), hipMemcpyHostToDevice, stream));
-        CR_TRY(fill_zero_u64(counter, 1, stream));
+        CR_TRY(fill_zero_u64(counter, kQueues * kQueuePitch, stream));
     }
     if (ev0) CR_HIP(hipEventRecord(ev0, stream));
     uint64_t a_A = A, a_seed = seed, a_items = items;
-    uint32_t a_n = n, a_G = G, a_nsegs = nsegs, a_nbins = nbins, a_rows = lds_rows;
+    uint32_t a_n = n, a_G = G, a_CJ = CJ, a_heads = CJ < kMaxChunk ? kQueues : 1, a_nsegs = nsegs, a_nbins = nbins, a_rows = lds_rows;
     const McSegment *a_segs = direct ? nullptr : d_segs;
     unsigned long long *a_counter = direct ? direct->queue : counter;
     McSegment a_single = segs[0];
     DirectResult a_direct = direct ? *direct : DirectResult{};
-    void *args[] = {&a_A, &a_n, &a_seed, &a_G, &a_segs, &a_nsegs, &a_items, &a_counter, &a_nbins, &a_rows, &a_single,
+    void *args[] = {&a_A, &a_n, &a_seed, &a_G, &a_CJ, &a_heads, &a_segs, &a_nsegs, &a_items, &a_counter, &a_nbins, &a_rows, &a_single,
                     &a_direct};
     CR_HIP(hipLaunchKernel(k, dim3((uint32_t)waves), dim3(64), args, lds, stream));
     if (ev1) CR_HIP(hipEventRecord(ev1, stream));

@@ -339,7 +339,7 @@ cr_status an_mc_ranges(cr_context *ctx, uint64_t A, uint32_t n, const uint64_t *
     if (kernel_ms) *kernel_ms = 0;
     const uint64_t entries = (uint64_t)count * need;
     CR_TRY(ctx->hist.reserve(entries * sizeof(uint64_t)));
-    CR_TRY(ctx->counters.reserve(sizeof(uint64_t)));
+    CR_TRY(ctx->counters.reserve(dev::kQueues * dev::kQueuePitch * sizeof(uint64_t)));
     CR_TRY(ctx->jobs.reserve(count * sizeof(McSegment)));
     unsigned long long *out = ctx->hist.as<unsigned long long>();
     std::vector<McSegment> segs;
