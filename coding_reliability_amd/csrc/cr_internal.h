@@ -286,23 +286,31 @@ bool carry_tiles_plan(uint64_t A, uint32_t k, CarryTilesPlan *p);
 cr_status carry_tiles_run(const CarryTilesPlan &p, void *table, unsigned long long *hist, int cus,
                           hipStream_t stream);
 
-// Weight histogram of consecutive data words by aligned blocks (see
+// Weight histogram of consecutive data words, bit by bit of their bounds (see
 // hamming_range.hip).
 struct HamRange {
-    struct Block {  // the words d0 | x, x < 2^m, counted `weight` times
-        uint64_t weight;
-        uint16_t m, ones, parity, reserved;  // ones: popcount(d0); parity: parity bits of d0
-    };
     unsigned long long *out;  // device histogram, nbins entries (written, not added to)
-    uint32_t r, nbins, nblocks, reserved;
-    uint32_t cols[64];        // parity bits of 2^m
-    Block blocks[136];        // in order of m: at most two of each size and one for whole turns
+    uint32_t r, nbins;
+    uint32_t steps;       // of two data bits, from the top
+    uint32_t start_bits;  // 1 for an odd width, whose top bit the start entries include
+    struct Start {
+        uint64_t weight;
+        uint32_t at, reserved;  // at: (popcount << r) + parity bits
+    } start[4];
+    struct Step {
+        uint16_t col[2];  // parity bits of the step's upper and lower data bit
+        struct {
+            uint16_t at;
+            int16_t sign;
+        } enter[6];  // words that leave the range's start (-1) or end (+1) in this step
+    } step[32];
 };
-// The blocks of [first, first + count) modulo 2^k.
+// The words [first, first + count) modulo 2^k; job->r is set.
 void ham_range_job(uint64_t first, uint64_t count, uint32_t k, const uint64_t masks[7], HamRange *job);
-// The jobs of a device array, or (single) one whose histogram goes to out.host.
-cr_status launch_ham_ranges(const HamRange *d_jobs, uint32_t njobs, const HamRange *single,
-                            const dev::DirectResult &out, hipStream_t stream);
+// The jobs of a device array, or (single) one whose histogram goes to out.host;
+// the largest width and parity bits among them.
+cr_status launch_ham_ranges(const HamRange *d_jobs, uint32_t njobs, const HamRange *single, uint32_t max_k,
+                            uint32_t max_r, const dev::DirectResult &out, hipStream_t stream);
 
 // Parity masks of the (N,k) extended Hamming codes, truncated to k bits;
 // returns the number of non-overall parity bits.

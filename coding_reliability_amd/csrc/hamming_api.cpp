@@ -118,7 +118,7 @@ cr_status hamming_single(cr_context *ctx, const cr_ham_request *req, uint64_t *h
     if (req->source == CR_HAM_RANGE) {
         CR_TRY(direct_result(ctx, &out));
         const HamRange job = ham_range(req, need, parity, masks);
-        CR_TRY(launch_ham_ranges(nullptr, 1, &job, out, ctx->stream));
+        CR_TRY(launch_ham_ranges(nullptr, 1, &job, req->k, parity, out, ctx->stream));
         return direct_wait(ctx, hist, need, nbins, kernel_ms);
     }
     const bool short_launch = (double)req->count / ham_rate(req) < 100e-6;
@@ -160,6 +160,7 @@ cr_status hamming_run(cr_context *ctx, const cr_ham_request *reqs, uint32_t n, u
         bool short_launch = false;
     } launches[2];
     std::vector<HamRange> ranges;
+    uint32_t range_k = 0, range_r = 0;
     struct Result {
         uint32_t index, need, copies;
         uint64_t at;
@@ -174,6 +175,8 @@ cr_status hamming_run(cr_context *ctx, const cr_ham_request *reqs, uint32_t n, u
         if (req->count == 0) continue;
         if (req->source == CR_HAM_RANGE) {
             ranges.push_back(ham_range(req, p.need, parity, p.masks));
+            range_k = std::max(range_k, req->k);
+            range_r = std::max(range_r, parity);
             range_results.push_back({q, p.need, 1, 0});
             continue;
         }
@@ -234,7 +237,8 @@ cr_status hamming_run(cr_context *ctx, const cr_ham_request *reqs, uint32_t n, u
     // HIP events before the first launch and after the last
     if (kernel_ms) CR_HIP(hipEventRecord(ctx->ev0, ctx->stream));
     if (!ranges.empty())
-        CR_TRY(launch_ham_ranges(d_ranges, (uint32_t)ranges.size(), nullptr, dev::DirectResult{}, ctx->stream));
+        CR_TRY(launch_ham_ranges(d_ranges, (uint32_t)ranges.size(), nullptr, range_k, range_r, dev::DirectResult{},
+                                 ctx->stream));
     for (int w = 0; w < 2; ++w) {
         const Launch &L = launches[w];
         if (L.jobs.empty()) continue;

@@ -1,5 +1,5 @@
-"""Range requests of the Extended Hamming weights by aligned blocks: the block
-identity restated with Python integers against the oracle (CPU), and the kernel
+"""Range requests of the Extended Hamming weights by the recursion over data
+bits: restated with Python integers against the oracle (CPU), and the kernel
 against the oracle, the word lists' kernel and the MacWilliams closed form (GPU)."""
 import random
 
@@ -10,49 +10,34 @@ import coding_reliability_amd as cra
 from oracle import oracle as O
 
 
-def blocks(lo, hi):
-    """[lo, hi) as aligned blocks (first word, log2 of the size)."""
-    m = 0
-    while lo < hi:
-        if lo & 1:
-            yield lo << m, m
-            lo += 1
-        if lo < hi and hi & 1:
-            hi -= 1
-            yield hi << m, m
-        lo, hi, m = lo >> 1, hi >> 1, m + 1
-
-
-@pytest.mark.parametrize("k,lo,hi", [(1, 0, 2), (5, 3, 29), (8, 0, 256), (11, 1, 2048), (16, 12345, 54321)])
-def test_blocks_give_the_weights(k, lo, hi):
-    # weight(d0 | x) = popcount(d0) + popcount(x) + popcount(S(d0) ^ S(x)) for the
-    # parity bits S, linear; S(x) read off the oracle's codewords
-    r = O.hamming_parity_bits(k)
+@pytest.mark.parametrize("k,lo,hi", [(1, 0, 2), (1, 1, 2), (5, 3, 29), (8, 0, 256), (11, 1, 2048), (16, 12345, 54321)])
+def test_recursion_gives_the_weights(k, lo, hi):
+    # whole extended codewords here: the bits of S are the codeword of a data bit
     S = [O.hamming_codeword_ext(1 << i, k) for i in range(k)]
-
-    def syn(x):
-        s = 0
-        for i in range(k):
-            if x >> i & 1:
-                s ^= S[i]
-        return s
-
-    J, at, out, m = {(0, 0): 1}, sorted(blocks(lo, hi), key=lambda b: b[1]), [0] * (k + r + 2), 0
-    for d0, size in at:
-        while m < size:
-            nxt = dict(J)
-            for (j, s), n in J.items():
-                key = (j + 1, s ^ S[m])
-                nxt[key] = nxt.get(key, 0) + n
-            J, m = nxt, m + 1
-        for (j, s), n in J.items():
-            out[(s ^ syn(d0)).bit_count()] += n  # whole extended codewords here
+    size, L = 1 << k, {}
+    ends = [(lo, -1), (hi % size, 1)]
+    if hi >= size:
+        L[0] = 1
+    for t in reversed(range(k)):
+        nxt = {}
+        for s, n in L.items():
+            for x in (s, s ^ S[t]):
+                nxt[x] = nxt.get(x, 0) + n
+        for v, sign in ends:
+            if v >> t & 1:  # the words below v that leave it at bit t
+                x = 0
+                for i in range(t + 1, k):
+                    x ^= S[i] if v >> i & 1 else 0
+                nxt[x] = nxt.get(x, 0) + sign
+        L = nxt
     want = O.hamming_weights(k, lo, hi)
-    ext = [0] * len(out)
-    for w, n in enumerate(want[:len(out)]):
-        if n:
-            ext[w + (w & 1)] += n
-    assert out == ext
+    ext = [0] * (len(want) + 1)
+    for w, n in enumerate(want):
+        ext[w + (w & 1)] += n
+    got = [0] * len(ext)
+    for s, n in L.items():
+        got[s.bit_count()] += n
+    assert got == ext
 
 
 @pytest.fixture(scope="module")
