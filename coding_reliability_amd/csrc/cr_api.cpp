@@ -387,7 +387,7 @@ cr_status cr_an_pairs_tuned(cr_context *ctx, uint64_t A, uint64_t num_words, uin
 cr_status cr_an_pairs(cr_context *ctx, uint64_t A, uint64_t num_words, uint64_t *raw, uint32_t nbins,
                       double *kernel_ms) {
     // the same histogram by whichever method is estimated to be the fastest:
-    // the short kernel (measured 18 us a call of 2^8 words, 29 us of 2^13), the
+    // the short kernel (measured 17 us a call of 2^8 words, 25 us of 2^13), the
     // pair kernel (40 us a call and about 7e12 pairs/s where it competes), the
     // sliced kernel (49 us at 2^14 words, then the rates of sliced_rate), the
     // code's spectrum, the recursions over carries
@@ -395,7 +395,7 @@ cr_status cr_an_pairs(cr_context *ctx, uint64_t A, uint64_t num_words, uint64_t 
     const double pairs = 0.5 * (double)num_words * (double)num_words;
     const bool is_short = A != 0 && num_words != 0 && num_words <= kShortWords &&
                           !((unsigned __int128)(num_words - 1) * A >> 64);
-    double best = is_short ? 20e-6 + pairs / 3.5e12 : 40e-6 + pairs / 7e12;
+    double best = is_short ? 20e-6 + pairs / 6.7e12 : 40e-6 + pairs / 7e12;
     SlicedJob sliced;
     bool by_planes = false;
     if (sliced_job(A, num_words, &sliced)) {
