@@ -28,7 +28,7 @@
 // 64 bits, so steps take two levels, not one); longer ones are bound by the 16
 // loads per counter (9 TB/s from L1 and L2 at A = 1021).  Measured for one
 // call, against the spectral path that served these codes before: 6-bit A at
-// k = 24 46 us (1.13 ms), at k = 32 64 us (993 ms), A = 1021 at k = 24 0.85 ms
+// k = 24 40 us (1.13 ms), at k = 32 57 us (993 ms), A = 1021 at k = 24 0.84 ms
 // (14.9 ms).
 #include <algorithm>
 #include <vector>
@@ -201,7 +201,7 @@ bool carry_plan(uint64_t A, uint32_t k, CarryPlan *p) {
     // 1021, k = 14 .. 32): 100 ps a carry pair for the first and the last
     // kernel, two levels 3.2 us and 6.5 ps a counter in 32 bits, 4.4 us and 11 ps
     // in 64.
-    double s = 22e-6 + 1.0e-10 * p->states;
+    double s = 17e-6 + 1.0e-10 * p->states;
     for (uint32_t r = kInitBits; r < p->levels;) {
         r += ((p->levels - r) & 1) ? 1 : 2;
         s += wide(r) ? 4.4e-6 : 3.2e-6;

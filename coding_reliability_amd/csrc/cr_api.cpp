@@ -1,5 +1,6 @@
 // Context management, error reporting and the exhaustive-AN entry point.
 #include <algorithm>
+#include <chrono>
 #include <cstdio>
 #include <cstring>
 
@@ -94,11 +95,20 @@ cr_status direct_result(cr_context *ctx, dev::DirectResult *r) {
     r->queue = r->copies + (size_t)dev::kHistCopies * dev::kDirectBins;
     r->tickets = reinterpret_cast<unsigned int *>(r->queue + dev::kQueues * dev::kQueuePitch);
     r->host = ctx->host.as<unsigned long long>();
+    r->host[dev::kDirectBins + 1] = 0;
     return CR_OK;
 }
 
 cr_status direct_wait(cr_context *ctx, uint64_t *raw, uint32_t need, uint32_t nbins, double *kernel_ms) {
-    CR_HIP(hipStreamSynchronize(ctx->stream));
+    // the kernel's last store, after its results: seen 3 to 6 us before the runtime
+    // reports the stream idle (calls of 17 to 46 us; a stream query after it
+    // costs 10 us).  Calls that take long, or fail, wait for the runtime.
+    const uint64_t *end = ctx->host.as<uint64_t>() + dev::kDirectBins + 1;
+    const auto limit = std::chrono::steady_clock::now() + std::chrono::microseconds(1000);
+    bool done;
+    while (!(done = __atomic_load_n(end, __ATOMIC_ACQUIRE) != 0) && std::chrono::steady_clock::now() < limit) {
+    }
+    if (!done) CR_HIP(hipStreamSynchronize(ctx->stream));
     memcpy(raw, ctx->host.ptr, need * sizeof(uint64_t));
     memset(raw + need, 0, (nbins - need) * sizeof(uint64_t));
     if (kernel_ms) {
@@ -387,19 +397,19 @@ cr_status cr_an_pairs_tuned(cr_context *ctx, uint64_t A, uint64_t num_words, uin
 cr_status cr_an_pairs(cr_context *ctx, uint64_t A, uint64_t num_words, uint64_t *raw, uint32_t nbins,
                       double *kernel_ms) {
     // the same histogram by whichever method is estimated to be the fastest:
-    // the short kernel (measured 17 us a call of 2^8 words, 25 us of 2^13), the
+    // the short kernel (measured 13 us a call of 2^8 words, 20 us of 2^13), the
     // pair kernel (40 us a call and about 7e12 pairs/s where it competes), the
-    // sliced kernel (49 us at 2^14 words, then the rates of sliced_rate), the
+    // sliced kernel (38 us at 2^14 words, then the rates of sliced_rate), the
     // code's spectrum, the recursions over carries
     uint32_t k = 0;
     const double pairs = 0.5 * (double)num_words * (double)num_words;
     const bool is_short = A != 0 && num_words != 0 && num_words <= kShortWords &&
                           !((unsigned __int128)(num_words - 1) * A >> 64);
-    double best = is_short ? 20e-6 + pairs / 6.7e12 : 40e-6 + pairs / 7e12;
+    double best = is_short ? 15e-6 + pairs / 6.7e12 : 40e-6 + pairs / 7e12;
     SlicedJob sliced;
     bool by_planes = false;
     if (sliced_job(A, num_words, &sliced)) {
-        const double s = 38e-6 + pairs / sliced_rate(sliced);
+        const double s = 33e-6 + pairs / sliced_rate(sliced);
         by_planes = s < best;
         best = std::min(best, s);
     }

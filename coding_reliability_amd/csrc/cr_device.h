@@ -84,10 +84,24 @@ constexpr uint32_t kQueues = 8, kQueuePitch = 16;
 constexpr size_t kDirectEntries =
     (size_t)kHistCopies * kDirectBins + kQueues * kQueuePitch + (kTicketGroups + 1) * kTicketPitch / 2;
 
+// A result; system scope, so that it goes past the caches.
+__device__ __forceinline__ void direct_store(const DirectResult &r, uint32_t i, unsigned long long x) {
+    __hip_atomic_store(r.host + i, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // The call's device time by the device's constant-rate clock: events around
 // the launch cost 9 to 18 us of a 15 us call.
 __device__ __forceinline__ void direct_start(const DirectResult &r) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) r.host[kDirectBins] = (unsigned long long)wall_clock64();
+    if (blockIdx.x == 0 && threadIdx.x == 0) direct_store(r, kDirectBins, (unsigned long long)wall_clock64());
+}
+
+// Called by every thread of the workgroup that has written the results.  The
+// end clock tells the host that they are there: it is written when every
+// wave's stores have been acknowledged.
+__device__ __forceinline__ void direct_end(const DirectResult &r) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) direct_store(r, kDirectBins + 1, (unsigned long long)wall_clock64());
 }
 
 // Called by every thread of every workgroup (a multiple of 64 threads) after
@@ -125,16 +139,14 @@ __device__ inline void direct_finish(const DirectResult &r, uint32_t nbins, uint
         for (int u = 0; u < 8; ++u) {
 #pragma unroll
             for (int d = kHistCopies / 2; d > 0; d >>= 1) s[u] += __shfl_xor(s[u], d, kHistCopies);
-            if (c == 0 && b0 + u * step < nbins) r.host[b0 + u * step] = s[u];
+            if (c == 0 && b0 + u * step < nbins) direct_store(r, b0 + u * step, s[u]);
         }
     }
     for (uint32_t g = threadIdx.x; g <= kTicketGroups; g += blockDim.x)
         __hip_atomic_store(r.tickets + g * kTicketPitch, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (threadIdx.x < kQueues)
         __hip_atomic_store(r.queue + threadIdx.x * kQueuePitch, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (threadIdx.x == 0) {
-        r.host[kDirectBins + 1] = (unsigned long long)wall_clock64();
-    }
+    direct_end(r);
 }
 
 // Work-queue head: lane 0 takes the next item, every lane sees it.

@@ -9,7 +9,7 @@
 // histogram (a counter a distance and lane, ds_add_u32 to the lane's own bank);
 // the last workgroup to finish writes the sums to pinned host memory
 // (direct_finish).  A call of 2^8 words takes one workgroup.  Measured a call
-// (device time): 2^8 words 19.6 us (3.5), 2^13 29 us (12); the pair kernel with
+// (device time): 2^8 words 13.5 us (3.5), 2^13 20 us (12); the pair kernel with
 // its fill, job upload, result copy and timing events 43 us (15) and 49 us (20).
 #include <algorithm>
 
@@ -94,15 +94,15 @@ __global__ __launch_bounds__(kThreads) void short_kernel(ShortJob job, DirectRes
         for (int d = 32; d > 0; d >>= 1) x += __shfl_xor(x, d, 64);
         if (lane == 0) {
             if (gridDim.x == 1)
-                out.host[b] = x;
+                direct_store(out, b, x);
             else if (x)
                 atomicAdd(hist_copy(out.copies, job.nbins, kHistCopies) + b, (unsigned long long)x);
         }
     }
     if (gridDim.x > 1)
         direct_finish(out, job.nbins, &flag);
-    else if (threadIdx.x == 0)
-        out.host[kDirectBins + 1] = (unsigned long long)wall_clock64();
+    else
+        direct_end(out);
 }
 
 const void *short_kernel_for(uint32_t R, bool w2) {
