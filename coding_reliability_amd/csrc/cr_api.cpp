@@ -399,7 +399,7 @@ cr_status cr_an_pairs(cr_context *ctx, uint64_t A, uint64_t num_words, uint64_t 
     // the same histogram by whichever method is estimated to be the fastest:
     // the short kernel (measured 13 us a call of 2^8 words, 20 us of 2^13), the
     // pair kernel (40 us a call and about 7e12 pairs/s where it competes), the
-    // sliced kernel (38 us at 2^14 words, then the rates of sliced_rate), the
+    // sliced kernel (34 us at 2^14 words, then the rates of sliced_rate), the
     // code's spectrum, the recursions over carries
     uint32_t k = 0;
     const double pairs = 0.5 * (double)num_words * (double)num_words;
@@ -409,7 +409,7 @@ cr_status cr_an_pairs(cr_context *ctx, uint64_t A, uint64_t num_words, uint64_t 
     SlicedJob sliced;
     bool by_planes = false;
     if (sliced_job(A, num_words, &sliced)) {
-        const double s = 33e-6 + pairs / sliced_rate(sliced);
+        const double s = 27e-6 + pairs / sliced_rate(sliced);
         by_planes = s < best;
         best = std::min(best, s);
     }

@@ -152,7 +152,7 @@ struct SlicedJob {
     uint32_t A, Ainv, tc;        // odd part, its inverse modulo 2^k, (A * Ainv - 1) >> k
     uint32_t k;                  // word bits, 11 .. 24
     uint32_t planes;             // codeword bits above the low k, at most 16
-    uint32_t parts;              // items that share a 64 x 64 block of words: 1, 2 or 4
+    uint32_t parts;              // items that share a 64 x 64 block of words: 1, 2, 4, 8 or 16
     uint32_t nbins, out_copies;  // as PairJob's
 };
 static_assert(sizeof(SlicedJob) == 56, "SlicedJob layout");

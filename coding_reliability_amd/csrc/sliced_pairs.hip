@@ -13,12 +13,12 @@
 // from which the counts of the values 0 .. 15 follow by inclusion-exclusion.
 // 68 instructions for 32 pairs of 16-bit h's, 58 for 15 bits, 54 for 12, 24 for
 // 7, where the pair kernel takes 3 and an LDS increment (which bounds it) for
-// one.  Bound by VALU issue: 19.9e12 pairs/s for 16-bit multipliers at k = 18
-// (9.4e12 in the pair kernel), 42e12 lane instructions/s of the 42e12 that the
-// device issues; 1024 mixed codes of 8 to 18 bits 199 ms (473 ms).  A single
-// code of 2^16 words takes 0.16 ms (0.34 ms), of 2^14 49 us (64 us); below that
-// four workgroups per block of 64 x 64 words are too few, and the short kernel
-// takes over.
+// one.  Bound by VALU issue: 20.3e12 pairs/s for 16-bit multipliers at k = 18
+// (9.4e12 in the pair kernel), 43e12 lane instructions/s, where bit counts
+// issue at 37e12 and XORs and bitop3 at up to 55e12 (51e12 in this mix); 1024
+// mixed codes of 8 to 18 bits 197 ms (473 ms).  A single code of 2^16 words takes
+// 0.155 ms (0.34 ms), of 2^14 34 us (64 us); below that four workgroups per
+// block of 64 x 64 words are too few, and the short kernel takes over.
 //
 // The first adders work on triples of planes (p1, p2, p3) stored as p1, p1 ^
 // p2, p1 ^ p3, p1 ^ p2 ^ p3, for either side: the sum is one XOR and the
@@ -30,7 +30,7 @@
 // popcount(delta), so that popcount(x) is the same for the wave and the product
 // counts are kept in registers over a popcount class; they are added to LDS
 // counters by class (popcount of delta and xb).  The four waves and up to four
-// workgroups share the 32 xb.
+// workgroups share the 32 xb, and in small launches up to four the delta.
 #include <algorithm>
 #include <atomic>
 
@@ -163,6 +163,22 @@ struct Lds {
     unsigned long long item;
 };
 
+// Bit i of byte j of the eight bytes of x (lower four) and y trades places with
+// bit j of byte i.
+__device__ __forceinline__ void transpose8(uint32_t &x, uint32_t &y) {
+    auto step = [](uint32_t &v, uint32_t shift, uint32_t mask) {
+        const uint32_t t = (v ^ (v >> shift)) & mask;
+        v = CR_XOR3(v, t, t << shift);
+    };
+    step(x, 7, 0x00AA00AAu);
+    step(y, 7, 0x00AA00AAu);
+    step(x, 14, 0x0000CCCCu);
+    step(y, 14, 0x0000CCCCu);
+    const uint32_t t = (x ^ (y << 4)) & 0xF0F0F0F0u;
+    x ^= t;
+    y ^= t >> 4;
+}
+
 // The planes of words 64 * block + l: thread (l, q) takes elements 8q .. 8q + 7
 // of its word, h advanced as in the spectral generator (see next_high there).
 __device__ __forceinline__ void generate(Lds &L, const SlicedJob &job, uint32_t block) {
@@ -170,16 +186,28 @@ __device__ __forceinline__ void generate(Lds &L, const SlicedJob &job, uint32_t 
     const uint32_t lo = ((block * 64 + l) << 5) + 8 * q;
     const uint32_t i = (lo * job.Ainv) & ((1u << job.k) - 1);
     uint32_t h = (uint32_t)(((uint64_t)job.A * i) >> job.k);
-    uint32_t byte[16] = {};
+    uint32_t two[4];  // elements 2e, 2e + 1
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-#pragma unroll
-        for (int b = 0; b < 16; ++b) byte[b] |= ((h >> b) & 1) << e;
+        two[e / 2] = e & 1 ? two[e / 2] | h << 16 : h;
         const uint32_t t = h + job.tc;
         h = min(t, t - job.A);
     }
+    // bytes of the planes 0 .. 7 and 8 .. 15
+    uint32_t low[2], high[2];
 #pragma unroll
-    for (int b = 0; b < 16; ++b) reinterpret_cast<uint8_t *>(L.plane)[(b * 64 + l) * 4 + q] = (uint8_t)byte[b];
+    for (int e = 0; e < 2; ++e) {
+        low[e] = __builtin_amdgcn_perm(two[2 * e + 1], two[2 * e], 0x06040200u);
+        high[e] = __builtin_amdgcn_perm(two[2 * e + 1], two[2 * e], 0x07050301u);
+    }
+    transpose8(low[0], low[1]);
+    transpose8(high[0], high[1]);
+    uint8_t *const at = reinterpret_cast<uint8_t *>(L.plane) + l * 4 + q;
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+        at[b * 256] = (uint8_t)(low[b / 4] >> (8 * (b & 3)));
+        at[(b + 8) * 256] = (uint8_t)(high[b / 4] >> (8 * (b & 3)));
+    }
 }
 
 template <int NP>
@@ -222,7 +250,10 @@ __device__ void run_item(Lds &L, const SlicedJob &job, uint32_t row, uint32_t co
     // the xb of this wave: index bits 0 .. 3 are bits 3, 4, 2, 1 of xb, so that
     // the steps of a Gray code are one byte or half-word move; each with xb's
     // bit 0 off (a) and on (b)
-    const uint32_t per = 4 / job.parts, first = (part * 4 + wave) * per;
+    const uint32_t xparts = min(job.parts, 4u), per = 4 / xparts, first = (part % xparts * 4 + wave) * per;
+    // and of the 64 delta those whose upper bits are the rest of the part
+    const uint32_t dbits = job.parts == 16 ? 4 : job.parts == 8 ? 5 : 6, dhigh = (part / xparts) << dbits;
+    const uint32_t base = __popc(dhigh);
     if (first & 1) swap_planes<3>(a);
     if (first & 2) swap_planes<4>(a);
     if (first & 4) swap_planes<2>(a);
@@ -234,13 +265,14 @@ __device__ void run_item(Lds &L, const SlicedJob &job, uint32_t row, uint32_t co
         const uint32_t index = first ^ (j ^ (j >> 1));
         const uint32_t xbits = __popc(index);
         uint32_t delta = 0;
-        for (uint32_t pd = 0; pd <= 6; ++pd) {
+        for (uint32_t pd = 0; pd <= dbits; ++pd) {
             uint32_t acca[kProducts] = {}, accb[kProducts] = {};
-            const uint32_t last = 63u & ~((1u << (6 - pd)) - 1);  // the largest with pd bits
+            const uint32_t last = ((1u << dbits) - 1) & ~((1u << (dbits - pd)) - 1);  // the largest with pd bits
             delta = (1u << pd) - 1;
             uint32_t n = 0;
             for (;;) {
-                const uint4 *rec = reinterpret_cast<const uint4 *>(L.rec) + (l ^ delta);
+                const uint32_t from = l ^ (delta | dhigh);
+                const uint4 *rec = reinterpret_cast<const uint4 *>(L.rec) + from;
                 Planes<NP> r;
 #pragma unroll
                 for (int c = 0; c < Planes<NP>::NT; ++c) {
@@ -250,7 +282,7 @@ __device__ void run_item(Lds &L, const SlicedJob &job, uint32_t row, uint32_t co
                     r.p13[c] = y.z;
                     r.p123[c] = y.w;
                 }
-                r.t = Planes<NP>::one ? L.rec[(kRecord - 1) * 256 + (l ^ delta)] : 0;
+                r.t = Planes<NP>::one ? L.rec[(kRecord - 1) * 256 + from] : 0;
                 uint32_t q[5];
                 distances<NP>(a, r, q);
                 count_products<NP>(q, acca);
@@ -262,7 +294,7 @@ __device__ void run_item(Lds &L, const SlicedJob &job, uint32_t row, uint32_t co
                 const uint32_t c = delta & (0u - delta), up = delta + c;
                 delta = up | (((up ^ delta) >> 2) >> __builtin_ctz(c));
             }
-            uint32_t *at = L.count + (pd + xbits) * (kProducts * kCols) + (l & (kCols - 1));
+            uint32_t *at = L.count + (base + pd + xbits) * (kProducts * kCols) + (l & (kCols - 1));
 #pragma unroll
             for (int x = 0; x < kProducts; ++x) {
                 if (x == 0 ? NP != 16 : NP == 7 && x >= 8) continue;
@@ -271,8 +303,8 @@ __device__ void run_item(Lds &L, const SlicedJob &job, uint32_t row, uint32_t co
                                        __HIP_MEMORY_SCOPE_WORKGROUP);
             }
             if (l == 0) {
-                __hip_atomic_fetch_add(L.pairs + pd + xbits, n * 2048, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                __hip_atomic_fetch_add(L.pairs + pd + xbits + 1, n * 2048, __ATOMIC_RELAXED,
+                __hip_atomic_fetch_add(L.pairs + base + pd + xbits, n * 2048, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                __hip_atomic_fetch_add(L.pairs + base + pd + xbits + 1, n * 2048, __ATOMIC_RELAXED,
                                        __HIP_MEMORY_SCOPE_WORKGROUP);
             }
         }
@@ -444,10 +476,12 @@ void sliced_ranges(std::vector<SlicedJob> &jobs, int cus, uint64_t *total_items)
     uint64_t whole = 0;
     for (const SlicedJob &j : jobs) whole += blocks(j);
     // an item of a whole block keeps a workgroup busy for some 0.2 ms on a full
-    // CU: below 8 per resident workgroup the blocks are split in four (which
-    // costs the generation of the words four times, about 8 % more)
+    // CU: below 8 per resident workgroup the blocks are split in four by xb
+    // (which generates the words four times, 4 % more), and the smallest
+    // launches further by delta: 2^15 words 67 us with 4 or 16 parts and 61 with
+    // 8, 2^14 42 us with 4 and 34 with 16; 2^16 166 us with 8, 157 with 4
     const uint64_t resident = (uint64_t)std::max(sliced_per_cu(), 1u) * (uint64_t)cus;
-    const uint32_t parts = whole < 8 * resident ? 4 : 1;
+    const uint32_t parts = whole * 16 < resident ? 16 : whole * 4 < resident ? 8 : whole < 8 * resident ? 4 : 1;
     uint64_t at = 0;
     for (SlicedJob &j : jobs) {
         j.parts = parts;
