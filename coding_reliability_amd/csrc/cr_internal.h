@@ -179,11 +179,9 @@ struct RectLaunch {
     uint64_t ncols = 0;
     uint32_t mask32 = 0;             // truncate generated rows to 32 bits
     bool w2 = false;                 // some codeword exceeds 32 bits
-    unsigned long long *counter = nullptr;
-    unsigned long long *out = nullptr;
     uint32_t nbins = 0, first_bin = 0, lds_rows = 0;
 };
-cr_status launch_rect(const RectLaunch &L, hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1, int cus);
+cr_status launch_rect(const RectLaunch &L, const dev::DirectResult &out, hipStream_t stream, int cus);
 
 // The same histogram over rows A*i, i < 2^n, by recursion over the carries
 // (see carry_rows.hip).

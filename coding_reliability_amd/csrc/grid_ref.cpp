@@ -150,10 +150,6 @@ extern "C" cr_status cr_an_grid_ref(cr_context *ctx, int gdim, uint32_t n, uint6
             return fail(CR_ERR_DEVICE, "grid recursion: inconsistent total");
         return CR_OK;
     }
-    CR_TRY(ctx->hist.reserve(need * sizeof(uint64_t)));
-    CR_TRY(ctx->counters.reserve(sizeof(uint64_t)));
-    CR_TRY(fill_zero_u64(ctx->hist.as<unsigned long long>(), need, ctx->stream));
-
     RectLaunch L;
     L.A = g.A;
     L.row0 = 0;
@@ -163,23 +159,13 @@ extern "C" cr_status cr_an_grid_ref(cr_context *ctx, int gdim, uint32_t n, uint6
     L.ncols = cols.size();
     L.mask32 = t32 ? 1 : 0;
     L.w2 = need - 1 > 32;
-    L.counter = ctx->counters.as<unsigned long long>();
-    L.out = ctx->hist.as<unsigned long long>();
     L.nbins = need;
     L.first_bin = gdim == 2 ? 1 : 0;  // dancoding_grid_2d flushes bins 1.. (an_coding_grid.cu:138)
     L.lds_rows = need + 1;
-    CR_TRY(launch_rect(L, ctx->stream, kernel_ms ? ctx->ev0 : nullptr, kernel_ms ? ctx->ev1 : nullptr, ctx->cus));
-    CR_TRY(ctx->host.reserve(need * sizeof(uint64_t)));
-    CR_HIP(hipMemcpyAsync(ctx->host.ptr, L.out, need * sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
-    CR_HIP(hipStreamSynchronize(ctx->stream));
-    memset(hist, 0, nbins * sizeof(uint64_t));
-    memcpy(hist, ctx->host.ptr, need * sizeof(uint64_t));
-    if (kernel_ms) {
-        float ms = 0;
-        CR_HIP(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
-        *kernel_ms = ms;
-    }
-    return CR_OK;
+    dev::DirectResult out;
+    CR_TRY(direct_result(ctx, &out));
+    CR_TRY(launch_rect(L, out, ctx->stream, ctx->cus));
+    return direct_wait(ctx, hist, need, nbins, kernel_ms);
 }
 
 extern "C" cr_status cr_an_grid_report(int gdim, uint32_t n, uint64_t m1, uint64_t m2, const uint64_t *hist,

@@ -12,6 +12,7 @@
 // distance_distribution/src/an_coding_grid.cu:60-140): 1D = every code word
 // against the sample list, 2D = grid words against the sample list.
 #include <algorithm>
+#include <atomic>
 
 #include "cr_device.h"
 #include "cr_internal.h"
@@ -117,10 +118,12 @@ __global__ __launch_bounds__(64) void rect_kernel(uint64_t A, uint64_t row0, uin
                                                   const uint64_t *__restrict__ rows,
                                                   const uint64_t *__restrict__ cols, uint64_t ncols, uint32_t CW,
                                                   uint64_t CC, uint64_t G, uint64_t RBlocks, uint64_t total_items,
-                                                  unsigned long long *__restrict__ counter,
-                                                  unsigned long long *__restrict__ out, uint32_t nbins,
-                                                  uint32_t first_bin, uint32_t lds_rows, uint32_t mask32) {
+                                                  uint32_t nbins, uint32_t first_bin, uint32_t lds_rows,
+                                                  uint32_t mask32, uint32_t heads, const DirectResult direct) {
     extern __shared__ uint32_t lds[];
+    direct_start(direct);
+    unsigned long long *const counter = direct.queue;
+    unsigned long long *const out = hist_copy(direct.copies, nbins, kHistCopies);
     const uint32_t lane = threadIdx.x;
     lds_clear(lds, lds_rows);
     uint32_t *const lane_col = lds + lane;
@@ -130,7 +133,7 @@ __global__ __launch_bounds__(64) void rect_kernel(uint64_t A, uint64_t row0, uin
     uint64_t pending = 0;
     bool dirty = false;
 
-    for (uint64_t t = first_item(); t < total_items; t = following_item(counter, t)) {
+    for (uint64_t t = first_item(); t < total_items; t = following_item_of(counter, heads)) {
         // item = (group of G row blocks, column chunk)
         const uint64_t rbg = uniform64(t / CC), cc = uniform64(t - (t / CC) * CC);
         const uint64_t j0 = cc * CW;
@@ -163,6 +166,7 @@ __global__ __launch_bounds__(64) void rect_kernel(uint64_t A, uint64_t row0, uin
         }
     }
     if (dirty) flush_rows(lds, first_bin, nbins, out);
+    direct_finish(direct, nbins, lds);
 }
 
 template <int R, bool W2>
@@ -172,43 +176,49 @@ const void *rect_ptr() {
 
 }  // namespace
 
-cr_status launch_rect(const RectLaunch &L, hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1, int cus) {
+cr_status launch_rect(const RectLaunch &L, const DirectResult &out, hipStream_t stream, int cus) {
     constexpr int R = 8;
     const void *k = L.w2 ? rect_ptr<R, true>() : rect_ptr<R, false>();
     if (L.nrows == 0 || L.ncols == 0) return CR_OK;
     if (L.lds_rows < 2 || L.lds_rows > 66) return fail(CR_ERR_INVALID_ARGUMENT, "bad histogram rows %u", L.lds_rows);
     const uint64_t RB = 64ull * R;
     const uint64_t RBlocks = (L.nrows + RB - 1) / RB;
-    // column chunk: about 16 items per resident wave, at most 2^22 columns
+    // column chunk: about 16 items per resident wave, 16 to 2^22 columns
     const size_t lds = (size_t)L.lds_rows * dev::kStride * sizeof(uint32_t);
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, 64, lds) != hipSuccess || per_cu <= 0)
-        return fail(CR_ERR_DEVICE, "occupancy query failed for the rect kernel");
+    static std::atomic<int> cache[2][67];
+    int per_cu = cache[L.w2][L.lds_rows].load(std::memory_order_relaxed);
+    if (per_cu <= 0) {
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, 64, lds) != hipSuccess || per_cu <= 0)
+            return fail(CR_ERR_DEVICE, "occupancy query failed for the rect kernel");
+        cache[L.w2][L.lds_rows].store(per_cu, std::memory_order_relaxed);
+    }
     const uint64_t waves_cap = (uint64_t)per_cu * cus;
     const uint64_t target = 16 * waves_cap;
     uint64_t CC = (target + RBlocks - 1) / RBlocks;
     if (CC < 1) CC = 1;
     uint64_t CW = (L.ncols + CC - 1) / CC;
     if (CW > (1u << 22)) CW = 1u << 22;
-    if (CW < 1) CW = 1;
+    if (CW < 16) CW = 16;
     CC = (L.ncols + CW - 1) / CW;
     // many more row blocks than waves (every word against a short sample
     // list): G row blocks per item keep the items near the target count, so
-    // the work-queue counter (one atomic per item) stays off the critical path
+    // the work-queue counter (one atomic per item) stays off the critical path;
+    // items below 2^17 pairs share eight heads (a head serves one in 12.5 ns, the
+    // LDS of the device counts 2^17 pairs in 14).  Chunks of one column and one
+    // head took 165 us for 2^16 words of A = 4001 against 101 samples, now 13; 2^20
+    // words of A = 58659 against 1001 samples 0.80 -> 0.14 ms.
     const uint64_t G = RBlocks > target ? RBlocks / target : 1;
     const uint64_t items = (RBlocks + G - 1) / G * CC;
     uint32_t waves = (uint32_t)std::min<uint64_t>(waves_cap, items);
-    CR_TRY(fill_zero_u64(L.counter, 1, stream));
-    if (ev0) CR_HIP(hipEventRecord(ev0, stream));
     uint64_t a_A = L.A, a_row0 = L.row0, a_nrows = L.nrows, a_ncols = L.ncols, a_CC = CC, a_items = items, a_G = G,
              a_RB = RBlocks;
     const uint64_t *a_rows = L.rows, *a_cols = L.cols;
     uint32_t a_CW = (uint32_t)CW, a_nbins = L.nbins, a_first = L.first_bin, a_lr = L.lds_rows, a_m32 = L.mask32;
-    unsigned long long *a_counter = L.counter, *a_out = L.out;
+    uint32_t a_heads = G * CW * RB < (1u << 17) ? kQueues : 1;
+    DirectResult a_out = out;
     void *args[] = {&a_A, &a_row0, &a_nrows, (void *)&a_rows, (void *)&a_cols, &a_ncols, &a_CW, &a_CC, &a_G,
-                    &a_RB, &a_items, &a_counter, &a_out, &a_nbins, &a_first, &a_lr, &a_m32};
+                    &a_RB, &a_items, &a_nbins, &a_first, &a_lr, &a_m32, &a_heads, &a_out};
     CR_HIP(hipLaunchKernel(k, dim3(waves), dim3(64), args, lds, stream));
-    if (ev1) CR_HIP(hipEventRecord(ev1, stream));
     return CR_OK;
 }
 
