@@ -198,7 +198,7 @@ __global__ void fill_zero_kernel(unsigned long long *p, size_t n) {
 template <int R, bool WIDE>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WIDE ? 3 : 1))) void pair_kernel(const PairJob *__restrict__ jobs, uint32_t njobs,
                                                   uint64_t total_items, unsigned long long *__restrict__ counter,
-                                                  uint32_t lds_rows) {
+                                                  uint32_t heads, uint32_t lds_rows) {
     extern __shared__ uint32_t lds[];
     const uint32_t lane = threadIdx.x;
     lds_clear(lds, lds_rows);
@@ -209,7 +209,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WIDE ? 3 : 1
     uint32_t cur = 0xFFFFFFFFu;  // job whose counts sit in LDS
     uint64_t pending = 0;        // columns accumulated since the last flush
 
-    for (uint64_t t = first_item(); t < total_items; t = following_item(counter, t)) {
+    for (uint64_t t = first_item(); t < total_items;
+         t = counter ? following_item_of(counter, heads) : t + gridDim.x) {
         // job lookup: current job first, else binary search over item_begin
         uint32_t jb;
         if (cur != 0xFFFFFFFFu && t >= jobs[cur].item_begin && t < jobs[cur].item_begin + jobs[cur].items) {
@@ -370,13 +371,15 @@ cr_status launch_pairs(const PairJob *d_jobs, uint32_t njobs, uint64_t total_ite
         const uint64_t per = (total_items + waves - 1) / waves;
         waves = (uint32_t)((total_items + per - 1) / per);
     }
-    if (cfg.zero_counter && counter) CR_TRY(fill_zero_u64(counter, 1, stream));
+    if (cfg.zero_counter && counter)
+        CR_TRY(fill_zero_u64(counter, cfg.heads > 1 ? kQueues * kQueuePitch : 1, stream));
     if (ev0) CR_HIP(hipEventRecord(ev0, stream));
     const PairJob *a_jobs = d_jobs;
-    uint32_t a_njobs = njobs, a_rows = cfg.lds_rows;
+    uint32_t a_njobs = njobs, a_heads = cfg.heads, a_rows = cfg.lds_rows;
     uint64_t a_items = total_items;
     unsigned long long *a_counter = counter;
-    void *args[] = {(void *)&a_jobs, (void *)&a_njobs, (void *)&a_items, (void *)&a_counter, (void *)&a_rows};
+    void *args[] = {(void *)&a_jobs, (void *)&a_njobs, (void *)&a_items, (void *)&a_counter, (void *)&a_heads,
+                    (void *)&a_rows};
     CR_HIP(hipLaunchKernel(k, dim3(waves), dim3(64), args, lds, stream));
     if (ev1) CR_HIP(hipEventRecord(ev1, stream));
     return CR_OK;

@@ -6,6 +6,7 @@
 #include <numeric>
 #include <vector>
 
+#include "cr_device.h"
 #include "cr_internal.h"
 
 namespace cr {
@@ -38,10 +39,9 @@ static_assert(alignof(PairJob) == alignof(SlicedJob) && sizeof(SlicedJob) % alig
 cr_status build_batch(cr_context *ctx, const cr_an_code *codes, uint32_t ncodes, uint32_t stride,
                       const cr_pair_tuning *tuning, unsigned long long *d_hist, BatchLayout &L) {
     if (!codes || ncodes == 0) return fail(CR_ERR_INVALID_ARGUMENT, "empty batch");
-    uint32_t R = tuning && tuning->rows_per_lane ? tuning->rows_per_lane : 8;
     const uint32_t ipw = tuning && tuning->items_per_wave ? tuning->items_per_wave : 16;
     uint32_t max_need = 0;
-    long double total_pairs = 0;
+    long double total_pairs = 0, short_pairs = 0;
     L.jobs.reserve(ncodes);
     for (uint32_t c = 0; c < ncodes; ++c) {
         const uint64_t A = codes[c].A, N = codes[c].num_words;
@@ -65,7 +65,12 @@ cr_status build_batch(cr_context *ctx, const cr_an_code *codes, uint32_t ncodes,
         L.jobs.push_back(j);
         max_need = std::max(max_need, need);
         total_pairs += (long double)N * (long double)(N - 1) / 2;
+        if (N < (1ull << 15)) short_pairs += (long double)N * (long double)(N - 1) / 2;
     }
+    // as for single codes: short codes waste less of a row block of 128 words
+    // than of one of 512 (16384 codes of 2^8 words 0.48 ms with 8 rows a lane, 0.20
+    // with 2; 4096 codes of 2^10 words 0.64 and 0.46)
+    const uint32_t R = tuning && tuning->rows_per_lane ? tuning->rows_per_lane : 2 * short_pairs >= total_pairs ? 2 : 8;
     L.cfg.R = R;
     L.cfg.lds_rows = std::max(max_need, 1u) + 1;
     L.cfg.waves = tuning ? tuning->waves : 0;
@@ -93,18 +98,23 @@ cr_status build_batch(cr_context *ctx, const cr_an_code *codes, uint32_t ncodes,
         total += j.items;
     }
     L.total_items = total;
+    // a head hands out an item in 12.5 ns, in which the device counts 2^17
+    // pairs: 16384 codes of 2^4 words 0.22 -> 0.06 ms with eight heads
+    L.cfg.heads = total_pairs < (long double)total * (1 << 17) ? dev::kQueues : 1;
     std::stable_sort(L.sliced.begin(), L.sliced.end(),
                      [](const SlicedJob &a, const SlicedJob &b) { return a.k > b.k; });
     sliced_ranges(L.sliced, ctx->cus, &L.sliced_items);
     return CR_OK;
 }
 
-// Both launches; counters: two work-queue heads.
+// Both launches; counters: the pair kernel's work-queue heads, then the sliced one's.
+constexpr size_t kCounters = dev::kQueues * dev::kQueuePitch + 1;
 cr_status launch_batch(cr_context *ctx, const BatchLayout &L, void *d_jobs, unsigned long long *counters) {
     const SlicedJob *sliced = static_cast<const SlicedJob *>(d_jobs);
     if (!L.sliced.empty()) {
-        CR_TRY(fill_zero_u64(counters + 1, 1, ctx->stream));
-        CR_TRY(launch_sliced(sliced, (uint32_t)L.sliced.size(), L.sliced_items, counters + 1, ctx->cus, ctx->stream));
+        unsigned long long *const head = counters + kCounters - 1;
+        CR_TRY(fill_zero_u64(head, 1, ctx->stream));
+        CR_TRY(launch_sliced(sliced, (uint32_t)L.sliced.size(), L.sliced_items, head, ctx->cus, ctx->stream));
     }
     if (!L.jobs.empty())
         CR_TRY(launch_pairs(reinterpret_cast<const PairJob *>(sliced + L.sliced.size()), (uint32_t)L.jobs.size(),
@@ -139,7 +149,7 @@ cr_status cr_an_batch(cr_context *ctx, const cr_an_code *codes, uint32_t ncodes,
     BatchLayout L;
     CR_TRY(build_batch(ctx, codes, ncodes, stride, tuning, ctx->hist.as<unsigned long long>(), L));
     CR_TRY(ctx->jobs.reserve(L.job_bytes()));
-    CR_TRY(ctx->counters.reserve(2 * sizeof(uint64_t)));
+    CR_TRY(ctx->counters.reserve(kCounters * sizeof(uint64_t)));
     CR_TRY(fill_zero_u64(ctx->hist.as<unsigned long long>(), n, ctx->stream));
     CR_HIP(L.upload(ctx->jobs.ptr, ctx->stream));
     if (kernel_ms) CR_HIP(hipEventRecord(ctx->ev0, ctx->stream));
@@ -187,7 +197,7 @@ cr_status cr_batch_plan_create(cr_context *ctx, const cr_an_code *codes, uint32_
     const size_t n = (size_t)ncodes * stride;
     cr_status s;
     if ((s = p->hist.reserve(n * sizeof(uint64_t))) != CR_OK) return bail(s);
-    if ((s = p->counter.reserve(2 * sizeof(uint64_t))) != CR_OK) return bail(s);
+    if ((s = p->counter.reserve(kCounters * sizeof(uint64_t))) != CR_OK) return bail(s);
     if ((s = p->host.reserve(n * sizeof(uint64_t))) != CR_OK) return bail(s);
     BatchLayout L;
     if ((s = build_batch(ctx, codes, ncodes, stride, tuning, p->hist.as<unsigned long long>(), L)) != CR_OK)

@@ -117,6 +117,7 @@ struct PairLaunchConfig {
     uint32_t waves = 0;         // 0 = resident capacity of the device
     uint32_t lds_rows = 0;      // histogram rows in LDS (max nbins + 1 dummy row)
     bool wide = false;          // some job has kModeWide
+    uint32_t heads = 1;         // work-queue heads (dev::kQueues of them dev::kQueuePitch apart)
     bool zero_counter = true;   // false: the caller cleared the queue head already
     bool allow_static = false;  // a short launch: static assignment of items to waves, no queue
 };
