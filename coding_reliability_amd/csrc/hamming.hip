@@ -33,15 +33,17 @@ using namespace dev;
 // GF(2), so it is the XOR of the syndromes of the data word's bytes; table f
 // holds the syndromes of byte f's 256 values, one byte each: 4 tables for 32-bit
 // data, 8 for 64-bit.  A 256-byte table has two dwords in every LDS bank, so
-// some lookups take two passes, where five 7-bit fields a half word would
-// not; but the kernel is bound by VALU issue, and four lookups take one
-// extraction less (LDS stays at about 0.65 of its rate).  Measured with the XORs
-// three operands at a time: (39,32) Monte Carlo of 2^34 words 10.6 -> 9.0 ms,
-// (72,64) of 2^30 1.40 -> 1.31 ms, a (39,32) stride grid of 2^30 0.50 -> 0.43 ms.
-constexpr uint32_t kFields = 4;  // bytes per 32-bit half
+// most lookups take two passes (the LDS is then busy nearly as long as the
+// VALU), where five 7-bit fields a half word would take one; but those need
+// more instructions and registers.  (39,32) Monte Carlo of 2^34 words with
+// fields of 8 / 7 / 6 bits: 9.0 / 9.8 / 11.2 ms, (72,64) of 2^30 1.24 / 1.39 /
+// 1.47 ms, a (39,32) stride grid of 2^30 0.43 / 0.46 / 0.47 ms.  With 7 bits,
+// two-operand XORs and scalar Philox keys: 10.6, 1.40 and 0.50 ms.
+constexpr uint32_t kBits = 8, kFields = 4;  // of a field; fields per 32-bit half
+constexpr uint32_t kTable = 1u << kBits;
 
 template <bool W64>
-constexpr uint32_t kTabBytes = (W64 ? 2 : 1) * kFields * 256;
+constexpr uint32_t kTabBytes = (W64 ? 2 : 1) * kFields * kTable;
 
 template <bool W64>
 __device__ void build_tables(uint8_t *tab, const uint64_t *masks) {
@@ -49,7 +51,8 @@ __device__ void build_tables(uint8_t *tab, const uint64_t *masks) {
 #pragma unroll
     for (int t = 0; t < 7; ++t) m[t] = masks[t];
     for (uint32_t e = threadIdx.x; e < kTabBytes<W64>; e += 64) {
-        const uint64_t x = (uint64_t)(e & 255) << (8 * (e >> 8));
+        const uint32_t f = e / kTable;
+        const uint64_t x = (uint64_t)(e % kTable) << (32 * (f / kFields) + kBits * (f % kFields));
         uint32_t syn = 0;
 #pragma unroll
         for (int t = 0; t < 7; ++t) syn |= (uint32_t)(__popcll(x & m[t]) & 1) << t;
@@ -70,7 +73,7 @@ __device__ __forceinline__ void table_reads(const uint64_t (&d)[U], const uint8_
 #pragma unroll
         for (uint32_t f = 0; f < (W64 ? 2 : 1) * kFields; ++f) {
             const uint32_t x = (uint32_t)(d[u] >> (32 * (f / kFields)));
-            r[u][f] = tab[256 * f + ((x >> (8 * (f % kFields))) & 255)];
+            r[u][f] = tab[kTable * f + ((x >> (kBits * (f % kFields))) & (kTable - 1))];
         }
 }
 
@@ -80,12 +83,11 @@ __device__ __forceinline__ void table_weights(const uint64_t (&d)[U], uint64_t d
                                               const uint32_t (&r)[U][(W64 ? 2 : 1) * kFields], uint32_t (&w)[U]) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-        uint32_t syn = r[u][kFields - 1];
-        if (W64) {
-            syn = __builtin_amdgcn_bitop3_b32(syn, r[u][2 * kFields - 1], r[u][2 * kFields - 2], 0x96);
-            syn = __builtin_amdgcn_bitop3_b32(syn, r[u][kFields], r[u][kFields + 1], 0x96);
-        }
-        syn = __builtin_amdgcn_bitop3_b32(syn, r[u][0], r[u][1], 0x96) ^ r[u][2];
+        constexpr uint32_t F = (W64 ? 2 : 1) * kFields;
+        uint32_t syn = r[u][0];
+#pragma unroll
+        for (uint32_t f = 1; f + 1 < F; f += 2) syn = __builtin_amdgcn_bitop3_b32(syn, r[u][f], r[u][f + 1], 0x96);
+        if (F % 2 == 0) syn ^= r[u][F - 1];
         const uint64_t dm = FULL ? d[u] : d[u] & dmask;
         w[u] = __popc(syn) + (W64 ? (uint32_t)__popcll(dm) : (uint32_t)__popc((uint32_t)dm));
     }
