@@ -89,7 +89,7 @@ def cpu_baseline(A: int, k: int, target_s: float) -> dict:
     _, pairs = O.an_cpu_counts(k, A, 0, shards)
     dt = time.perf_counter() - t0
     # the CPU Hamming loop (hamming.cpp:43-63) on the (39,32) code: all 2^32
-    # data words, the exhaustive run the GPU does in half a millisecond
+    # data words, the run the GPU answers from the code's structure
     hw = 1 << 32
     t0 = time.perf_counter()
     hh = O.hamming_weights(32, 0, hw)
@@ -155,20 +155,16 @@ def run_batched(ctx, ceil: dict | None = None, autotune: bool = True) -> dict:
         "speedup_graph_vs_per_launch": round(t_per / t_graph, 3),
         "tuning": tune, "bit_exact": True,
     }
-    # the bound batching can reach on this mix: its codes with k >= 17 hold
-    # most of the pairs and each fills the device alone, so a batched launch
-    # can at best run every pair at the LDS-increment ceiling; what batching
-    # removes is the per-code launch and synchronisation time
+    # codes of 2^11 words and more run in the sliced kernel, the others at best
+    # at the LDS-increment ceiling: what one increment per pair would take
     big = WL.pairs_of([(A, N) for A, N in codes if N >= 1 << 17])
     if ceil:
-        t_floor = pairs / ceil["lds"]
         out["codes4096"].update({
             "share_of_pairs_k17_18": round(big / pairs, 4),
-            "batched_floor_s": round(t_floor, 4),
-            "speedup_bound": round(t_per / t_floor, 3),
-            "bound_note": "batched_floor_s = pairs / the run's LDS-increment ceiling (one increment per pair); the "
-                          "per-launch run is already within per_launch_s - batched_floor_s of it, so no batching "
-                          "of this mix can exceed speedup_bound",
+            "lds_increment_s": round(pairs / ceil["lds"], 4),
+            "lds_increment_note": "pairs / the run's LDS-increment ceiling: the pair kernel's floor, which the sliced "
+                                  "kernel (32 pairs an instruction) is not bound by; the per-launch side runs the "
+                                  "pair kernel",
         })
     # the reference's published per-launch sweep: super-A k=8, 16384 codes
     sweep = WL.supera_codes(8, 16)
@@ -197,26 +193,25 @@ def run_batched(ctx, ceil: dict | None = None, autotune: bool = True) -> dict:
 
 # kernel executes `valu` VALU instructions -- the SQ_INSTS_VALU counts of its
 # profile under profiles/, divided by the units of the launch --, `lds`
-# histogram increments (wave-wide ds_add_u32 lanes) and `reads` syndrome-table
-# lookups (ds_read_u8 lanes).  frac_valu is the VALU issue utilisation
+# histogram increments (wave-wide ds_add_u32 lanes) and `reads` passes of
+# syndrome-table lookups (ds_read_u8 lanes; two passes a lookup where random
+# words meet two dwords in a bank).  frac_valu is the VALU issue utilisation
 # (executed instructions/s over the ceiling), frac_lds the share of time the
 # LDS is busy (increments over the increment ceiling plus lookups over the
 # table-read ceiling); frac is the larger (the two pipelines run
 # concurrently), named by "bound".  `ops` is the algorithmic int32 work per
-# unit for reference: xor + popcount + increment per enumerated word or pair
-# (2W+1 with the high dword folded), per sampled 32-bit word 5 field lookups
-# + 4 xors + 2 popcounts + 1 increment (10 + 9 + 3 + 1 for 64-bit), 40 per
+# unit for reference: xor + popcount + increment per pair
+# (2W+1 with the high dword folded), per sampled 32-bit word 4 field lookups
+# + 3 xors + 2 popcounts + 1 increment (8 + 7 + 3 + 1 for 64-bit), 40 per
 # Philox block (10 per 32-bit Monte Carlo word, 20 per 64-bit), 9 per
 # ANcandidates step.
 KERNEL_WORK = {
     # name: (executed VALU per unit, LDS increments per unit, LDS table reads per unit,
     #        algorithmic ops per unit, profile)
-    "hamming_exhaustive_39_32": (3.07, 1, 0, 3, "profiles/ham_kernel_39_32_exhaustive_grid_mc_and_72_64_mc.md"),
-    "hamming_grid_39_32": (None, 1, 5, 12, "latency-bound launch"),
-    "hamming_mc_39_32": (21.92, 1, 5, 22, "profiles/ham_kernel_39_32_exhaustive_grid_mc_and_72_64_mc.md"),
-    "hamming_mc_72_64": (42.47, 1, 10, 43, "profiles/ham_kernel_39_32_exhaustive_grid_mc_and_72_64_mc.md"),
-    "an_grid1d_ref": (3.01, 1, 0, 3, "profiles/rect_kernel_grid1d_A61_k32_m1001.md"),
-    "an_mc": (16.02, 1, 0, 14, "profiles/an_mc_kernel_A61_k24_m65536.md"),
+    "hamming_grid_39_32": (None, 1, 4, 10, "latency-bound launch"),
+    "hamming_mc_39_32": (19.97, 1, 8, 20, "profiles/ham_kernel_mc_39_32_and_72_64.md"),
+    "hamming_mc_72_64": (39.0, 1, 16, 39, "profiles/ham_kernel_mc_39_32_and_72_64.md"),
+    "an_mc": (13.55, 1, 0, 14, "profiles/an_mc_kernel_A61_k24.md"),
     "an_candidates": (None, 0, 0, 9, "lower bound: algorithmic steps of the maximising A"),
 }
 
@@ -235,12 +230,21 @@ def _kernel_entry(name: str, units: float, ms: float, unit: str, ceil: dict, wor
             "frac": round(max(f_valu, f_lds), 4)}
 
 
+def _recursion_entry(units: float, ms: float, unit: str, workload: str) -> dict:
+    """A histogram that comes from the code's structure, not unit by unit:
+    the words or pairs it covers per second, with no roofline of theirs."""
+    return {"workload": workload, "kernel_ms": round(ms, 4), "equivalent_rate": round(units / (ms / 1e3) / 1e9, 3),
+            "rate_unit": unit, "bound": "latency of the recursion's levels", "frac": None}
+
+
 def _ceilings_json(ceil: dict) -> dict:
     return {"valu": round(ceil["valu"] / 1e12, 4), "lds": round(ceil["lds"] / 1e12, 4),
             "lds_read": round(ceil["lds_read"] / 1e12, 4),
             "write": round(ceil["write"] / 1e12, 4), "read": round(ceil["read"] / 1e12, 4),
             "unit": "T/s: VALU lane-instructions, LDS lane increments, LDS lane-reads from 128-byte tables, TB/s "
-                    "streaming stores and loads over 256 MiB (cr_probe_ceiling, this run)",
+                    "streaming stores and loads over 256 MiB (cr_probe_ceiling, this run); the VALU probes' "
+                    "instructions take a scalar operand or count bits: XORs, ANDs and bitop3 of vector registers "
+                    "alone issue at up to 1.5 times that, so a kernel of those can exceed it",
             "probes": {kk: round(v / 1e12, 4) for kk, v in ceil["probes"].items()}}
 
 
@@ -281,8 +285,8 @@ def run_kernels(ctx, ceil: dict) -> dict:
     k = 32
     h, ms = _warm(lambda: ctx.hamming_weights(k, cra.HAM_RANGE, 0, 1 << k))
     assert sum(h) == 1 << k
-    out["hamming_exhaustive_39_32"] = _kernel_entry("hamming_exhaustive_39_32", 1 << k, ms, "Gwords/s", ceil,
-                                                    "(39,32) weights of all 2^32 data words")
+    out["hamming_exhaustive_39_32"] = _recursion_entry(1 << k, ms, "Gwords/s",
+                                                       "(39,32) weights of all 2^32 data words")
     h_grid, ms = _warm(lambda: ctx.hamming_weights(k, cra.HAM_STRIDE, 0, 1 << 20, stride=65537))
     assert sum(h_grid) == 1 << 20
     e = _kernel_entry("hamming_grid_39_32", 1 << 20, ms, "Gwords/s", ceil,
@@ -320,8 +324,8 @@ def run_kernels(ctx, ceil: dict) -> dict:
     out["hamming_mc_72_64"] = _kernel_entry("hamming_mc_72_64", S, ms, "Gwords/s", ceil, "(72,64) 2^30 Philox words")
     h, ms = _warm(lambda: ctx.an_grid_ref(1, 32, 1001, 0, 61))
     pairs = sum(h)
-    out["an_grid1d_ref"] = _kernel_entry("an_grid1d_ref", pairs, ms, "Gpairs/s", ceil,
-                                         f"reference grid 1D, A=61, k=32, m=1001 (38-bit codewords, {pairs} pairs)")
+    out["an_grid1d_ref"] = _recursion_entry(pairs, ms, "Gpairs/s", "reference grid 1D, A=61, k=32, m=1001 "
+                                            f"(38-bit codewords, {pairs} pairs)")
     m = 1 << 16
     h, ms = _warm(lambda: ctx.an_mc(61, 24, m, 16384))
     assert sum(h) == (1 << 24) * m
@@ -354,13 +358,18 @@ REFERENCE_RECORDED = {
 
 def run_spectral(ctx, A: int, k: int, raw_pairs: list, pair_kernel_s: float, ceil: dict | None = None) -> dict:
     """The headline histogram again, from the code's Walsh-Hadamard spectrum
-    (cr_an_pairs_spectral, the path cr_an_pairs takes for this code): one
-    untimed call, one timed call, checked equal to the pair kernel's."""
+    (cr_an_pairs_spectral): one untimed call, one timed call, checked equal to
+    the pair kernel's; and by the method cr_an_pairs picks for this code."""
     ctx.an_pairs_spectral(A, k)
     t0 = time.perf_counter()
     raw, ms = ctx.an_pairs_spectral(A, k)
     dt = time.perf_counter() - t0
     assert raw == raw_pairs, "spectral histogram differs from the pair kernel's"
+    ctx.an_pairs_auto(A, 1 << k)
+    t0 = time.perf_counter()
+    raw, _ = ctx.an_pairs_auto(A, 1 << k)
+    dt_auto = time.perf_counter() - t0
+    assert raw == raw_pairs, "cr_an_pairs' histogram differs from the pair kernel's"
     N = 1 << k
     Ao = A // (A & -A)  # odd part: the same distances
     n = max((Ao * (N - 1)).bit_length(), k)
@@ -388,6 +397,8 @@ def run_spectral(ctx, A: int, k: int, raw_pairs: list, pair_kernel_s: float, cei
         "device_seconds": round(ms / 1e3, 4),
         "equivalent_gpairs_per_s": round(N * (N - 1) / 2 / dt / 1e9, 1),
         "speedup_vs_pair_kernel": round(pair_kernel_s / dt, 2),
+        "cr_an_pairs_seconds": round(dt_auto, 5),
+        "cr_an_pairs_speedup_vs_pair_kernel": round(pair_kernel_s / dt_auto, 1),
         "transforms": 1 << (n - k),
         "transform_length": N,
         "memory_roofline": memory,
@@ -403,7 +414,7 @@ def run_vs_reference(ctx) -> dict:
 
     def entry(key, secs, extra=None, out_key=None):
         ref, src = REFERENCE_RECORDED[key]
-        e = {"seconds": round(secs, 4), "reference_seconds": ref, "reference_source": src,
+        e = {"seconds": round(secs, 6), "reference_seconds": ref, "reference_source": src,
              "speedup_vs_reference": round(ref / secs, 1)}
         e.update(extra or {})
         out[out_key or key] = e
@@ -414,19 +425,19 @@ def run_vs_reference(ctx) -> dict:
         raw, ms = ctx.an_pairs(A, N)
         assert sum(raw) == N * (N - 1) // 2
         entry(key, ms / 1e3, {"gpairs_per_s": round(N * (N - 1) / 2 / (ms / 1e3) / 1e9, 1), "method": "pair kernel"})
-        # the same histogram from the code's spectrum (what cr_an_pairs picks)
-        ctx.an_pairs_spectral(A, 24)
+        # the same histogram by the method cr_an_pairs picks
+        ctx.an_pairs_auto(A, N)
         t0 = time.perf_counter()
-        raw_s, ms_s = ctx.an_pairs_spectral(A, 24)
+        raw_s, ms_s = ctx.an_pairs_auto(A, N)
         dt = time.perf_counter() - t0
         assert raw_s == raw
-        entry(key, dt, {"device_seconds": round(ms_s / 1e3, 4),
-                        "method": "Walsh-Hadamard spectrum (cr_an_pairs_spectral), bit-exact against the pair kernel"},
-              out_key=key + "_spectral")
-    # the exact k = 32 distribution the grid above approximates (spectral path)
-    ctx.an_pairs_spectral(3, 32)
+        entry(key, dt, {"device_seconds": round(ms_s / 1e3, 6),
+                        "method": "recursion over carries (cr_an_pairs), bit-exact against the pair kernel"},
+              out_key=key + "_auto")
+    # the exact k = 32 distribution the grid above approximates
+    ctx.an_pairs_auto(61, 1 << 32)
     t0 = time.perf_counter()
-    raw32, ms32 = ctx.an_pairs_spectral(61, 32)
+    raw32, ms32 = ctx.an_pairs_auto(61, 1 << 32)
     dt = time.perf_counter() - t0
     exact = [1 << 32] + [2 * x for x in raw32[1:]]
     assert sum(exact) == 1 << 64
@@ -437,8 +448,8 @@ def run_vs_reference(ctx) -> dict:
         g = [r for r in grids if r["n"] == 32 and r["A"] == 61 and r["m"] == m][0]["counts"]
         errs[f"recorded_grid_m{m}_max_rel_error"] = round(max(abs(g[d] / exact[d] - 1) for d in range(1, 38)
                                                               if exact[d] > 0), 6)
-    entry("grid1d_A61_k32_m1001", dt, dict(errs, device_seconds=round(ms32 / 1e3, 4),
-                                           method="exact distribution (spectral path, 64 transforms of 2^32) "
+    entry("grid1d_A61_k32_m1001", dt, dict(errs, device_seconds=round(ms32 / 1e3, 6),
+                                           method="exact distribution (cr_an_pairs, recursion over carries) "
                                                   "against the reference's m=1001 grid approximation"),
           out_key="exact_A61_k32")
     for k, m, key in ((32, 1001, "grid1d_A61_k32_m1001"), (40, 101, "grid1d_A61_k40_m101")):
@@ -732,7 +743,7 @@ def main() -> int:
         log("other kernels ...")
         kernels = run_kernels(ctx, ceil)
         for name, e in kernels.items():
-            log(f"{name}: {e['rate']} {e['rate_unit']}, frac {e['frac']}")
+            log(f"{name}: {e.get('rate', e.get('equivalent_rate'))} {e['rate_unit']}, frac {e['frac']}")
 
     served = None
     if not args.no_served:

@@ -45,8 +45,8 @@ def hamming_report(k: int, weights: list[int], with_1bit: bool) -> list[int]:
 def hamming_sdc_table(k: int, method: int = 2, ctx: "Context | None" = None) -> tuple[str, list[int]]:
     """SDC table text of the (N,k) Extended Hamming code in the legacy table
     layout (legacy/hamming_count_undetectable_errors.cpp:226-339) and the
-    non-extended weight distribution it was built from.  method 1 enumerates
-    all 2^k words on the device (k <= 40, needs ctx), 2 uses the MacWilliams
+    non-extended weight distribution it was built from.  method 1 takes the
+    weights of all 2^k words from the device (k <= 40, needs ctx), 2 uses the MacWilliams
     identity, 0 picks."""
     N = hamming_N(k)
     w = np.zeros(2 * (N + 1), dtype=np.uint64)
@@ -166,7 +166,7 @@ class Context:
 
     def an_pairs_auto(self, A: int, num_words: int, nbins: int | None = None) -> tuple[list[int], float]:
         """The same histogram as an_pairs through cr_an_pairs, which picks the
-        spectral path for 2^16 / 2^24 words when it is estimated cheaper."""
+        method it estimates to be the fastest."""
         if nbins is None:
             nbins = an_bins(A, num_words)
         out = (C.c_uint64 * nbins)()

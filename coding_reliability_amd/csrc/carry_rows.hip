@@ -17,7 +17,7 @@
 // distances at a time: distance d reads only d and d - 1.  Up to 64 carries a
 // sample takes one wave, without barriers, and a workgroup four samples.  Bound
 // by LDS, two reads and a write per counter, and for few samples by the chain
-// of n levels.  Measured: a call with a 6-bit A, n = 32 and 1001 samples 58 us,
+// of n levels.  Measured: a call with a 6-bit A, n = 32 and 1001 samples 43 us,
 // against 449 ms in the rectangle kernel (4.3e12 pairs at one LDS increment
 // each).
 #include <algorithm>

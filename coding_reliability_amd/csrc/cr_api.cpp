@@ -27,8 +27,10 @@ cr_status DeviceBuffer::reserve(size_t want) {
     size_t n = std::max(want, (size_t)256);
     void *p = nullptr;
     hipError_t e = hipMalloc(&p, n);
-    if (e != hipSuccess)
+    if (e != hipSuccess) {
+        (void)hipGetLastError();  // or the next launch reports it
         return fail(CR_ERR_OUT_OF_MEMORY, "hipMalloc(%zu) failed: %s", n, hipGetErrorString(e));
+    }
     ptr = p;
     bytes = n;
     return CR_OK;
@@ -421,8 +423,15 @@ cr_status cr_an_pairs(cr_context *ctx, uint64_t A, uint64_t num_words, uint64_t 
     const bool recursion = carry_preferred(A, num_words, best, &carry);
     if (recursion) best = carry.seconds;
     CarryTilesPlan tiles;
-    if (tiles_preferred(A, num_words, best, &tiles)) return an_pairs_tiles(ctx, tiles, A, raw, nbins, kernel_ms);
-    if (recursion) return an_pairs_carry(ctx, carry, A, raw, nbins, kernel_ms);
+    // without memory for a recursion's tables (up to 4 GiB) the next method
+    if (tiles_preferred(A, num_words, best, &tiles)) {
+        const cr_status s = an_pairs_tiles(ctx, tiles, A, raw, nbins, kernel_ms);
+        if (s != CR_ERR_OUT_OF_MEMORY) return s;
+    }
+    if (recursion) {
+        const cr_status s = an_pairs_carry(ctx, carry, A, raw, nbins, kernel_ms);
+        if (s != CR_ERR_OUT_OF_MEMORY) return s;
+    }
     if (spectral && spectral_s < pairwise) return cr_an_pairs_spectral(ctx, A, k, raw, nbins, kernel_ms);
     if (by_planes) return an_pairs_sliced(ctx, sliced, A, num_words, raw, nbins, kernel_ms);
     if (is_short) return an_pairs_short(ctx, A, num_words, raw, nbins, kernel_ms);

@@ -70,8 +70,7 @@ cr_status cr_device_memory(cr_context *ctx, uint64_t *free_bytes, uint64_t *tota
  * probe kernel on every resident single-wave workgroup for `iters` loop
  * iterations and returns the rate it sustained:
  *   probe 0, 4: VALU lane-instructions/s of xor + popcount-accumulate on 8 or
- *               16 independent chains (the pair, grid and exhaustive Hamming
- *               inner loops);
+ *               16 independent chains (the pair and grid inner loops);
  *   probe 1:    VALU lane-instructions/s of Philox4x32-10 (the Monte Carlo
  *               generator: 20 64-bit multiplies and 20 three-input xors per
  *               block);
@@ -84,7 +83,8 @@ cr_status cr_device_memory(cr_context *ctx, uint64_t *free_bytes, uint64_t *tota
  *               passes (at most 64) over a 256 MiB buffer, the size of the
  *               spectral path's batches;
  *   probe 8:    lane-reads/s of ds_read_u8 from 128-byte LDS tables (one
- *               dword per bank), the Hamming kernels' syndrome lookups.
+ *               dword per bank), one pass of the Hamming kernel's syndrome
+ *               lookups.
  * kernel_ms (may be NULL) receives the probe's device time. */
 cr_status cr_probe_ceiling(cr_context *ctx, uint32_t probe, uint32_t iters, double *units_per_s, double *kernel_ms);
 
@@ -97,11 +97,15 @@ cr_status cr_probe_ceiling(cr_context *ctx, uint32_t probe, uint32_t iters, doub
  * (distance_distribution/src/an_coding.cu:50-105) before run_ancoding doubles it
  * (an_coding.cu:287-292).  With A = A0*s and num_words = m it is the
  * integer-stride grid {A0*(i*s) : i < m}.
- * For num_words = 2^k, 14 <= k <= 32, the same histogram is computed from the code's
- * Walsh-Hadamard spectrum (cr_an_pairs_spectral) when that is estimated at
- * under 80 % of the pair kernel's time (multipliers well below 2^k);
- * cr_an_pairs_tuned always runs the pair kernel.
- * kernel_ms (may be NULL) receives the device time of the launches. */
+ * The method is the one estimated to be the fastest, all exact: short codes
+ * (up to 2^13 words) in one launch; for num_words = 2^k a bit-sliced kernel (up
+ * to 2^24 words of multipliers up to 16 bits), recursions over the carries of
+ * the product (odd part of A below 4096 and k <= 32, or below 65536 and k <=
+ * 26) and the Walsh-Hadamard spectrum (cr_an_pairs_spectral); otherwise the
+ * pair kernel, which cr_an_pairs_tuned always runs.  The recursions take device
+ * tables of up to 2 GiB each, kept by the context up to 1 GiB.
+ * kernel_ms (may be NULL) receives the device time of the launches (of calls
+ * of one launch and of the recursions by the device's constant-rate clock). */
 cr_status cr_an_pairs(cr_context *ctx, uint64_t A, uint64_t num_words, uint64_t *raw, uint32_t nbins,
                       double *kernel_ms);
 
@@ -211,9 +215,9 @@ cr_status cr_hamming_weights(cr_context *ctx, const cr_ham_request *req, uint64_
 
 /* n requests (1..4096) in one call: hists[i * nbins + w] is request i's
  * histogram, equal to cr_hamming_weights of that request; nbins must exceed
- * every request's largest weight.  The requests of k <= 32 run as the jobs of
- * one kernel launch, those of k > 32 as the jobs of a second; kernel_ms spans
- * both.  No counterpart in the reference: it puts small requests (the (39,32)
+ * every request's largest weight.  Ranges run as the workgroups of one kernel
+ * launch, the other requests of k <= 32 as the jobs of another, those of k > 32 as
+ * the jobs of a third; kernel_ms spans them.  No counterpart in the reference: it puts small requests (the (39,32)
  * stride grid of 2^20 words, a few microseconds of work) into the launch of a
  * larger one (its 2^34-word Monte Carlo run) instead of paying a launch each. */
 cr_status cr_hamming_weights_batch(cr_context *ctx, const cr_ham_request *reqs, uint32_t n, uint64_t *hists,
@@ -232,9 +236,9 @@ cr_status cr_hamming_report(uint32_t k, const uint64_t *weights, int with_1bit, 
  * its countHammingUndetectableErrors<k> output): per weight i = 0..N the
  * non-extended weight distribution, the detecting-only and correcting Extended
  * Hamming distributions, their totals x 2^k, 2^k * C(N, i) and the two
- * probabilities.  method 0: device enumeration of all 2^k words for k <= 40,
- * else the MacWilliams identity over the 2^r dual words (exact, any k); 1:
- * device enumeration (k <= 40); 2: MacWilliams (ctx may be NULL).  If
+ * probabilities.  method 0: the device weights of all 2^k words for k <= 40
+ * (the range request of cr_hamming_weights), else the MacWilliams identity over
+ * the 2^r dual words (exact, any k); 1: device weights (k <= 40); 2: MacWilliams (ctx may be NULL).  If
  * weights_u128 is not NULL it receives the N+1 non-extended weights as (lo, hi)
  * pairs (nweights >= N+1).  *text is released with cr_free. */
 cr_status cr_hamming_sdc_table(cr_context *ctx, uint32_t k, int method, uint64_t *weights_u128, uint32_t nweights,
