@@ -242,6 +242,19 @@ cr_status carry_run(const CarryPlan &p, void *table0, void *table1, const Direct
     return CR_OK;
 }
 
+cr_status ordered_finish(uint64_t words, uint32_t bins, const uint64_t *hist, uint64_t *raw, uint32_t nbins) {
+    uint64_t total = 0;
+    for (uint32_t b = 0; b < nbins; ++b) raw[b] = 0;
+    for (uint32_t b = 0; b < bins; ++b) {
+        total += hist[b];
+        if (b == 0 ? hist[b] != words : b >= nbins ? hist[b] != 0 : (hist[b] & 1) != 0)
+            return fail(CR_ERR_DEVICE, "carry recursion: inconsistent count at distance %u", b);
+        if (b > 0 && b < nbins) raw[b] = hist[b] / 2;
+    }
+    if (total != words * words) return fail(CR_ERR_DEVICE, "carry recursion: inconsistent total");
+    return CR_OK;
+}
+
 cr_status carry_finish(uint32_t k, uint32_t bins, const uint64_t *hist, uint32_t copies, uint64_t *raw,
                        uint32_t nbins) {
     const uint64_t stride = hist_copy_stride(bins);

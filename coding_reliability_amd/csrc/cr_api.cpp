@@ -156,6 +156,24 @@ cr_status an_pairs_carry(cr_context *ctx, const CarryPlan &p, uint64_t A, uint64
     return st;
 }
 
+// Any word count (carry_ragged.hip).
+cr_status an_pairs_ragged(cr_context *ctx, const CarryRaggedPlan &p, uint64_t A, uint64_t num_words, uint64_t *raw,
+                          uint32_t nbins, double *kernel_ms) {
+    clear_error();
+    if (!ctx || !raw) return fail(CR_ERR_INVALID_ARGUMENT, "NULL argument");
+    const uint32_t need = pair_max_distance(A, num_words) + 1;
+    if (nbins < need) return fail(CR_ERR_INVALID_ARGUMENT, "nbins=%u but distances reach %u", nbins, need - 1);
+    CR_HIP(hipSetDevice(ctx->device));
+    CR_TRY(ctx->table_a.reserve(p.table_bytes));
+    CR_TRY(ctx->table_b.reserve(p.table_bytes));
+    dev::DirectResult out;
+    CR_TRY(direct_result(ctx, &out));
+    CR_TRY(carry_ragged_run(p, ctx->table_a.ptr, ctx->table_b.ptr, out, ctx->cus, ctx->stream));
+    uint64_t ordered[dev::kDirectBins];
+    CR_TRY(direct_wait(ctx, ordered, p.nbins, p.nbins, kernel_ms));
+    return ordered_finish(num_words, p.nbins, ordered, raw, nbins);
+}
+
 // The same by tiles (carry_tiles.hip).
 cr_status an_pairs_tiles(cr_context *ctx, const CarryTilesPlan &p, uint64_t A, uint64_t *raw, uint32_t nbins,
                          double *kernel_ms) {
@@ -430,6 +448,12 @@ cr_status cr_an_pairs(cr_context *ctx, uint64_t A, uint64_t num_words, uint64_t 
     }
     if (recursion) {
         const cr_status s = an_pairs_carry(ctx, carry, A, raw, nbins, kernel_ms);
+        if (s != CR_ERR_OUT_OF_MEMORY) return s;
+    }
+    CarryRaggedPlan ragged;
+    if (!((unsigned __int128)(num_words - 1) * A >> 64) && carry_ragged_plan(A, num_words, &ragged) &&
+        ragged.seconds < best) {
+        const cr_status s = an_pairs_ragged(ctx, ragged, A, num_words, raw, nbins, kernel_ms);
         if (s != CR_ERR_OUT_OF_MEMORY) return s;
     }
     if (spectral && spectral_s < pairwise) return cr_an_pairs_spectral(ctx, A, k, raw, nbins, kernel_ms);

@@ -271,6 +271,25 @@ cr_status carry_run(const CarryPlan &p, void *table0, void *table1, const dev::D
 cr_status carry_finish(uint32_t k, uint32_t bins, const uint64_t *hist, uint32_t copies, uint64_t *raw,
                        uint32_t nbins);
 
+// The same for any word count, odd parts below 1024 (see carry_ragged.hip).
+struct CarryRaggedPlan {
+    uint32_t A = 0, N = 0;      // odd part of the multiplier, words
+    uint32_t T = 0;             // 2^T > A, at least 7
+    uint32_t levels = 0;        // the highest bit of N
+    uint32_t states = 0;        // carry pairs, A^2
+    uint32_t tail = 0;          // words paired one by one
+    uint32_t nbins = 0;
+    uint64_t table_bytes = 0;   // of each of the two tables
+    double seconds = 0;         // estimated time of a call
+};
+bool carry_ragged_plan(uint64_t A, uint64_t num_words, CarryRaggedPlan *p);
+// Leaves the distribution over ordered pairs, p.nbins counts, in out.host.
+cr_status carry_ragged_run(const CarryRaggedPlan &p, void *table0, void *table1, const dev::DirectResult &out, int cus,
+                           hipStream_t stream);
+// raw[] (nbins entries, pair-kernel form) from `bins` counts of ordered pairs of
+// `words` words; checks the words at distance 0 and the total.
+cr_status ordered_finish(uint64_t words, uint32_t bins, const uint64_t *hist, uint64_t *raw, uint32_t nbins);
+
 // The same recursion for long multipliers, by tiles of carry pairs with four
 // levels a kernel (see carry_tiles.hip).
 struct CarryTilesPlan {

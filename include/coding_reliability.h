@@ -101,9 +101,11 @@ cr_status cr_probe_ceiling(cr_context *ctx, uint32_t probe, uint32_t iters, doub
  * (up to 2^13 words) in one launch; for num_words = 2^k a bit-sliced kernel (up
  * to 2^24 words of multipliers up to 16 bits), recursions over the carries of
  * the product (odd part of A below 4096 and k <= 32, or below 65536 and k <=
- * 26) and the Walsh-Hadamard spectrum (cr_an_pairs_spectral); otherwise the
- * pair kernel, which cr_an_pairs_tuned always runs.  The recursions take device
- * tables of up to 2 GiB each, kept by the context up to 1 GiB.
+ * 26) and the Walsh-Hadamard spectrum (cr_an_pairs_spectral); for other counts
+ * below 2^21 and odd parts below 1024 a recursion too; otherwise the pair
+ * kernel, which cr_an_pairs_tuned always runs.  The recursions take device
+ * tables of up to 2 GiB each, kept by the context up to 1 GiB; without memory
+ * for them the next method runs.
  * kernel_ms (may be NULL) receives the device time of the launches (of calls
  * of one launch and of the recursions by the device's constant-rate clock). */
 cr_status cr_an_pairs(cr_context *ctx, uint64_t A, uint64_t num_words, uint64_t *raw, uint32_t nbins,
