@@ -417,7 +417,8 @@ cr_status cr_an_pairs_tuned(cr_context *ctx, uint64_t A, uint64_t num_words, uin
 cr_status cr_an_pairs(cr_context *ctx, uint64_t A, uint64_t num_words, uint64_t *raw, uint32_t nbins,
                       double *kernel_ms) {
     // the same histogram by whichever method is estimated to be the fastest:
-    // the short kernel (measured 13 us a call of 2^8 words, 20 us of 2^13), the
+    // the short kernel (measured 13 us a call of 2^8 words, 20 us of 2^13, 0.2 ms
+    // of 50000), the
     // pair kernel (40 us a call and about 7e12 pairs/s where it competes), the
     // sliced kernel (34 us at 2^14 words, then the rates of sliced_rate), the
     // code's spectrum, the recursions over carries

@@ -135,7 +135,7 @@ cr_status launch_pairs(const PairJob *d_jobs, uint32_t njobs, uint64_t total_ite
 uint32_t pair_waves_per_cu(uint32_t R, uint32_t lds_rows, bool wide);
 
 // Pair histogram of a short code in one launch (see short_pairs.hip).
-constexpr uint32_t kShortWords = 1u << 13;
+constexpr uint32_t kShortWords = (1u << 16) - 1;
 namespace dev {
 struct DirectResult;
 }

@@ -1,6 +1,6 @@
 // Pair-distance histograms of short codes in one launch (gfx950): the same
-// raw[] as the pair kernel for up to 2^13 words, where a call is bound by its
-// launches, copies and tail and not by its pairs.
+// raw[] as the pair kernel for fewer than 2^16 words, where a call is bound by
+// its launches, copies and tail as much as by its pairs.
 //
 // Rows in blocks of 64 * R (R codewords a lane in registers), the columns from
 // the block's first row to the end in steps of one wave-uniform column; the
@@ -9,8 +9,10 @@
 // histogram (a counter a distance and lane, ds_add_u32 to the lane's own bank);
 // the last workgroup to finish writes the sums to pinned host memory
 // (direct_finish).  A call of 2^8 words takes one workgroup.  Measured a call
-// (device time): 2^8 words 13.5 us (3.5), 2^13 20 us (12); the pair kernel with
-// its fill, job upload, result copy and timing events 43 us (15) and 49 us (20).
+// (device time): 2^8 words 13.5 us (3.5), 2^13 20 us (12); 10001 words 25 us,
+// 20001 50 us, 50001 200 us; the pair kernel with its fill, job upload, result
+// copy and timing events 43 us (15), 49 us (20), 48, 73 and 344 us.  At 2^16 words
+// both take 0.32 ms (one workgroup a CU here).
 #include <algorithm>
 
 #include "cr_device.h"
@@ -124,7 +126,7 @@ cr_status launch_short_pairs(uint64_t A, uint32_t N, uint32_t nbins, const dev::
     job.R = N >= 2048 ? 4 : 1;
     job.nbins = nbins;
     for (uint32_t b = 0; b < N; b += 64 * job.R) job.steps += N - b;
-    // at least 32 steps a wave; a counter is below 2^13 * R
+    // at least 32 steps a wave; a counter is below 2^16 * R
     const uint32_t groups = std::min<uint32_t>((uint32_t)cus, std::max<uint32_t>(1, job.steps / (32 * kWaves)));
     job.share = (job.steps + groups * kWaves - 1) / (groups * kWaves);
     dev::DirectResult a_out = out;

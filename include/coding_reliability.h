@@ -98,7 +98,7 @@ cr_status cr_probe_ceiling(cr_context *ctx, uint32_t probe, uint32_t iters, doub
  * (an_coding.cu:287-292).  With A = A0*s and num_words = m it is the
  * integer-stride grid {A0*(i*s) : i < m}.
  * The method is the one estimated to be the fastest, all exact: short codes
- * (up to 2^13 words) in one launch; for num_words = 2^k a bit-sliced kernel (up
+ * (below 2^16 words) in one launch; for num_words = 2^k a bit-sliced kernel (up
  * to 2^24 words of multipliers up to 16 bits), recursions over the carries of
  * the product (odd part of A below 4096 and k <= 32, or below 65536 and k <=
  * 26) and the Walsh-Hadamard spectrum (cr_an_pairs_spectral); for other counts

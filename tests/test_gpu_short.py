@@ -82,3 +82,11 @@ def test_single_requests_between_short_codes(ctx):
         n = min(k, 20)
         got, _ = ctx.an_mc(61, n, 33, seed=k)
         assert got == O.an_mc(61, n, 33, k)[:len(got)]
+
+
+@pytest.mark.parametrize("A", [4097, 58659, 58659 * 4097, (1 << 40) + 1])
+@pytest.mark.parametrize("N", [8195, 12289, 16383, 30000, 65535])
+def test_longer_short_codes_match_the_pair_kernel(ctx, A, N):
+    # every workgroup busy, waves that start and end inside row blocks; the last
+    # word count of the short kernel
+    assert ctx.an_pairs_auto(A, N)[0] == ctx.an_pairs(A, N)[0]
