@@ -101,7 +101,7 @@ cr_status direct_result(cr_context *ctx, dev::DirectResult *r) {
     return CR_OK;
 }
 
-cr_status direct_wait(cr_context *ctx, uint64_t *raw, uint32_t need, uint32_t nbins, double *kernel_ms) {
+cr_status direct_poll(cr_context *ctx, double *kernel_ms) {
     // the kernel's last store, after its results: seen 3 to 6 us before the runtime
     // reports the stream idle (calls of 17 to 46 us; a stream query after it
     // costs 10 us).  Calls that take long, or fail, wait for the runtime.
@@ -111,12 +111,17 @@ cr_status direct_wait(cr_context *ctx, uint64_t *raw, uint32_t need, uint32_t nb
     while (!(done = __atomic_load_n(end, __ATOMIC_ACQUIRE) != 0) && std::chrono::steady_clock::now() < limit) {
     }
     if (!done) CR_HIP(hipStreamSynchronize(ctx->stream));
-    memcpy(raw, ctx->host.ptr, need * sizeof(uint64_t));
-    memset(raw + need, 0, (nbins - need) * sizeof(uint64_t));
     if (kernel_ms) {
         const uint64_t *clock = ctx->host.as<uint64_t>() + dev::kDirectBins;
         *kernel_ms = (double)std::max<int64_t>((int64_t)(clock[1] - clock[0]), 1) / ctx->wall_khz;
     }
+    return CR_OK;
+}
+
+cr_status direct_wait(cr_context *ctx, uint64_t *raw, uint32_t need, uint32_t nbins, double *kernel_ms) {
+    CR_TRY(direct_poll(ctx, kernel_ms));
+    memcpy(raw, ctx->host.ptr, need * sizeof(uint64_t));
+    memset(raw + need, 0, (nbins - need) * sizeof(uint64_t));
     return CR_OK;
 }
 

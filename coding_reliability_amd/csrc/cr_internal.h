@@ -144,6 +144,7 @@ cr_status launch_short_pairs(uint64_t A, uint32_t N, uint32_t nbins, const dev::
 // Buffers of a one-launch call on a context, and its end: waits, raw[0, need)
 // from pinned memory, zeros above, the device time.
 cr_status direct_result(cr_context *ctx, dev::DirectResult *r);
+cr_status direct_poll(cr_context *ctx, double *kernel_ms);
 cr_status direct_wait(cr_context *ctx, uint64_t *raw, uint32_t need, uint32_t nbins, double *kernel_ms);
 
 // Pair histograms of whole codes by bit planes (see sliced_pairs.hip).
@@ -344,6 +345,12 @@ cr_status launch_hamming(const HamJob *d_jobs, uint32_t njobs, uint64_t total_it
                          unsigned long long *counter, bool allow_static, uint32_t lds_rows, int cus,
                          hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1);
 // One job whose histogram goes to `out` (out_copies: dev::kHistCopies).
+// The first and the last launch of a small batch: `entries` counters cleared and
+// the start clock; the counters copied to pinned memory and the end clock.
+cr_status launch_batch_begin(unsigned long long *hist, uint32_t entries, const dev::DirectResult &out,
+                             hipStream_t stream);
+cr_status launch_batch_end(const unsigned long long *hist, uint32_t entries, unsigned long long *host,
+                           const dev::DirectResult &out, hipStream_t stream);
 cr_status launch_hamming_direct(const HamJob &job, bool w64, bool allow_static, uint32_t lds_rows,
                                 const dev::DirectResult &out, int cus, hipStream_t stream);
 // A sample range of an AN Monte Carlo launch and its histogram: the pairs

@@ -441,6 +441,20 @@ __global__ __launch_bounds__(64) void an_mc_kernel(uint64_t A, uint32_t n, uint6
     if (ONE) direct_finish(direct, nbins, lds);
 }
 
+__global__ __launch_bounds__(256) void batch_begin(unsigned long long *__restrict__ hist, uint32_t entries,
+                                                   const DirectResult out) {
+    direct_start(out);
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < entries; i += gridDim.x * 256) hist[i] = 0;
+}
+
+// One workgroup: the stores that the end clock waits for are its own.
+__global__ __launch_bounds__(1024) void batch_end(const unsigned long long *__restrict__ hist, uint32_t entries,
+                                                  unsigned long long *__restrict__ host, const DirectResult out) {
+    for (uint32_t i = threadIdx.x; i < entries; i += 1024)
+        __hip_atomic_store(host + i, hist[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    direct_end(out);
+}
+
 // Dynamic LDS of a Hamming wave: the histogram rows (the syndrome tables are
 // the kernel's static LDS).
 size_t ham_lds_bytes(uint32_t lds_rows) { return (size_t)lds_rows * kStride * sizeof(uint32_t); }
@@ -516,6 +530,19 @@ cr_status launch_hamming(const HamJob *d_jobs, uint32_t njobs, uint64_t total_it
     if (ev0) CR_HIP(hipEventRecord(ev0, stream));
     CR_TRY(ham_launch(d_jobs, njobs, total_items, w64, counter, lds_rows, waves, HamJob{}, DirectResult{}, stream));
     if (ev1) CR_HIP(hipEventRecord(ev1, stream));
+    return CR_OK;
+}
+
+cr_status launch_batch_begin(unsigned long long *hist, uint32_t entries, const DirectResult &out, hipStream_t stream) {
+    hipLaunchKernelGGL(batch_begin, dim3((entries + 255) / 256), dim3(256), 0, stream, hist, entries, out);
+    CR_HIP(hipGetLastError());
+    return CR_OK;
+}
+
+cr_status launch_batch_end(const unsigned long long *hist, uint32_t entries, unsigned long long *host,
+                           const DirectResult &out, hipStream_t stream) {
+    hipLaunchKernelGGL(batch_end, dim3(1), dim3(1024), 0, stream, hist, entries, host, out);
+    CR_HIP(hipGetLastError());
     return CR_OK;
 }
 

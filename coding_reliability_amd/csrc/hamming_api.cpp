@@ -101,6 +101,8 @@ HamJob ham_job(const cr_ham_request *req, uint32_t need, const uint64_t masks[7]
     return job;
 }
 
+constexpr uint64_t kSmallBatch = 16384;  // counters that one workgroup copies in a few us: seven requests of 72 weights
+
 // One request in one launch.
 cr_status hamming_single(cr_context *ctx, const cr_ham_request *req, uint64_t *hist, uint32_t nbins,
                          double *kernel_ms) {
@@ -229,13 +231,25 @@ cr_status hamming_run(cr_context *ctx, const cr_ham_request *reqs, uint32_t n, u
             all.push_back(job);
         }
     for (size_t j = 0; j < ranges.size(); ++j) ranges[j].out = hist + range_results[j].at;
-    CR_TRY(fill_zero_u64(hist, entries, ctx->stream));
+    // few requests: the counters come back as one-launch calls' do, without the
+    // copy, the events and the runtime's wait (the (39,32) stride grid of 2^20
+    // words beside one of 2^20 Monte Carlo words: 43 -> 31 us)
+    constexpr uint32_t kHeader = dev::kDirectBins + 2;
+    const bool small = entries <= kSmallBatch;
+    CR_TRY(ctx->host.reserve((kHeader + entries) * sizeof(uint64_t)));
+    dev::DirectResult out;
+    if (small) {
+        CR_TRY(direct_result(ctx, &out));
+        CR_TRY(launch_batch_begin(hist, (uint32_t)entries, out, ctx->stream));
+    } else {
+        CR_TRY(fill_zero_u64(hist, entries, ctx->stream));
+    }
     if (njobs) CR_HIP(hipMemcpyAsync(ctx->jobs.ptr, all.data(), job_bytes, hipMemcpyHostToDevice, ctx->stream));
     HamRange *d_ranges = reinterpret_cast<HamRange *>(ctx->jobs.as<char>() + job_bytes);
     if (!ranges.empty())
         CR_HIP(hipMemcpyAsync(d_ranges, ranges.data(), range_bytes, hipMemcpyHostToDevice, ctx->stream));
     // HIP events before the first launch and after the last
-    if (kernel_ms) CR_HIP(hipEventRecord(ctx->ev0, ctx->stream));
+    if (kernel_ms && !small) CR_HIP(hipEventRecord(ctx->ev0, ctx->stream));
     if (!ranges.empty())
         CR_TRY(launch_ham_ranges(d_ranges, (uint32_t)ranges.size(), nullptr, range_k, range_r, dev::DirectResult{},
                                  ctx->stream));
@@ -246,18 +260,23 @@ cr_status hamming_run(cr_context *ctx, const cr_ham_request *reqs, uint32_t n, u
                               L.items, w == 1, ctx->counters.as<unsigned long long>() + w, L.short_launch, L.rows,
                               ctx->cus, ctx->stream, nullptr, nullptr));
     }
-    if (kernel_ms) CR_HIP(hipEventRecord(ctx->ev1, ctx->stream));
-    CR_TRY(ctx->host.reserve(entries * sizeof(uint64_t)));
-    CR_HIP(hipMemcpyAsync(ctx->host.ptr, hist, entries * sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
-    CR_HIP(hipStreamSynchronize(ctx->stream));
-    const uint64_t *copies = static_cast<const uint64_t *>(ctx->host.ptr);
+    uint64_t *const copies = ctx->host.as<uint64_t>() + kHeader;
+    if (small) {
+        CR_TRY(launch_batch_end(hist, (uint32_t)entries, reinterpret_cast<unsigned long long *>(copies), out,
+                                ctx->stream));
+        CR_TRY(direct_poll(ctx, kernel_ms));
+    } else {
+        if (kernel_ms) CR_HIP(hipEventRecord(ctx->ev1, ctx->stream));
+        CR_HIP(hipMemcpyAsync(copies, hist, entries * sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
+        CR_HIP(hipStreamSynchronize(ctx->stream));
+    }
     results.insert(results.end(), range_results.begin(), range_results.end());
     for (const Result &r : results) {
         uint64_t *h = hists + (uint64_t)r.index * nbins;
         for (uint32_t c = 0; c < r.copies; ++c)
             for (uint32_t b = 0; b < r.need; ++b) h[b] += copies[r.at + c * dev::hist_copy_stride(r.need) + b];
     }
-    if (kernel_ms) {
+    if (kernel_ms && !small) {
         float ms = 0;
         CR_HIP(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
         *kernel_ms = ms;
