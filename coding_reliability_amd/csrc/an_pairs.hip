@@ -371,11 +371,12 @@ cr_status launch_pairs(const PairJob *d_jobs, uint32_t njobs, uint64_t total_ite
         const uint64_t per = (total_items + waves - 1) / waves;
         waves = (uint32_t)((total_items + per - 1) / per);
     }
-    if (cfg.zero_counter && counter)
-        CR_TRY(fill_zero_u64(counter, cfg.heads > 1 ? kQueues * kQueuePitch : 1, stream));
+    // a head without a wave would keep its items: the caller may ask for fewer waves
+    const uint32_t heads = std::min(cfg.heads, waves);
+    if (cfg.zero_counter && counter) CR_TRY(fill_zero_u64(counter, heads > 1 ? kQueues * kQueuePitch : 1, stream));
     if (ev0) CR_HIP(hipEventRecord(ev0, stream));
     const PairJob *a_jobs = d_jobs;
-    uint32_t a_njobs = njobs, a_heads = cfg.heads, a_rows = cfg.lds_rows;
+    uint32_t a_njobs = njobs, a_heads = heads, a_rows = cfg.lds_rows;
     uint64_t a_items = total_items;
     unsigned long long *a_counter = counter;
     void *args[] = {(void *)&a_jobs, (void *)&a_njobs, (void *)&a_items, (void *)&a_counter, (void *)&a_heads,

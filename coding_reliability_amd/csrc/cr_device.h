@@ -168,8 +168,8 @@ __device__ __forceinline__ uint64_t following_item(unsigned long long *counter, 
 }
 
 // The same over n <= kQueues heads: item t belongs to the queue t mod n, wave w
-// to the queue w mod n (with fewer waves than queues each wave has an item and
-// none is left).
+// to the queue w mod n.  The launch has at least n waves, or as many as items
+// (each then has one and none is left): a queue without a wave is never served.
 __device__ __forceinline__ uint64_t following_item_of(unsigned long long *heads, uint32_t n) {
     const uint32_t q = blockIdx.x % n, waves = (gridDim.x - q + n - 1) / n;
     return q + (uint64_t)n * (waves + next_item(heads + q * kQueuePitch));
