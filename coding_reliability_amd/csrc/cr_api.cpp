@@ -84,15 +84,13 @@ void auto_pair_tuning(uint64_t N, uint32_t resident_waves, uint32_t &R, uint32_t
 namespace cr {
 
 cr_status direct_result(cr_context *ctx, dev::DirectResult *r) {
-    if (!ctx->direct.ptr) {
-        CR_TRY(ctx->direct.reserve(dev::kDirectEntries * sizeof(uint64_t)));
-        const cr_status s = fill_zero_u64(ctx->direct.as<unsigned long long>(), dev::kDirectEntries, ctx->stream);
-        if (s != CR_OK) {
-            ctx->direct.release();
-            return s;
-        }
-    }
+    CR_TRY(ctx->direct.reserve(dev::kDirectEntries * sizeof(uint64_t)));
     CR_TRY(ctx->host.reserve((dev::kDirectBins + 2) * sizeof(uint64_t)));
+    // new, or left by a call that did not come to its end (a refused launch
+    // after one that had added counts)
+    if (!ctx->direct_clean)
+        CR_TRY(fill_zero_u64(ctx->direct.as<unsigned long long>(), dev::kDirectEntries, ctx->stream));
+    ctx->direct_clean = false;
     r->copies = ctx->direct.as<unsigned long long>();
     r->queue = r->copies + (size_t)dev::kHistCopies * dev::kDirectBins;
     r->tickets = reinterpret_cast<unsigned int *>(r->queue + dev::kQueues * dev::kQueuePitch);
@@ -111,6 +109,7 @@ cr_status direct_poll(cr_context *ctx, double *kernel_ms) {
     while (!(done = __atomic_load_n(end, __ATOMIC_ACQUIRE) != 0) && std::chrono::steady_clock::now() < limit) {
     }
     if (!done) CR_HIP(hipStreamSynchronize(ctx->stream));
+    ctx->direct_clean = true;
     if (kernel_ms) {
         const uint64_t *clock = ctx->host.as<uint64_t>() + dev::kDirectBins;
         *kernel_ms = (double)std::max<int64_t>((int64_t)(clock[1] - clock[0]), 1) / ctx->wall_khz;

@@ -67,7 +67,8 @@ __device__ __forceinline__ unsigned long long *hist_copy(unsigned long long *out
 // A call of one launch: the workgroups add to the histogram copies, the last
 // one to finish sums them into pinned host memory.  The copies, the queue head
 // and the tickets are zero between launches: the last workgroup leaves them so,
-// so a call needs no fill before and no copy after its kernel.
+// so a call needs no fill before and no copy after its kernel (only one after
+// a call that ended early does).
 struct DirectResult {
     unsigned long long *copies = nullptr;  // kHistCopies copies, hist_copy_stride(nbins) apart
     unsigned long long *queue = nullptr;   // work-queue heads, kQueuePitch apart

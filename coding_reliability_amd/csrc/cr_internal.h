@@ -141,8 +141,9 @@ struct DirectResult;
 }
 cr_status launch_short_pairs(uint64_t A, uint32_t N, uint32_t nbins, const dev::DirectResult &out, int cus,
                              hipStream_t stream);
-// Buffers of a one-launch call on a context, and its end: waits, raw[0, need)
-// from pinned memory, zeros above, the device time.
+// Buffers of a one-launch call on a context, cleared if an earlier call left
+// counts in them, and its end: waits, raw[0, need) from pinned memory, zeros
+// above, the device time.
 cr_status direct_result(cr_context *ctx, dev::DirectResult *r);
 cr_status direct_poll(cr_context *ctx, double *kernel_ms);
 cr_status direct_wait(cr_context *ctx, uint64_t *raw, uint32_t need, uint32_t nbins, double *kernel_ms);
@@ -388,7 +389,8 @@ struct cr_context {
     cr::DeviceBuffer jobs;     // PairJob array
     cr::DeviceBuffer counters; // work-queue heads
     cr::DeviceBuffer hist;     // histograms
-    cr::DeviceBuffer direct;   // histogram copies, queue head and tickets of one-launch calls, zero between them
+    cr::DeviceBuffer direct;   // histogram copies, queue heads and tickets of one-launch calls
+    bool direct_clean = false; // they are zero: the last such call came to its end
     cr::DeviceBuffer table_a;  // row / sample tables
     cr::DeviceBuffer table_b;
     cr::HostBuffer host;       // pinned staging
