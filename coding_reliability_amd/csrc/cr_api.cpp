@@ -244,7 +244,53 @@ bool tiles_preferred(uint64_t A, uint64_t num_words, double seconds, CarryTilesP
     return carry_tiles_plan(A, (uint32_t)__builtin_ctzll(num_words), p) && p->seconds < seconds;
 }
 
+cr_status an_pairs_by(cr_context *ctx, const PairsPlan &p, uint32_t method, uint64_t A, uint64_t num_words,
+                      uint64_t *raw, uint32_t nbins, double *kernel_ms) {
+    switch (method) {
+    case kByTiles: return an_pairs_tiles(ctx, p.tiles, A, raw, nbins, kernel_ms);
+    case kByCarry: return an_pairs_carry(ctx, p.carry, A, raw, nbins, kernel_ms);
+    case kByBlocks: return an_pairs_ragged(ctx, p.ragged, A, num_words, raw, nbins, kernel_ms);
+    case kBySpectrum: return cr_an_pairs_spectral(ctx, A, p.k, raw, nbins, kernel_ms);
+    case kByPlanes: return an_pairs_sliced(ctx, p.sliced, A, num_words, raw, nbins, kernel_ms);
+    case kByShort: return an_pairs_short(ctx, A, num_words, raw, nbins, kernel_ms);
+    default: return cr_an_pairs_tuned(ctx, A, num_words, raw, nbins, nullptr, kernel_ms);
+    }
+}
+
 }  // namespace
+
+// the short kernel (measured 13 us a call of 2^8 words, 20 us of 2^13, 0.2 ms of
+// 50000), the pair kernel (40 us a call and about 7e12 pairs/s where it
+// competes), the sliced kernel (34 us at 2^14 words, then the rates of
+// sliced_rate), the code's spectrum, the recursions over carries
+void pairs_plan(uint64_t A, uint64_t num_words, PairsPlan *p) {
+    p->methods = 0;
+    auto then = [p](PairsMethod m) { p->method[p->methods++] = m; };
+    const double pairs = 0.5 * (double)num_words * (double)num_words;
+    const bool is_short = A != 0 && num_words != 0 && num_words <= kShortWords &&
+                          !((unsigned __int128)(num_words - 1) * A >> 64);
+    double best = is_short ? 15e-6 + pairs / 6.7e12 : 40e-6 + pairs / 7e12;
+    bool by_planes = false;
+    if (sliced_job(A, num_words, &p->sliced)) {
+        const double s = 27e-6 + pairs / sliced_rate(p->sliced);
+        by_planes = s < best;
+        best = std::min(best, s);
+    }
+    const double pairwise = best;
+    double spectral_s = 0;
+    const bool spectral = spectral_preferred(A, num_words, &p->k, &spectral_s);
+    if (spectral) best = std::min(best, spectral_s);
+    const bool recursion = carry_preferred(A, num_words, best, &p->carry);
+    if (recursion) best = p->carry.seconds;
+    if (tiles_preferred(A, num_words, best, &p->tiles)) then(kByTiles);
+    if (recursion) then(kByCarry);
+    if (!((unsigned __int128)(num_words - 1) * A >> 64) && carry_ragged_plan(A, num_words, &p->ragged) &&
+        p->ragged.seconds < best)
+        then(kByBlocks);
+    if (spectral && spectral_s < pairwise) then(kBySpectrum);
+    then(by_planes ? kByPlanes : is_short ? kByShort : kByPairs);
+}
+
 }  // namespace cr
 
 using namespace cr;
@@ -420,51 +466,13 @@ cr_status cr_an_pairs_tuned(cr_context *ctx, uint64_t A, uint64_t num_words, uin
 
 cr_status cr_an_pairs(cr_context *ctx, uint64_t A, uint64_t num_words, uint64_t *raw, uint32_t nbins,
                       double *kernel_ms) {
-    // the same histogram by whichever method is estimated to be the fastest:
-    // the short kernel (measured 13 us a call of 2^8 words, 20 us of 2^13, 0.2 ms
-    // of 50000), the
-    // pair kernel (40 us a call and about 7e12 pairs/s where it competes), the
-    // sliced kernel (34 us at 2^14 words, then the rates of sliced_rate), the
-    // code's spectrum, the recursions over carries
-    uint32_t k = 0;
-    const double pairs = 0.5 * (double)num_words * (double)num_words;
-    const bool is_short = A != 0 && num_words != 0 && num_words <= kShortWords &&
-                          !((unsigned __int128)(num_words - 1) * A >> 64);
-    double best = is_short ? 15e-6 + pairs / 6.7e12 : 40e-6 + pairs / 7e12;
-    SlicedJob sliced;
-    bool by_planes = false;
-    if (sliced_job(A, num_words, &sliced)) {
-        const double s = 27e-6 + pairs / sliced_rate(sliced);
-        by_planes = s < best;
-        best = std::min(best, s);
+    PairsPlan p;
+    pairs_plan(A, num_words, &p);
+    for (uint32_t i = 0;; ++i) {
+        // without memory for a method's tables (up to 4 GiB) the next one
+        const cr_status s = an_pairs_by(ctx, p, p.method[i], A, num_words, raw, nbins, kernel_ms);
+        if (s != CR_ERR_OUT_OF_MEMORY || i + 1 >= p.methods) return s;
     }
-    const double pairwise = best;
-    double spectral_s = 0;
-    const bool spectral = spectral_preferred(A, num_words, &k, &spectral_s);
-    if (spectral) best = std::min(best, spectral_s);
-    CarryPlan carry;
-    const bool recursion = carry_preferred(A, num_words, best, &carry);
-    if (recursion) best = carry.seconds;
-    CarryTilesPlan tiles;
-    // without memory for a recursion's tables (up to 4 GiB) the next method
-    if (tiles_preferred(A, num_words, best, &tiles)) {
-        const cr_status s = an_pairs_tiles(ctx, tiles, A, raw, nbins, kernel_ms);
-        if (s != CR_ERR_OUT_OF_MEMORY) return s;
-    }
-    if (recursion) {
-        const cr_status s = an_pairs_carry(ctx, carry, A, raw, nbins, kernel_ms);
-        if (s != CR_ERR_OUT_OF_MEMORY) return s;
-    }
-    CarryRaggedPlan ragged;
-    if (!((unsigned __int128)(num_words - 1) * A >> 64) && carry_ragged_plan(A, num_words, &ragged) &&
-        ragged.seconds < best) {
-        const cr_status s = an_pairs_ragged(ctx, ragged, A, num_words, raw, nbins, kernel_ms);
-        if (s != CR_ERR_OUT_OF_MEMORY) return s;
-    }
-    if (spectral && spectral_s < pairwise) return cr_an_pairs_spectral(ctx, A, k, raw, nbins, kernel_ms);
-    if (by_planes) return an_pairs_sliced(ctx, sliced, A, num_words, raw, nbins, kernel_ms);
-    if (is_short) return an_pairs_short(ctx, A, num_words, raw, nbins, kernel_ms);
-    return cr_an_pairs_tuned(ctx, A, num_words, raw, nbins, nullptr, kernel_ms);
 }
 
 }  // extern "C"

@@ -306,6 +306,21 @@ bool carry_tiles_plan(uint64_t A, uint32_t k, CarryTilesPlan *p);
 cr_status carry_tiles_run(const CarryTilesPlan &p, void *table, unsigned long long *hist, int cus,
                           hipStream_t stream);
 
+// The methods of cr_an_pairs for a code, by their estimated times: the fastest,
+// then those that take its place when device memory for its tables lacks.  The
+// last one takes no tables.
+enum PairsMethod : uint32_t { kByPairs, kByShort, kByPlanes, kBySpectrum, kByCarry, kByTiles, kByBlocks };
+struct PairsPlan {
+    uint32_t methods = 0;
+    uint32_t method[5];
+    uint32_t k = 0;  // kBySpectrum: 2^k words
+    SlicedJob sliced;
+    CarryPlan carry;
+    CarryTilesPlan tiles;
+    CarryRaggedPlan ragged;
+};
+void pairs_plan(uint64_t A, uint64_t num_words, PairsPlan *p);
+
 // Weight histogram of consecutive data words, bit by bit of their bounds (see
 // hamming_range.hip).
 struct HamRange {

@@ -29,6 +29,20 @@ def padded_eq(a, b):
     return list(a) + [0] * (n - len(a)) == list(b) + [0] * (n - len(b))
 
 
+def pairs_methods(A, num_words):
+    """The methods of cr_an_pairs for a code, the fastest by estimate first, then
+    those that take its place without device memory for its tables."""
+    import ctypes as C
+    from coding_reliability_amd._lib import lib
+    plan = lib()._ZN2cr10pairs_planEmmPNS_9PairsPlanE
+    plan.argtypes, plan.restype = [C.c_uint64, C.c_uint64, C.c_void_p], None
+    p = (C.c_uint64 * 256)()  # cr::PairsPlan: the number of methods, the methods, their plans
+    plan(A, num_words, p)
+    words = C.cast(p, C.POINTER(C.c_uint32))
+    names = ["pairs", "short", "planes", "spectrum", "carry", "tiles", "blocks"]
+    return [names[words[1 + i]] for i in range(words[0])]
+
+
 import math
 
 
