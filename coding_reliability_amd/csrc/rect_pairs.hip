@@ -179,7 +179,8 @@ const void *rect_ptr() {
 cr_status launch_rect(const RectLaunch &L, const DirectResult &out, hipStream_t stream, int cus) {
     constexpr int R = 8;
     const void *k = L.w2 ? rect_ptr<R, true>() : rect_ptr<R, false>();
-    if (L.nrows == 0 || L.ncols == 0) return CR_OK;
+    // nothing would be launched, and the caller waits for a kernel's results
+    if (L.nrows == 0 || L.ncols == 0) return fail(CR_ERR_INVALID_ARGUMENT, "empty rectangle");
     if (L.lds_rows < 2 || L.lds_rows > 66) return fail(CR_ERR_INVALID_ARGUMENT, "bad histogram rows %u", L.lds_rows);
     const uint64_t RB = 64ull * R;
     const uint64_t RBlocks = (L.nrows + RB - 1) / RB;
