@@ -8,6 +8,7 @@ from __future__ import annotations
 
 import ctypes as C
 import itertools
+import operator
 
 import numpy as np
 
@@ -213,6 +214,8 @@ class Context:
         return BatchPlan(self, codes, rows_per_lane, items_per_wave)
 
     def autotune_batch(self, codes, repeats: int = 1) -> tuple[dict, float]:
+        # an array of codes takes floats and longer tuples without a word
+        codes = [(operator.index(A), operator.index(N)) for A, N in codes]
         best = cr_pair_tuning()
         ms = C.c_double(0)
         check(lib().cr_autotune_batch(self._h, self._codes(codes), len(codes), repeats, C.byref(best), C.byref(ms)))
