@@ -48,8 +48,10 @@ cr_status HostBuffer::reserve(size_t want) {
     size_t n = std::max(want, (size_t)4096);
     void *p = nullptr;
     hipError_t e = hipHostMalloc(&p, n, hipHostMallocDefault);
-    if (e != hipSuccess)
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
         return fail(CR_ERR_OUT_OF_MEMORY, "hipHostMalloc(%zu) failed: %s", n, hipGetErrorString(e));
+    }
     ptr = p;
     bytes = n;
     return CR_OK;

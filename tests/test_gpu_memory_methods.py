@@ -40,3 +40,17 @@ def test_tables_that_do_not_fit(A, N, left, methods):
         assert got == want and again == want
         if N < 1 << 24:
             assert ctx.an_pairs(A, N)[0] == want
+
+
+@pytest.mark.parametrize("buffer", ["DeviceBuffer", "HostBuffer"])
+def test_refused_allocation_leaves_no_error_behind(buffer):
+    # the runtime's last error is what the next launch would report
+    import ctypes as C
+    from coding_reliability_amd._lib import lib
+    with cra.Context(0):
+        reserve = getattr(lib(), f"_ZN2cr{len(buffer)}{buffer}7reserveEm")
+        reserve.argtypes, reserve.restype = [C.c_void_p, C.c_size_t], C.c_int
+        empty = (C.c_uint64 * 2)()  # ptr, bytes
+        assert lib().hipGetLastError() == 0
+        assert reserve(empty, 1 << 60) == 4 and list(empty) == [0, 0]
+        assert lib().hipGetLastError() == 0
