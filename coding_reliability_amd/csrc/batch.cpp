@@ -40,7 +40,7 @@ cr_status build_batch(cr_context *ctx, const cr_an_code *codes, uint32_t ncodes,
                       const cr_pair_tuning *tuning, unsigned long long *d_hist, BatchLayout &L) {
     if (!codes || ncodes == 0) return fail(CR_ERR_INVALID_ARGUMENT, "empty batch");
     const uint32_t ipw = tuning && tuning->items_per_wave ? tuning->items_per_wave : 16;
-    uint32_t max_need = 0;
+    uint32_t max_need = 0;  // of the pair kernel's codes: its waves per CU follow from their bins
     long double total_pairs = 0, short_pairs = 0;
     L.jobs.reserve(ncodes);
     for (uint32_t c = 0; c < ncodes; ++c) {
@@ -49,7 +49,6 @@ cr_status build_batch(cr_context *ctx, const cr_an_code *codes, uint32_t ncodes,
         if ((unsigned __int128)(N - 1) * A >> 64) return fail(CR_ERR_UNSUPPORTED, "code %u exceeds 64-bit codewords", c);
         const uint32_t need = pair_max_distance(A, N) + 1;
         if (need > stride) return fail(CR_ERR_INVALID_ARGUMENT, "code %u needs %u bins > stride %u", c, need, stride);
-        max_need = std::max(max_need, need);
         SlicedJob sj;
         if (sliced_job(A, N, &sj)) {
             sj.out = d_hist + (size_t)c * stride;
