@@ -9,7 +9,7 @@
 //   list    d = list[s]                         (the reference grid's sample points)
 //   mc      d = Philox word s of (seed, stream) (replaces dhamming_mc's cuRAND draw)
 // (Ranges of consecutive words, dhamming's exhaustive mode, hamming.cu:64-81, need
-// no enumeration: hamming_range.hip.)
+// no enumeration, see hamming_range.hip; a few words come here as a grid of stride 1.)
 // AN Monte Carlo: every word A*i against m Philox samples A*u_ij
 // (replaces dancoding_mc_shared, an_coding_mc.cu:94-158).
 #include <algorithm>

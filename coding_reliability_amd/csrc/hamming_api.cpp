@@ -101,7 +101,25 @@ HamJob ham_job(const cr_ham_request *req, uint32_t need, const uint64_t masks[7]
     return job;
 }
 
-constexpr uint64_t kSmallBatch = 16384;  // counters that one workgroup copies in a few us: seven requests of 72 weights
+// Ranges as the grids of stride 1 that they are, word by word, where a few words
+// take less time than the launch of the recursion over their bits: in a launch
+// of their width that is there anyway, in calls that are no small batch in
+// either way, and from k = 58 on, where the recursion takes 25 to 29 us.  Measured
+// beside 2^20 Monte Carlo words of the same width: 1000 words of k = 64 39 us for
+// 70, of k = 57 44 for 62, of k = 32 30 for 43; four ranges of 2^20 words 90 us for
+// 74 at k = 64, 60 for 51 at k = 20.
+constexpr double kWordsSeconds = 2e-6;    // of all of them, by ham_rate
+constexpr uint32_t kWordsMinK = 58;
+constexpr uint32_t kWordRanges = 4;       // eight: 0.85 to 1.22 of the recursion's time
+cr_ham_request as_words(const cr_ham_request *range) {
+    cr_ham_request r = *range;
+    r.source = CR_HAM_STRIDE;
+    r.stride = 1;
+    return r;
+}
+
+// Counters that one workgroup copies in a few us: of six requests of k = 64, ten of k = 32.
+constexpr uint64_t kSmallBatch = 16384;
 
 // One request in one launch.
 cr_status hamming_single(cr_context *ctx, const cr_ham_request *req, uint64_t *hist, uint32_t nbins,
@@ -117,6 +135,12 @@ cr_status hamming_single(cr_context *ctx, const cr_ham_request *req, uint64_t *h
         return CR_OK;
     }
     dev::DirectResult out;
+    cr_ham_request words;
+    if (req->source == CR_HAM_RANGE && req->k >= kWordsMinK &&
+        (double)req->count / ham_rate(req) < kWordsSeconds) {
+        words = as_words(req);
+        req = &words;
+    }
     if (req->source == CR_HAM_RANGE) {
         CR_TRY(direct_result(ctx, &out));
         const HamRange job = ham_range(req, need, parity, masks);
@@ -138,11 +162,11 @@ cr_status hamming_single(cr_context *ctx, const cr_ham_request *req, uint64_t *h
     return direct_wait(ctx, hist, need, nbins, kernel_ms);
 }
 
-// Requests [0, n): ranges as the workgroups of one launch, the others as one
-// Hamming job each, those of 32-bit words in one launch, those of 64-bit words
-// (k > 32) in another on the same stream, each launch's jobs in request order;
-// requests without samples launch nothing.  hists[i * nbins + b] is request
-// i's count of weight b.
+// Requests [0, n): ranges as the workgroups of one launch (few short ones as
+// Hamming jobs, see kWordsSeconds), the others as one Hamming job each, those of
+// 32-bit words in one launch, those of 64-bit words (k > 32) in another on the
+// same stream; requests without samples launch nothing.  hists[i * nbins + b] is
+// request i's count of weight b.
 cr_status hamming_run(cr_context *ctx, const cr_ham_request *reqs, uint32_t n, uint64_t *hists, uint32_t nbins,
                       double *kernel_ms) {
     if (!ctx || !reqs || !hists) return fail(CR_ERR_INVALID_ARGUMENT, "NULL argument");
@@ -150,7 +174,7 @@ cr_status hamming_run(cr_context *ctx, const cr_ham_request *reqs, uint32_t n, u
         return fail(CR_ERR_INVALID_ARGUMENT, "%u requests outside [1, %u]", n, kHamMaxBatch);
     if (n == 1) return hamming_single(ctx, reqs, hists, nbins, kernel_ms);
     struct Pending {
-        uint32_t index, need;
+        uint32_t index, need, parity;
         uint64_t masks[7];
     };
     struct Launch {
@@ -160,7 +184,13 @@ cr_status hamming_run(cr_context *ctx, const cr_ham_request *reqs, uint32_t n, u
         uint32_t rows = 2;
         uint64_t items = 0;
         bool short_launch = false;
+        void add(const cr_ham_request *req, const Pending &p) {
+            est_s += (double)req->count / ham_rate(req);
+            rows = std::max(rows, p.need + 1);
+            requests.push_back(p);
+        }
     } launches[2];
+    std::vector<Pending> range_requests;
     std::vector<HamRange> ranges;
     uint32_t range_k = 0, range_r = 0;
     struct Result {
@@ -169,24 +199,46 @@ cr_status hamming_run(cr_context *ctx, const cr_ham_request *reqs, uint32_t n, u
     };
     std::vector<Result> results, range_results;
     uint64_t list_words = 0, entries = 0;
+    uint64_t job_entries = 0, range_entries = 0;  // counters of the jobs, of the ranges in one copy
+    auto job_counters = [](const Pending &p) { return dev::hist_copy_stride(p.need) * dev::kHistCopies; };
     for (uint32_t q = 0; q < n; ++q) {
         const cr_ham_request *req = reqs + q;
-        Pending p{q, 0, {}};
-        uint32_t parity = 0;
-        CR_TRY(ham_check(req, nbins, &p.need, &parity, p.masks));
+        Pending p{q, 0, 0, {}};
+        CR_TRY(ham_check(req, nbins, &p.need, &p.parity, p.masks));
         if (req->count == 0) continue;
         if (req->source == CR_HAM_RANGE) {
-            ranges.push_back(ham_range(req, p.need, parity, p.masks));
-            range_k = std::max(range_k, req->k);
-            range_r = std::max(range_r, parity);
-            range_results.push_back({q, p.need, 1, 0});
+            range_requests.push_back(p);
+            range_entries += dev::hist_copy_stride(p.need);
             continue;
         }
         if (req->source == CR_HAM_LIST) list_words += req->count;
-        Launch &L = launches[req->k > 32];
-        L.est_s += (double)req->count / ham_rate(req);
-        L.rows = std::max(L.rows, p.need + 1);
-        L.requests.push_back(p);
+        launches[req->k > 32].add(req, p);
+        job_entries += job_counters(p);
+    }
+    // the ranges all one way or the other: the recursion's launch would stay for one
+    double range_s = 0;
+    bool joined = true, longest = true;  // launches of their widths are there; k of kWordsMinK and more
+    uint64_t word_entries = job_entries;
+    for (const Pending &p : range_requests) {
+        const cr_ham_request *req = reqs + p.index;
+        range_s += (double)req->count / ham_rate(req);
+        joined = joined && !launches[req->k > 32].requests.empty();
+        longest = longest && req->k >= kWordsMinK;
+        word_entries += job_counters(p);
+    }
+    const bool words = range_requests.size() <= kWordRanges && range_s < kWordsSeconds &&
+                       (longest || job_entries + range_entries > kSmallBatch ||
+                        (joined && word_entries <= kSmallBatch));
+    for (const Pending &p : range_requests) {
+        const cr_ham_request *req = reqs + p.index;
+        if (words) {
+            launches[req->k > 32].add(req, p);
+            continue;
+        }
+        ranges.push_back(ham_range(req, p.need, p.parity, p.masks));
+        range_k = std::max(range_k, req->k);
+        range_r = std::max(range_r, p.parity);
+        range_results.push_back({p.index, p.need, 1, 0});
     }
     CR_HIP(hipSetDevice(ctx->device));
     memset(hists, 0, (size_t)n * nbins * sizeof(uint64_t));
@@ -198,7 +250,12 @@ cr_status hamming_run(cr_context *ctx, const cr_ham_request *reqs, uint32_t n, u
         L.short_launch = L.est_s < 100e-6;
         const uint64_t waves = (uint64_t)hamming_waves_per_cu(L.rows) * ctx->cus;
         for (const Pending &p : L.requests) {
+            cr_ham_request words_of;
             const cr_ham_request *req = reqs + p.index;
+            if (req->source == CR_HAM_RANGE) {
+                words_of = as_words(req);
+                req = &words_of;
+            }
             HamJob job = ham_job(req, p.need, p.masks, L.short_launch, waves);
             job.item_begin = L.items;
             L.items += job.items;

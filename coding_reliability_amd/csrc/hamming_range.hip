@@ -17,7 +17,8 @@
 // turn, so that a step is one barrier; bound by that latency (0.35 us a step of
 // the (39,32) code, k = 64 by the LDS too).  Several counters of a thread in
 // flight did not help, 512 threads took 24 us where 1024 take 23.  Measured, a call
-// for 2^30 words of the (39,32) code 20 us (word by word 541 us), k = 64 42 us.
+// for 2^30 words of the (39,32) code 20 us (word by word 541 us), k = 64 42 us (a
+// few words 33 us word by word, so they do not come here: hamming_api.cpp).
 #include <algorithm>
 
 #include "cr_device.h"

@@ -218,8 +218,9 @@ cr_status cr_hamming_weights(cr_context *ctx, const cr_ham_request *req, uint64_
 /* n requests (1..4096) in one call: hists[i * nbins + w] is request i's
  * histogram, equal to cr_hamming_weights of that request; nbins must exceed
  * every request's largest weight.  Ranges run as the workgroups of one kernel
- * launch, the other requests of k <= 32 as the jobs of another, those of k > 32 as
- * the jobs of a third; kernel_ms spans them.  No counterpart in the reference: it puts small requests (the (39,32)
+ * launch (up to four of few words as jobs of the next two), the other requests of
+ * k <= 32 as the jobs of another, those of k > 32 as the jobs of a third; kernel_ms
+ * spans them.  No counterpart in the reference: it puts small requests (the (39,32)
  * stride grid of 2^20 words, a few microseconds of work) into the launch of a
  * larger one (its 2^34-word Monte Carlo run) instead of paying a launch each. */
 cr_status cr_hamming_weights_batch(cr_context *ctx, const cr_ham_request *reqs, uint32_t n, uint64_t *hists,
