@@ -41,6 +41,24 @@ template <int R>
 __device__ void pairs_masked(uint32_t *lane_col, const Rows<R> &rw, uint64_t A, uint64_t j0, uint64_t j1,
                              uint32_t dummy) {
     uint64_t v = A * j0;
+    if constexpr (R == 16) {
+        // XORs, then counts, then increments: left to itself the compiler may put
+        // one pair behind the other (which it does depends on the rest of the
+        // kernel), and a single wave, as of a short code, takes 15 % longer
+        for (uint64_t j = j0; j < j1; ++j, v += A) {
+            uint64_t x[R];
+            uint32_t c[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) x[r] = rw.w[r] ^ v;
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int r = 0; r < R; ++r) c[r] = (uint32_t)__popcll(x[r]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int r = 0; r < R; ++r) lds_inc(lane_col + (j > rw.i[r] ? c[r] : dummy) * kStride);
+        }
+        return;
+    }
     for (uint64_t j = j0; j < j1; ++j, v += A) {
 #pragma unroll
         for (int r = 0; r < R; ++r) {
@@ -195,10 +213,15 @@ __global__ void fill_zero_kernel(unsigned long long *p, size_t n) {
 // WIDE: also the code for kModeWide, whose tiles take 130 to 170 registers (3
 // waves a SIMD, which is what keeps the LDS busiest: 9.25e12 pairs/s, 9.0 to
 // 9.1 with 4); with it in one kernel the narrow codes lost 2 to 6 %.
+// 16 rows a lane: scheduled for the 4 waves a SIMD that its registers leave (the
+// compiler otherwise aims at 5 and misses them).  Measured with 16 rows: 1000
+// words 0.36 -> 0.32 ms, 65537 words of A = 58659 0.61 -> 0.55, 80001 0.67 -> 0.62,
+// 16384 codes of 256 words 0.92 -> 0.89.
 template <int R, bool WIDE>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WIDE ? 3 : 1))) void pair_kernel(const PairJob *__restrict__ jobs, uint32_t njobs,
-                                                  uint64_t total_items, unsigned long long *__restrict__ counter,
-                                                  uint32_t heads, uint32_t lds_rows) {
+__global__ __launch_bounds__(64)
+__attribute__((amdgpu_waves_per_eu(WIDE ? 3 : R == 16 ? 4 : 1, !WIDE && R == 16 ? 4 : 8)))
+void pair_kernel(const PairJob *__restrict__ jobs, uint32_t njobs, uint64_t total_items,
+                 unsigned long long *__restrict__ counter, uint32_t heads, uint32_t lds_rows) {
     extern __shared__ uint32_t lds[];
     const uint32_t lane = threadIdx.x;
     lds_clear(lds, lds_rows);
