@@ -73,6 +73,7 @@ cr_status build_batch(cr_context *ctx, const cr_an_code *codes, uint32_t ncodes,
     L.cfg.R = R;
     L.cfg.lds_rows = std::max(max_need, 1u) + 1;
     L.cfg.waves = tuning ? tuning->waves : 0;
+    L.cfg.zero_counter = false;
     for (PairJob &j : L.jobs) {
         j.mode = pair_mode(j.A, j.N);
         L.cfg.wide = L.cfg.wide || j.mode == kModeWide;
@@ -106,15 +107,18 @@ cr_status build_batch(cr_context *ctx, const cr_an_code *codes, uint32_t ncodes,
     return CR_OK;
 }
 
-// Both launches; counters: the pair kernel's work-queue heads, then the sliced one's.
+// The work-queue heads lie behind the n counts of the histograms, on lines of
+// their own, so that one fill clears both: the pair kernel's, then the sliced one's.
 constexpr size_t kCounters = dev::kQueues * dev::kQueuePitch + 1;
+size_t counters_at(size_t n) { return (n + dev::kQueuePitch - 1) / dev::kQueuePitch * dev::kQueuePitch; }
+size_t batch_entries(size_t n) { return counters_at(n) + kCounters; }
+
+// Both launches, the heads cleared.
 cr_status launch_batch(cr_context *ctx, const BatchLayout &L, void *d_jobs, unsigned long long *counters) {
     const SlicedJob *sliced = static_cast<const SlicedJob *>(d_jobs);
-    if (!L.sliced.empty()) {
-        unsigned long long *const head = counters + kCounters - 1;
-        CR_TRY(fill_zero_u64(head, 1, ctx->stream));
-        CR_TRY(launch_sliced(sliced, (uint32_t)L.sliced.size(), L.sliced_items, head, ctx->cus, ctx->stream));
-    }
+    if (!L.sliced.empty())
+        CR_TRY(launch_sliced(sliced, (uint32_t)L.sliced.size(), L.sliced_items, counters + kCounters - 1, ctx->cus,
+                             ctx->stream));
     if (!L.jobs.empty())
         CR_TRY(launch_pairs(reinterpret_cast<const PairJob *>(sliced + L.sliced.size()), (uint32_t)L.jobs.size(),
                             L.total_items, counters, L.cfg, ctx->cus, ctx->stream, nullptr, nullptr));
@@ -130,7 +134,7 @@ using namespace cr;
 struct cr_batch_plan {
     cr_context *ctx = nullptr;
     uint32_t ncodes = 0, stride = 0;
-    DeviceBuffer jobs, hist, counter;
+    DeviceBuffer jobs, hist;
     HostBuffer host;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -144,15 +148,15 @@ cr_status cr_an_batch(cr_context *ctx, const cr_an_code *codes, uint32_t ncodes,
     if (!ctx || !raw) return fail(CR_ERR_INVALID_ARGUMENT, "NULL argument");
     CR_HIP(hipSetDevice(ctx->device));
     const size_t n = (size_t)ncodes * stride;
-    CR_TRY(ctx->hist.reserve(n * sizeof(uint64_t)));
+    CR_TRY(ctx->hist.reserve(batch_entries(n) * sizeof(uint64_t)));
+    unsigned long long *const hist = ctx->hist.as<unsigned long long>();
     BatchLayout L;
-    CR_TRY(build_batch(ctx, codes, ncodes, stride, tuning, ctx->hist.as<unsigned long long>(), L));
+    CR_TRY(build_batch(ctx, codes, ncodes, stride, tuning, hist, L));
     CR_TRY(ctx->jobs.reserve(L.job_bytes()));
-    CR_TRY(ctx->counters.reserve(kCounters * sizeof(uint64_t)));
-    CR_TRY(fill_zero_u64(ctx->hist.as<unsigned long long>(), n, ctx->stream));
+    CR_TRY(fill_zero_u64(hist, batch_entries(n), ctx->stream));
     CR_HIP(L.upload(ctx->jobs.ptr, ctx->stream));
     if (kernel_ms) CR_HIP(hipEventRecord(ctx->ev0, ctx->stream));
-    CR_TRY(launch_batch(ctx, L, ctx->jobs.ptr, ctx->counters.as<unsigned long long>()));
+    CR_TRY(launch_batch(ctx, L, ctx->jobs.ptr, hist + counters_at(n)));
     if (kernel_ms) CR_HIP(hipEventRecord(ctx->ev1, ctx->stream));
     CR_TRY(ctx->host.reserve(n * sizeof(uint64_t)));
     CR_HIP(hipMemcpyAsync(ctx->host.ptr, ctx->hist.ptr, n * sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
@@ -173,7 +177,6 @@ cr_status cr_batch_plan_destroy(cr_batch_plan *p) {
     if (p->graph) (void)hipGraphDestroy(p->graph);
     p->jobs.release();
     p->hist.release();
-    p->counter.release();
     p->host.release();
     delete p;
     return CR_OK;
@@ -195,21 +198,21 @@ cr_status cr_batch_plan_create(cr_context *ctx, const cr_an_code *codes, uint32_
     };
     const size_t n = (size_t)ncodes * stride;
     cr_status s;
-    if ((s = p->hist.reserve(n * sizeof(uint64_t))) != CR_OK) return bail(s);
-    if ((s = p->counter.reserve(kCounters * sizeof(uint64_t))) != CR_OK) return bail(s);
+    if ((s = p->hist.reserve(batch_entries(n) * sizeof(uint64_t))) != CR_OK) return bail(s);
+    unsigned long long *const hist = p->hist.as<unsigned long long>();
     if ((s = p->host.reserve(n * sizeof(uint64_t))) != CR_OK) return bail(s);
     BatchLayout L;
-    if ((s = build_batch(ctx, codes, ncodes, stride, tuning, p->hist.as<unsigned long long>(), L)) != CR_OK)
+    if ((s = build_batch(ctx, codes, ncodes, stride, tuning, hist, L)) != CR_OK)
         return bail(s);
     if ((s = p->jobs.reserve(L.job_bytes())) != CR_OK) return bail(s);
     hipError_t e = L.upload(p->jobs.ptr, ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);  // L goes with this call
     if (e != hipSuccess) return bail(fail(CR_ERR_DEVICE, "job upload failed: %s", hipGetErrorString(e)));
-    // capture: zero histograms, zero queue heads + kernels, copy back
+    // capture: zero histograms and queue heads, kernels, copy back
     e = hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return bail(fail(CR_ERR_DEVICE, "graph capture failed: %s", hipGetErrorString(e)));
-    cr_status cs = fill_zero_u64(p->hist.as<unsigned long long>(), n, ctx->stream);
-    if (cs == CR_OK) cs = launch_batch(ctx, L, p->jobs.ptr, p->counter.as<unsigned long long>());
+    cr_status cs = fill_zero_u64(hist, batch_entries(n), ctx->stream);
+    if (cs == CR_OK) cs = launch_batch(ctx, L, p->jobs.ptr, hist + counters_at(n));
     if (cs == CR_OK) {
         e = hipMemcpyAsync(p->host.ptr, p->hist.ptr, n * sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream);
         if (e != hipSuccess) cs = fail(CR_ERR_DEVICE, "capture of copy-back failed: %s", hipGetErrorString(e));
