@@ -41,8 +41,23 @@ cr_status build_batch(cr_context *ctx, const cr_an_code *codes, uint32_t ncodes,
     if (!codes || ncodes == 0) return fail(CR_ERR_INVALID_ARGUMENT, "empty batch");
     const uint32_t ipw = tuning && tuning->items_per_wave ? tuning->items_per_wave : 16;
     uint32_t max_need = 0;  // of the pair kernel's codes: its waves per CU follow from their bins
-    long double total_pairs = 0, short_pairs = 0;
+    long double total_pairs = 0, short_pairs = 0, sliced_pairs = 0;
+    uint64_t most_words = 0, most_sliced = 0;
     L.jobs.reserve(ncodes);
+    std::vector<uint32_t> sliced;  // codes that the sliced kernel can take
+    auto to_pairs = [&](uint32_t c) {
+        PairJob j{};
+        j.A = codes[c].A;
+        j.N = codes[c].num_words;
+        j.out = d_hist + (size_t)c * stride;
+        j.nbins = pair_max_distance(j.A, j.N) + 1;
+        L.jobs.push_back(j);
+        max_need = std::max(max_need, j.nbins);
+        const long double pairs = (long double)j.N * (long double)(j.N - 1) / 2;
+        total_pairs += pairs;
+        if (j.N < (1ull << 15)) short_pairs += pairs;
+        most_words = std::max(most_words, j.N);
+    };
     for (uint32_t c = 0; c < ncodes; ++c) {
         const uint64_t A = codes[c].A, N = codes[c].num_words;
         if (A == 0 || N == 0) return fail(CR_ERR_INVALID_ARGUMENT, "code %u: A and num_words must be >= 1", c);
@@ -54,22 +69,28 @@ cr_status build_batch(cr_context *ctx, const cr_an_code *codes, uint32_t ncodes,
             sj.out = d_hist + (size_t)c * stride;
             sj.nbins = need;
             L.sliced.push_back(sj);
-            continue;
+            sliced.push_back(c);
+            sliced_pairs += (long double)N * (long double)N / 2;
+            most_sliced = std::max(most_sliced, N);
+        } else {
+            to_pairs(c);
         }
-        PairJob j{};
-        j.A = A;
-        j.N = N;
-        j.out = d_hist + (size_t)c * stride;
-        j.nbins = need;
-        L.jobs.push_back(j);
-        max_need = std::max(max_need, need);
-        total_pairs += (long double)N * (long double)(N - 1) / 2;
-        if (N < (1ull << 15)) short_pairs += (long double)N * (long double)(N - 1) / 2;
     }
     // as for single codes: short codes waste less of a row block of 128 words
     // than of one of 512 (16384 codes of 2^8 words 0.48 ms with 8 rows a lane, 0.20
     // with 2; 4096 codes of 2^10 words 0.64 and 0.46)
     const uint32_t R = tuning && tuning->rows_per_lane ? tuning->rows_per_lane : 2 * short_pairs >= total_pairs ? 2 : 8;
+    // Few pairs of the sliced kernel's codes do not pay for its launch (14 us at
+    // least): they go with the pair kernel's codes where those take a wave as long,
+    // a row block of 64 R words against itself (26 us with 4 rows a lane, 85 with
+    // 8), and are not too long for so few rows.  60 codes of 3000 words and four of
+    // 2^11 102 -> 88 us (4 rows 110 -> 94, 8 rows 172 -> 156); not so 60 of 200 words
+    // and one of 2^13 57 -> 69 (8 rows 82 -> 112).
+    if (!L.jobs.empty() && sliced_pairs < 2.5e7L * std::max(R, 4u) && most_words > 48ull * R &&
+        most_sliced <= 2048ull * R) {
+        for (uint32_t c : sliced) to_pairs(c);
+        L.sliced.clear();
+    }
     L.cfg.R = R;
     L.cfg.lds_rows = std::max(max_need, 1u) + 1;
     L.cfg.waves = tuning ? tuning->waves : 0;
