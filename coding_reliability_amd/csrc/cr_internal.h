@@ -375,7 +375,8 @@ struct McSegment {
     uint64_t j0, j1;
     uint64_t item_begin;      // first work item of the range (set by launch_an_mc)
     uint64_t chunks;          // sample chunks of the range (set by launch_an_mc)
-    unsigned long long *out;  // device histogram, nbins entries (zeroed by the caller)
+    unsigned long long *out;  // device histogram (zeroed by the caller), out_copies copies of it
+    uint64_t out_copies;
 };
 constexpr uint32_t kMcMaxRanges = 64;  // sample ranges per AN Monte Carlo launch
 // segs (host, nsegs entries, kept alive until the stream is synchronized) is

@@ -394,7 +394,8 @@ __global__ __launch_bounds__(64) void an_mc_kernel(uint64_t A, uint32_t n, uint6
     uint32_t cur = 0xFFFFFFFFu;  // segment whose counts the LDS rows hold
     auto flush = [&] {
         if (cur != 0xFFFFFFFFu)
-            flush_rows(lds, 0, nbins, ONE ? hist_copy(direct.copies, nbins, kHistCopies) : segs[cur].out);
+            flush_rows(lds, 0, nbins, ONE ? hist_copy(direct.copies, nbins, kHistCopies)
+                                          : hist_copy(segs[cur].out, nbins, (uint32_t)segs[cur].out_copies));
     };
     for (uint64_t t = first_item(); t < total_items; t = following_item_of(counter, heads)) {
         uint32_t sg = cur == 0xFFFFFFFFu ? 0 : cur;
