@@ -12,12 +12,17 @@
 // at a time, 100 MB) stays in the last-level cache:
 //   tiles_low   level 4 of the carry pairs that the block comes from, 32 x 32
 //               at a time: level 1 from the words themselves, levels 2, 3 in
-//               LDS, four 8-bit counters a dword (a level-r polynomial sums to
-//               4^r);
+//               LDS, four 8-bit counters a dword;
 //   tiles_high  levels 5 .. 4 + F in LDS, two 16-bit counters a dword, and the
 //               last one straight into the histogram: carry pair (c, c') serves
 //               every pair (i, j) of low parts with those carries, shifted by
 //               the distance of the low parts' own bits.
+// A level-r polynomial sums to 4^r: 256 at level 4, 65536 at level 8, one more
+// than the packed counters hold.  No coefficient takes the whole sum: for no odd
+// A < 2^16 and no two carries are all 256 pairs of level 4 at one distance
+// (enumerated; all c + A*i, i < 16, would have one parity, which leaves 112970
+// carries of all A together), so neither are the 65536 of level 8, whose terms
+// these are.
 // By symmetry only blocks and tiles with c-tile <= c'-tile run; a tile off the
 // diagonal counts twice.
 //
