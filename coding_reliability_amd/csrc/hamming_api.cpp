@@ -59,11 +59,12 @@ HamRange ham_range(const cr_ham_request *req, uint32_t need, uint32_t parity, co
     return job;
 }
 
-// Measured rates (words/s): 32-bit stride 1.9e12, 64-bit 0.55e12, Monte Carlo
-// 1.55e12 / 0.75e12, lists about half the stride rates.
+// Measured rates (words/s, launches of 2^30 words; 64-bit strides reach 1.2e12 there
+// and this at 2^27): 32-bit stride 2.5e12, 64-bit 0.9e12, Monte Carlo 1.9e12 /
+// 0.87e12, lists about half the stride rates.
 double ham_rate(const cr_ham_request *req) {
-    if (req->source == CR_HAM_MC) return req->k > 32 ? 0.75e12 : 1.55e12;
-    return (req->k > 32 ? 0.55e12 : 1.9e12) * (req->source == CR_HAM_LIST ? 0.5 : 1.0);
+    if (req->source == CR_HAM_MC) return req->k > 32 ? 0.87e12 : 1.9e12;
+    return (req->k > 32 ? 0.9e12 : 2.5e12) * (req->source == CR_HAM_LIST ? 0.5 : 1.0);
 }
 
 // A job and its work assignment in a launch of `waves` resident waves.  The
@@ -71,7 +72,10 @@ double ham_rate(const cr_ham_request *req) {
 // measured about 25 % slower on launches of 0.5 ms and more), but each queue
 // step is a device-scope atomic on one counter, serialized at about 12.5 ns, one
 // per item plus one per wave: 40-150 us per launch.  Launches estimated below
-// 100 us of work (short_launch) therefore run with a static assignment.
+// kShortLaunch of work therefore run with a static assignment (calls of 2.1e8
+// 32-bit stride words 124 us with it, 120 with the queue; of 8e7 64-bit Monte
+// Carlo words 176 and 148).
+constexpr double kShortLaunch = 82e-6;
 HamJob ham_job(const cr_ham_request *req, uint32_t need, const uint64_t masks[7], bool short_launch, uint64_t waves) {
     HamJob job{};
     memcpy(job.masks, masks, sizeof(job.masks));
@@ -108,7 +112,7 @@ HamJob ham_job(const cr_ham_request *req, uint32_t need, const uint64_t masks[7]
 // beside 2^20 Monte Carlo words of the same width: 1000 words of k = 64 39 us for
 // 70, of k = 57 44 for 62, of k = 32 30 for 43; four ranges of 2^20 words 90 us for
 // 74 at k = 64, 60 for 51 at k = 20.
-constexpr double kWordsSeconds = 2e-6;    // of all of them, by ham_rate
+constexpr double kWordsSeconds = 1.25e-6;  // of all of them, by ham_rate
 constexpr uint32_t kWordsMinK = 58;
 constexpr uint32_t kWordRanges = 4;       // eight: 0.85 to 1.22 of the recursion's time
 cr_ham_request as_words(const cr_ham_request *range) {
@@ -147,7 +151,7 @@ cr_status hamming_single(cr_context *ctx, const cr_ham_request *req, uint64_t *h
         CR_TRY(launch_ham_ranges(nullptr, 1, &job, req->k, parity, out, ctx->stream));
         return direct_wait(ctx, hist, need, nbins, kernel_ms);
     }
-    const bool short_launch = (double)req->count / ham_rate(req) < 100e-6;
+    const bool short_launch = (double)req->count / ham_rate(req) < kShortLaunch;
     const uint32_t rows = need + 1;
     HamJob job = ham_job(req, need, masks, short_launch, (uint64_t)hamming_waves_per_cu(rows) * ctx->cus);
     if (req->source == CR_HAM_LIST) {
@@ -247,7 +251,7 @@ cr_status hamming_run(cr_context *ctx, const cr_ham_request *reqs, uint32_t n, u
     if (list_words) CR_TRY(ctx->table_a.reserve(list_words * sizeof(uint64_t)));
     uint64_t list_at = 0;
     for (Launch &L : launches) {
-        L.short_launch = L.est_s < 100e-6;
+        L.short_launch = L.est_s < kShortLaunch;
         const uint64_t waves = (uint64_t)hamming_waves_per_cu(L.rows) * ctx->cus;
         for (const Pending &p : L.requests) {
             cr_ham_request words_of;

@@ -43,7 +43,7 @@ def test_few_ranges_beside_other_requests(ctx, k, others):
         assert got == want, n
 
 
-@pytest.mark.parametrize("k,edge", [(32, int(2e-6 * 1.9e12)), (58, int(2e-6 * 0.55e12)), (64, int(2e-6 * 0.55e12))])
+@pytest.mark.parametrize("k,edge", [(32, int(1.25e-6 * 2.5e12)), (58, int(1.25e-6 * 0.9e12)), (64, int(1.25e-6 * 0.9e12))])
 def test_both_sides_of_the_rule(ctx, k, edge):
     # the same words in one range on either side of the rule and in two parts
     mc = dict(k=k, source=cra.HAM_MC, count=1024, seed=5, stream=2)
