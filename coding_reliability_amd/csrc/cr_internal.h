@@ -359,14 +359,14 @@ uint32_t hamming_waves_per_cu(uint32_t lds_rows);
 // the queue.
 cr_status launch_hamming(const HamJob *d_jobs, uint32_t njobs, uint64_t total_items, bool w64,
                          unsigned long long *counter, bool allow_static, uint32_t lds_rows, int cus,
-                         hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1);
-// One job whose histogram goes to `out` (out_copies: dev::kHistCopies).
+                         hipStream_t stream);
 // The first and the last launch of a small batch: `entries` counters cleared and
 // the start clock; the counters copied to pinned memory and the end clock.
 cr_status launch_batch_begin(unsigned long long *hist, uint32_t entries, const dev::DirectResult &out,
                              hipStream_t stream);
 cr_status launch_batch_end(const unsigned long long *hist, uint32_t entries, unsigned long long *host,
                            const dev::DirectResult &out, hipStream_t stream);
+// One job whose histogram goes to `out` (out_copies: dev::kHistCopies).
 cr_status launch_hamming_direct(const HamJob &job, bool w64, bool allow_static, uint32_t lds_rows,
                                 const dev::DirectResult &out, int cus, hipStream_t stream);
 // A sample range of an AN Monte Carlo launch and its histogram: the pairs

@@ -308,7 +308,7 @@ constexpr uint32_t kMaxChunk = 256;  // most samples per item (CJ: a power of tw
 // multiply, xor and popcount), 1: the multiplier does, 2: any.  S64: 64-bit
 // samples (n > 32).  The first two rounds split into what depends on the row,
 // computed once, and what depends on the block number, scalar but for S64.
-// Bound by VALU issue: 2.95e12 pairs/s at A = 61 (32-bit words; 2.2e12 with whole
+// Bound by VALU issue: 3.16e12 pairs/s at A = 61 (24-bit samples, long launches; 2.2e12 with whole
 // rounds, scalar keys and a 64-bit sample counter), 2.5e12 at A = 58659, n = 24.  CHECK: rows past 2^n and samples outside [jlo, j1) (a partial
 // chunk) go to the dummy row; without CHECK, jlo = j0 and j1 - j0 is a
 // multiple of the words per Philox block.
@@ -523,15 +523,12 @@ cr_status ham_launch(const HamJob *jobs, uint32_t njobs, uint64_t total_items, b
 
 cr_status launch_hamming(const HamJob *d_jobs, uint32_t njobs, uint64_t total_items, bool w64,
                          unsigned long long *counter, bool allow_static, uint32_t lds_rows, int cus,
-                         hipStream_t stream, hipEvent_t ev0, hipEvent_t ev1) {
+                         hipStream_t stream) {
     uint64_t waves = 0;
     CR_TRY(ham_waves(w64, total_items, allow_static, lds_rows, cus, &waves));
     if (allow_static && total_items > 0) counter = nullptr;
     if (counter) CR_TRY(fill_zero_u64(counter, 1, stream));
-    if (ev0) CR_HIP(hipEventRecord(ev0, stream));
-    CR_TRY(ham_launch(d_jobs, njobs, total_items, w64, counter, lds_rows, waves, HamJob{}, DirectResult{}, stream));
-    if (ev1) CR_HIP(hipEventRecord(ev1, stream));
-    return CR_OK;
+    return ham_launch(d_jobs, njobs, total_items, w64, counter, lds_rows, waves, HamJob{}, DirectResult{}, stream);
 }
 
 cr_status launch_batch_begin(unsigned long long *hist, uint32_t entries, const DirectResult &out, hipStream_t stream) {

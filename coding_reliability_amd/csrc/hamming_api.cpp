@@ -319,7 +319,7 @@ cr_status hamming_run(cr_context *ctx, const cr_ham_request *reqs, uint32_t n, u
         if (L.jobs.empty()) continue;
         CR_TRY(launch_hamming(ctx->jobs.as<HamJob>() + (w ? launches[0].jobs.size() : 0), (uint32_t)L.jobs.size(),
                               L.items, w == 1, ctx->counters.as<unsigned long long>() + w, L.short_launch, L.rows,
-                              ctx->cus, ctx->stream, nullptr, nullptr));
+                              ctx->cus, ctx->stream));
     }
     uint64_t *const copies = ctx->host.as<uint64_t>() + kHeader;
     if (small) {

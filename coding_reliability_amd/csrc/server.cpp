@@ -290,10 +290,10 @@ cr_status cr_server::iterate(std::vector<Request *> &run) {
     CR_HIP(hipEventRecord(evm, stream));
     if (!h32.empty())
         CR_TRY(launch_hamming(ham_jobs.as<HamJob>(), (uint32_t)h32.size(), t32, false, ctr + 1, false, lds_ham,
-                              ctx->cus, stream, nullptr, nullptr));
+                              ctx->cus, stream));
     if (!h64.empty())
         CR_TRY(launch_hamming(ham_jobs.as<HamJob>() + h32.size(), (uint32_t)h64.size(), t64, true, ctr + 2, false,
-                              lds_ham, ctx->cus, stream, nullptr, nullptr));
+                              lds_ham, ctx->cus, stream));
     CR_HIP(hipEventRecord(ev1, stream));
     for (auto &sr : spec) {
         Request *r = sr.first;
