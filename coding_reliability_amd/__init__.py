@@ -214,6 +214,9 @@ class Context:
         return BatchPlan(self, codes, rows_per_lane, items_per_wave)
 
     def autotune_batch(self, codes, repeats: int = 1) -> tuple[dict, float]:
+        """The fastest of the explicit settings of the batched pair kernel on these
+        codes and its time in ms (cr_autotune_batch); the automatic one (0, 0),
+        the faster for short codes, is not timed."""
         # an array of codes takes floats and longer tuples without a word
         codes = [(operator.index(A), operator.index(N)) for A, N in codes]
         best = cr_pair_tuning()
