@@ -51,6 +51,8 @@ cr_status build_batch(cr_context *ctx, const cr_an_code *codes, uint32_t ncodes,
         j.N = codes[c].num_words;
         j.out = d_hist + (size_t)c * stride;
         j.nbins = pair_max_distance(j.A, j.N) + 1;
+        j.mode = pair_mode(j.A, j.N);
+        L.cfg.wide = L.cfg.wide || j.mode == kModeWide;
         L.jobs.push_back(j);
         max_need = std::max(max_need, j.nbins);
         const long double pairs = (long double)j.N * (long double)(j.N - 1) / 2;
@@ -83,10 +85,11 @@ cr_status build_batch(cr_context *ctx, const cr_an_code *codes, uint32_t ncodes,
     // Few pairs of the sliced kernel's codes do not pay for its launch (14 us at
     // least): they go with the pair kernel's codes where those take a wave as long,
     // a row block of 64 R words against itself (26 us with 4 rows a lane, 85 with
-    // 8), and are not too long for so few rows.  60 codes of 3000 words and four of
+    // 8), are not too long for so few rows, and need no matrix instructions (whose
+    // kernel is the slower one for other codes).  60 codes of 3000 words and four of
     // 2^11 102 -> 88 us (4 rows 110 -> 94, 8 rows 172 -> 156); not so 60 of 200 words
     // and one of 2^13 57 -> 69 (8 rows 82 -> 112).
-    if (!L.jobs.empty() && sliced_pairs < 2.5e7L * std::max(R, 4u) && most_words > 48ull * R &&
+    if (!L.jobs.empty() && !L.cfg.wide && sliced_pairs < 2.5e7L * std::max(R, 4u) && most_words > 48ull * R &&
         most_sliced <= 2048ull * R) {
         for (uint32_t c : sliced) to_pairs(c);
         L.sliced.clear();
@@ -95,10 +98,6 @@ cr_status build_batch(cr_context *ctx, const cr_an_code *codes, uint32_t ncodes,
     L.cfg.lds_rows = std::max(max_need, 1u) + 1;
     L.cfg.waves = tuning ? tuning->waves : 0;
     L.cfg.zero_counter = false;
-    for (PairJob &j : L.jobs) {
-        j.mode = pair_mode(j.A, j.N);
-        L.cfg.wide = L.cfg.wide || j.mode == kModeWide;
-    }
     const uint32_t per_cu = pair_waves_per_cu(R, L.cfg.lds_rows, L.cfg.wide);
     if (per_cu == 0) return fail(CR_ERR_INVALID_ARGUMENT, "rows_per_lane must be 2, 4, 8 or 16 (got %u)", R);
     const long double waves = (long double)per_cu * ctx->cus;
