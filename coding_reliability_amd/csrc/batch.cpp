@@ -84,7 +84,7 @@ cr_status build_batch(cr_context *ctx, const cr_an_code *codes, uint32_t ncodes,
     const uint32_t R = tuning && tuning->rows_per_lane ? tuning->rows_per_lane : 2 * short_pairs >= total_pairs ? 2 : 8;
     // Few pairs of the sliced kernel's codes do not pay for its launch (14 us at
     // least): they go with the pair kernel's codes where those take a wave as long,
-    // a row block of 64 R words against itself (26 us with 4 rows a lane, 85 with
+    // a row block of 64 R words against itself (31 us with 4 rows a lane, 86 with
     // 8), are not too long for so few rows, and need no matrix instructions (whose
     // kernel is the slower one for other codes).  60 codes of 3000 words and four of
     // 2^11 102 -> 88 us (4 rows 110 -> 94, 8 rows 172 -> 156); not so 60 of 200 words
